@@ -1,10 +1,13 @@
 // Quantize-on-append: encode 128-token codec pages of pre-RoPE keys and values
-// straight into 16-token physical pages, gfx950.
+// straight into 16-token physical pages, gfx950 -- the recipe's page and the
+// general page (include/bmx_k2b.h).
 //
-// Three launches per call (all codec pages of the call in each):
-//   k2b_us_kernel    Us = M * basis32 (or the first page's SVD factor), fp16
-//   k2b_kres_kernel  R = M - Us16 * basis16^T, per-channel 64-token RTN at 3 bits
-//   k2b_v_kernel     per (token, head): fp16 norm, sign flip, FWHT, Lloyd codes
+//   append_us_kernel     Us = M * basis32 (or the first page's SVD factor), fp16
+//   append_codes_kernel  (recipe's page) two kinds of workgroup in one launch:
+//                        R = M - Us16 * basis16^T with its per-channel RTN, and
+//                        per (token, head) the value's fp16 norm and Lloyd codes
+//   gen_kres_kernel, value_codes_kernel  the same two as launches of their own
+//                        (general page; the values of spectral pages)
 // Reference semantics: cache/packed_streaming.py:475-580 (page commit),
 // cache/codecs.py:616-636, 677-695, 786-796 (codecs), quant/rtn.py:23-44 (RTN),
 // quant/hadamard.py:12-33 (FWHT).  Element-wise steps follow the reference's
@@ -12,234 +15,441 @@
 // this file is built without floating-point contraction, so codes are identical
 // to the reference's whenever the reduction results (Us, the norm) agree.
 
+#include <algorithm>
+#include <cmath>
+#include <string>
+#include <type_traits>
+
 #include "k2b_common.h"
 #include "k2b_general.h"
 
 namespace bmx {
 
-// grid (n_codec_pages * 8), block 256 = 4 waves, one 16-token page slot each.
-// Us[t][r] = sum_c M[t][c] basis32[c][r] in fp32 (the reference's M @ V).  The
-// page's 16 key rows are staged in LDS (rows padded by one bank); wave w sums
-// channels [w C/4, (w+1) C/4) in order, lane (t = lane & 15, quad rq = lane >> 4)
-// owns ranks rq R/4 .. + R/4; the four partial sums are then added in wave
-// order.  The first codec page of a sequence takes its SVD factor instead.
-template <int R>
-__global__ __launch_bounds__(256) void k2b_us_kernel(const AppendKArgs a) {
-  constexpr int RQ = R / 4;
-  extern __shared__ uint16_t s_m[];          // [kPT][C + 2] fp16 key rows
-  __shared__ float s_part[4][kPT][R + 1];
-  const int pg = blockIdx.x;                  // physical page slot (16 tokens)
-  const int cp = pg / 8, pl = pg % 8;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int C = kD * a.h_kv, ld = C + 2;
-  uint8_t* page = a.pages + clamp_page(a.page_ids[pg], a.n_pool) * a.L.bytes;
-  if (a.us_first != nullptr && cp == 0) {
-    for (int e = tid; e < kPT * R; e += 256) {
-      const int t = e / R, r = e % R;
-      *reinterpret_cast<uint16_t*>(page + a.L.us + us_half(R, t, r) * 2) =
-          float_to_half_bits(a.us_first[(pl * kPT + t) * R + r]);
-    }
-    return;
-  }
-  for (int e = tid; e < kPT * C; e += 256) {
-    const int t = e / C, c = e % C;
-    s_m[t * ld + c] = a.k_pre[(c / kD) * a.ksh + (int64_t)(pg * kPT + t) * a.kst + (c % kD)];
-  }
-  __syncthreads();
-  const int t = lane & 15, rq = lane >> 4;
-  float acc[RQ];
-#pragma unroll
-  for (int k = 0; k < RQ; ++k) acc[k] = 0.f;
-  const int c0 = wave * (C / 4), c1 = c0 + C / 4;
-#pragma unroll 4
-  for (int c = c0; c < c1; ++c) {
-    const float m = half_bits_to_float(s_m[t * ld + c]);
-    const float4* b = reinterpret_cast<const float4*>(a.basis32 + (int64_t)c * R + rq * RQ);
-#pragma unroll
-    for (int k4 = 0; k4 < RQ / 4; ++k4) {
-      const float4 bv = b[k4];
-      acc[4 * k4 + 0] = __builtin_fmaf(m, bv.x, acc[4 * k4 + 0]);
-      acc[4 * k4 + 1] = __builtin_fmaf(m, bv.y, acc[4 * k4 + 1]);
-      acc[4 * k4 + 2] = __builtin_fmaf(m, bv.z, acc[4 * k4 + 2]);
-      acc[4 * k4 + 3] = __builtin_fmaf(m, bv.w, acc[4 * k4 + 3]);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < RQ; ++k) s_part[wave][t][rq * RQ + k] = acc[k];
-  __syncthreads();
-  for (int e = tid; e < kPT * R; e += 256) {
-    const int tt = e / R, r = e % R;
-    const float us = ((s_part[0][tt][r] + s_part[1][tt][r]) + s_part[2][tt][r]) + s_part[3][tt][r];
-    *reinterpret_cast<uint16_t*>(page + a.L.us + us_half(R, tt, r) * 2) = float_to_half_bits(us);
-  }
+__device__ __forceinline__ uint8_t* append_page(const AppendKArgs& a, int slot) {
+  return a.pages + clamp_page(a.page_ids[slot], a.n_pool) * (int64_t)a.L.bytes;
 }
 
-// grid (n_codec_pages * 2 groups, h_kv), block 256: 64 tokens x 128 channels.
-__global__ __launch_bounds__(256) void k2b_kres_kernel(const AppendKArgs a) {
-  const int gi = blockIdx.x;        // 64-token group index within the call
-  const int h = blockIdx.y;
-  const int cp = gi / 2, grp_in = gi % 2;
-  const int C = kD * a.h_kv;
-  const int R = a.R;
-  __shared__ float s_us[kGroup][33];
-  __shared__ float s_b[kD][33];
-  __shared__ float s_amax[2][kD];
-  __shared__ int8_t s_code[kGroup][kD + 4];
+// x / d correctly rounded from r = fl(1 / d): two residual corrections of x r.
+// The first leaves a quotient within an ulp, the second then rounds correctly
+// (Markstein 1990; d, r and the quotient normal, |x| >= 2^-100 or x = 0).
+// 5 instructions against ~11 of the general division.
+__device__ __forceinline__ float div_by(float x, float d, float r) {
+  const float q0 = x * r;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, d, x), r, q0);
+  return __builtin_fmaf(__builtin_fmaf(-q1, d, x), r, q1);
+}
 
-  const int tid = threadIdx.x;
-  // Us16 of the group's 64 tokens (already written to the 4 pages)
-  for (int e = tid; e < kGroup * R; e += 256) {
-    const int t = e / R, r = e % R;
-    const int pslot = cp * 8 + grp_in * 4 + t / kPT;
-    const uint8_t* page = a.pages + clamp_page(a.page_ids[pslot], a.n_pool) * a.L.bytes;
-    s_us[t][r] = half_bits_to_float(*reinterpret_cast<const uint16_t*>(page + a.L.us + us_half(R, t % kPT, r) * 2));
+// grid (16-token pages of the call, R / 16), block 256 = 4 waves.
+// Us[t][r] = sum_c M[t][c] basis32[c][r] in fp32 (the reference's M @ V): wave w
+// sums channels [w C/4, (w+1) C/4) in order, lane (t = lane & 15, rq = lane >> 4)
+// owns ranks 16 blockIdx.y + 4 rq .. + 3, and the four partial sums are added in
+// wave order.  The first codec page of a sequence takes its SVD factor instead.
+// Bound: one wave's chain of C / 4 dependent steps (a commit of one codec page
+// has only 8 R / 16 workgroups), so a step must cost its 4 FMAs and no memory
+// round trip: the workgroup's 16 basis columns are staged in LDS up front, the
+// lane's key row is read 8 channels per 16-byte load with 16 loads in flight,
+// and a chunk's basis values leave LDS a chunk ahead of their FMAs.
+// Measured at h_kv 8: 10.8 us for one codec page at R 32, 16.3 us for 63 at
+// R 16; with the basis read from global memory inside the chain and the keys
+// staged in LDS 26.0 and 35.4 us.
+// kVec: rows 16-byte aligned; else the 8 channels are read one by one.
+template <bool kVec>
+__global__ __launch_bounds__(256) void append_us_kernel(const AppendKArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float s_b[];   // [C][16] fp32 basis columns
+  __shared__ float s_part[4][kPT][17];
+  const int pg = blockIdx.x, rg = blockIdx.y;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int C = a.C, R = a.R, ld = a.log2d, d = 1 << ld;
+  uint8_t* page = append_page(a, pg);
+  uint16_t* us = reinterpret_cast<uint16_t*>(page + a.L.us);
+  const int ot = tid >> 4, orank = 16 * rg + (tid & 15);     // the output of this thread
+  const int oi = a.general ? ot * R + orank : us_half(R, ot, orank);
+  if (a.us_first != nullptr && pg < 8) {
+    us[oi] = float_to_half_bits(a.us_first[(pg * kPT + ot) * R + orank]);
+    return;
   }
-  for (int e = tid; e < kD * R; e += 256) {
-    const int j = e / R, r = e % R;
-    s_b[j][r] = half_bits_to_float(a.basis16[(int64_t)(h * kD + j) * R + r]);
+  const int t = lane & 15, rq = lane >> 4;
+  const uint16_t* row = a.k_pre + (int64_t)(pg * kPT + t) * a.kst;
+  const int c0 = wave * (C / 4), n8 = C / 32;     // the wave's channels, in chunks of 8
+  auto load8 = [&](int k) -> uint4 {
+    const int c = c0 + 8 * min(k, n8 - 1);
+    const uint16_t* p = row + (int64_t)(c >> ld) * a.ksh + (c & (d - 1));
+    if constexpr (kVec) return *reinterpret_cast<const uint4*>(p);
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = p[2 * i] | (uint32_t)p[2 * i + 1] << 16;
+    return make_uint4(w[0], w[1], w[2], w[3]);
+  };
+  // the row in batches of 4 chunks, 4 batches in flight (a ring of registers)
+  constexpr int kB = 4, kSets = 4;
+  const int nb = n8 / kB;
+  uint4 ring[kSets][kB];
+#pragma unroll
+  for (int s = 0; s < kSets; ++s)
+#pragma unroll
+    for (int i = 0; i < kB; ++i) ring[s][i] = load8(kB * s + i);
+  for (int e0 = tid; e0 < C * 4; e0 += 8 * 256) {   // 8 loads in flight per thread
+    float4_t v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int e = min(e0 + 256 * i, C * 4 - 1);
+      v[i] = *reinterpret_cast<const float4_t*>(a.basis32 + (int64_t)(e >> 2) * R + 16 * rg + 4 * (e & 3));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (e0 + 256 * i < C * 4) reinterpret_cast<float4_t*>(s_b)[e0 + 256 * i] = v[i];
   }
   __syncthreads();
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  float4_t b[2][8];   // the basis values of a chunk, read one chunk ahead of their FMAs
+  auto read_b = [&](float4_t (&dst)[8], int k) {
+    const float4_t* p = reinterpret_cast<const float4_t*>(s_b + (c0 + 8 * min(k, n8 - 1)) * 16 + 4 * rq);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) dst[j] = p[4 * j];
+  };
+  auto chunk = [&](const uint4& x, const float4_t (&bv)[8]) {
+    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float m = (float)as_h2(w[j >> 1])[j & 1];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf(m, bv[j][r], acc[r]);
+    }
+  };
+  read_b(b[0], 0);
+  for (int k0 = 0; k0 < nb; k0 += kSets) {
+#pragma unroll
+    for (int s = 0; s < kSets; ++s) {
+      if (k0 + s >= nb) break;
+#pragma unroll
+      for (int i = 0; i < kB; ++i) {
+        read_b(b[(i + 1) & 1], kB * (k0 + s) + i + 1);
+        __builtin_amdgcn_sched_barrier(0);   // the reads stay a chunk ahead
+        chunk(ring[s][i], b[i & 1]);
+      }
+#pragma unroll
+      for (int i = 0; i < kB; ++i) ring[s][i] = load8(kB * (k0 + s + kSets) + i);
+    }
+  }
+  for (int k = kB * nb; k < n8; ++k) {   // C / 32 not a multiple of 4
+    read_b(b[0], k);
+    chunk(load8(k), b[0]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) s_part[wave][t][4 * rq + r] = acc[r];
+  __syncthreads();
+  const int o = tid & 15;
+  us[oi] = float_to_half_bits(((s_part[0][ot][o] + s_part[1][ot][o]) + s_part[2][ot][o]) + s_part[3][ot][o]);
+}
 
-  const int j = tid & 127, half = tid >> 7;
-  float res[32];
+// One residual group's tokens x one head's channels, 512 threads: thread
+// (channel j = tid % d, part tid / d) takes tokens part, part + 512/d, ...
+// (PER of them): L = sum_r Us16[t][r] basis16[c][r] (fp32, ranks in order),
+// R = M - L; the channel's scale is max |R| over the group / qmax and its codes
+// clamp(rint(R / scale), -qmax - 1, qmax).  VALU-bound: R FMAs per element.
+// The thread's basis row stays in registers (fp16 pairs, exact) and a token's
+// Us row is one LDS broadcast per 8 ranks: 32 FMAs to 4 LDS reads at R 32,
+// where both operands from LDS made 2 reads per FMA.
+template <int R, int PER>
+struct ResidualLds {
+  static constexpr int kNG = 16 * PER < 128 ? 16 * PER : 128;   // tokens of a group, at most
+  uint16_t us[kNG * R];
+  float amax[512];
+  int8_t code[512 * PER + 4 * kNG];                             // [tokens][d + 4]
+};
+
+template <int R, int PER, bool kGeneral>
+__device__ __forceinline__ void encode_residual(const AppendKArgs& a, ResidualLds<R, PER>& s, int gi, int h) {
+  const int tid = threadIdx.x, ld = kGeneral ? a.log2d : 7, D = 1 << ld;
+  const int NG = (512 * PER) >> ld, C = a.C;
+  const int slot0 = gi * (NG / kPT);                 // first 16-token page slot of the group
+  const int j = tid & (D - 1), part = tid >> ld, parts = 512 >> ld;
+  half8_t b[R / 8];                                  // the channel's basis row
+  const uint16_t* bp = a.basis16 + (int64_t)(h * D + j) * R;
+  if ((reinterpret_cast<uintptr_t>(a.basis16) & 15) == 0) {
+#pragma unroll
+    for (int i = 0; i < R / 8; ++i) b[i] = *reinterpret_cast<const half8_t*>(bp + 8 * i);
+  } else {
+#pragma unroll
+    for (int i = 0; i < R; ++i) b[i / 8][i % 8] = __builtin_bit_cast(_Float16, bp[i]);
+  }
+  float res[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    res[k] = half_bits_to_float(a.k_pre[h * a.ksh + (int64_t)(slot0 * kPT + part + parts * k) * a.kst + j]);
+  for (int e = tid; e < NG * R / 2; e += 512) {      // rank pairs (2 e' even: within one row of either page)
+    const int t = 2 * e / R, r = 2 * e % R;
+    const uint8_t* page = append_page(a, slot0 + t / kPT);
+    const int i = kGeneral ? (t % kPT) * R + r : us_half(R, t % kPT, r);
+    reinterpret_cast<uint32_t*>(s.us)[e] = *reinterpret_cast<const uint32_t*>(page + a.L.us + 2 * i);
+  }
+  __syncthreads();
   float amax = 0.f;
 #pragma unroll
-  for (int tt = 0; tt < 32; ++tt) {
-    const int t = half * 32 + tt;                                  // token within group
-    const int tg = cp * kCodec + grp_in * kGroup + t;             // token within call
+  for (int k = 0; k < PER; ++k) {
+    const half8_t* u = reinterpret_cast<const half8_t*>(s.us + (part + parts * k) * R);
     float L = 0.f;
-    for (int r = 0; r < R; ++r) L = __builtin_fmaf(s_us[t][r], s_b[j][r], L);
-    const float m = half_bits_to_float(a.k_pre[h * a.ksh + (int64_t)tg * a.kst + j]);
-    res[tt] = m - L;
-    amax = fmaxf(amax, fabsf(res[tt]));
-  }
-  s_amax[half][j] = amax;
-  __syncthreads();
-  const float scale = fmaxf(fmaxf(s_amax[0][j], s_amax[1][j]), 1e-12f) / 3.0f;
 #pragma unroll
-  for (int tt = 0; tt < 32; ++tt) {
-    float cq = rintf(res[tt] / scale);
-    cq = fminf(fmaxf(cq, -4.0f), 3.0f);
-    s_code[half * 32 + tt][j] = (int8_t)cq;
+    for (int i = 0; i < R / 8; ++i) {
+      const half8_t uv = u[i];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) L = __builtin_fmaf((float)uv[e], (float)b[i][e], L);
+    }
+    res[k] = res[k] - L;
+    amax = fmaxf(amax, fabsf(res[k]));
   }
-  if (half == 0) {
-    const int f = kscale_flat(h * kD + j), quarter = C / 4;
-    const int slot = f / quarter, off = f % quarter;
-    uint8_t* page = a.pages + clamp_page(a.page_ids[cp * 8 + grp_in * 4 + slot], a.n_pool) * a.L.bytes;
-    *reinterpret_cast<uint16_t*>(page + a.L.kscale + off * 2) = float_to_half_bits(scale);
+  s.amax[tid] = amax;
+  __syncthreads();
+  float mx = s.amax[j];
+  for (int p = 1; p < parts; ++p) mx = fmaxf(mx, s.amax[(p << ld) + j]);
+  const int qmax = kGeneral ? (1 << (a.bits - 1)) - 1 : 3;
+  const float scale = fmaxf(mx, 1e-12f) / (float)qmax;
+  const float lo = (float)(-qmax - 1), hi = (float)qmax;
+  // scale is at least 1e-12 / 7; only the rounding near half codes matters, so
+  // tiny residuals need no exact quotient
+  if (__all(scale < 3.0e38f)) {
+    const float rs = 1.0f / scale;
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      s.code[(part + parts * k) * (D + 4) + j] = (int8_t)fminf(fmaxf(rintf(div_by(res[k], scale, rs)), lo), hi);
+  } else {
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      s.code[(part + parts * k) * (D + 4) + j] = (int8_t)fminf(fmaxf(rintf(res[k] / scale), lo), hi);
+  }
+  if (part == 0) {
+    const int f = kGeneral ? h * D + j : kscale_flat(h * D + j), per_slot = C / (NG / kPT);
+    const int slot = f / per_slot;
+    *reinterpret_cast<uint16_t*>(append_page(a, slot0 + slot) + a.L.kscale + (f - slot * per_slot) * 2) =
+        float_to_half_bits(scale);
   }
   __syncthreads();
-  // pack: thread -> (page pl, lane 16q+n); pair p = 4b+i is channels (j, j+64),
-  // j = 16b + 4q + i, stored offset-binary
-  {
+  if constexpr (kGeneral) {
+    // KRES: 8 channels (4 bytes) of one token per item, offset-binary nibbles
+    const int off = 1 << (a.bits - 1), l8 = ld - 3;
+    for (int e = tid; e < NG << l8; e += 512) {
+      const int t = e >> l8, j8 = e & ((1 << l8) - 1);
+      uint32_t w = 0u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) w |= (uint32_t)(s.code[t * (D + 4) + 8 * j8 + i] + off) << (4 * i);
+      *reinterpret_cast<uint32_t*>(append_page(a, slot0 + t / kPT) + a.L.kres + (h * kPT + t % kPT) * (D / 2) +
+                                   4 * j8) = w;
+    }
+  } else if (tid < 256) {
+    // thread -> (page pl, lane 16q+n); pair p = 4b+i is channels (j, j+64),
+    // j = 16b + 4q + i, stored offset-binary
     const int pl = tid >> 6, lane = tid & 63, q = lane >> 4, n = lane & 15;
-    const int t = pl * kPT + n;
+    const int8_t* c = s.code + (pl * kPT + n) * (kD + 4);
     uint32_t w[3] = {0u, 0u, 0u};
 #pragma unroll
     for (int p = 0; p < 16; ++p) {
       const int jj = 16 * (p >> 2) + 4 * q + (p & 3);
-      const uint32_t lo = (uint32_t)(s_code[t][jj] + 4), hi = (uint32_t)(s_code[t][jj + 64] + 4);
+      const uint32_t lo3 = (uint32_t)(c[jj] + 4), hi3 = (uint32_t)(c[jj + 64] + 4);
       if (p < 15) {
-        w[p / 5] |= (lo << (3 * (p % 5))) | (hi << (16 + 3 * (p % 5)));
+        w[p / 5] |= (lo3 << (3 * (p % 5))) | (hi3 << (16 + 3 * (p % 5)));
       } else {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) w[k] |= (((lo >> k) & 1u) << 15) | (((hi >> k) & 1u) << 31);
+        for (int k = 0; k < 3; ++k) w[k] |= (((lo3 >> k) & 1u) << 15) | (((hi3 >> k) & 1u) << 31);
       }
     }
-    uint8_t* page = a.pages + clamp_page(a.page_ids[cp * 8 + grp_in * 4 + pl], a.n_pool) * a.L.bytes;
-    uint32_t* dst = reinterpret_cast<uint32_t*>(page + a.L.kres + h * 768 + lane * 12);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(append_page(a, slot0 + pl) + a.L.kres + h * 768 + lane * 12);
     dst[0] = w[0]; dst[1] = w[1]; dst[2] = w[2];
   }
 }
 
-// grid (n_codec_pages * 8, h_kv), block 256: 16 tokens x 128 channels.
-__global__ __launch_bounds__(256) void k2b_v_kernel(const AppendKArgs a) {
-  const int pg = blockIdx.x, h = blockIdx.y;
-  const int tid = threadIdx.x;
-  __shared__ float x[kPT][kD];
-  __shared__ float s_norm[kPT];
-  __shared__ uint8_t code[kPT][kD];
-  uint8_t* page = a.pages + clamp_page(a.page_ids[pg], a.n_pool) * a.L.bytes;
-
-  for (int e = tid; e < kPT * kD; e += 256) {
-    const int t = e / kD, c = e % kD;
-    const int64_t i = h * a.vsh + (int64_t)(pg * kPT + t) * a.vst + c;
-    float val;
-    if (a.v_dtype == BMX_K2B_F32)
-      val = static_cast<const float*>(a.v)[i];
-    else if (a.v_dtype == BMX_K2B_BF16)
-      val = __uint_as_float((uint32_t)static_cast<const uint16_t*>(a.v)[i] << 16);
-    else
-      val = half_bits_to_float(static_cast<const uint16_t*>(a.v)[i]);
-    x[t][c] = val;
-  }
-  __syncthreads();
-  // norms: one thread per token, in the order torch's CPU 2-norm reduces a
-  // 128-float row (8 strided FMA accumulators, then a left-to-right sum, then a
-  // correctly rounded sqrt), so the fp16 norm is identical to the reference's
-  if (tid < kPT) {
-    const int t = tid;
-    float acc8[8];
+// Eight tokens of one head, one wave: lane 8t + j holds channels 8i + j of
+// token t.  The fp16 norm in the order torch's CPU 2-norm reduces a row (8
+// strided FMA accumulators -- one per lane --, then those left to right, then a
+// correctly rounded sqrt), the unit row times the signs, the FWHT's stages in
+// the reference's order (channel bits 0..2 across the token's lanes by DPP, the
+// others in registers), and each code as the count of thresholds the rotated
+// value reaches (code_cuts: the values from which (x / sqrt(d)) * sqrt(d) > mid).
+// No LDS and no barrier; VALU-bound, ~27 instructions a value.
+template <int D>
+__device__ __forceinline__ void encode_values(const AppendKArgs& a, int pg, int half, int h, bool recipe) {
+  constexpr int NI = D / 8;
+  const int lane = threadIdx.x & 63, j = lane & 7, tok = 8 * half + (lane >> 3);
+  const int64_t row = h * a.vsh + (int64_t)(pg * kPT + tok) * a.vst + j;
+  float x[NI];
+  bool tiny = false;   // a nonzero value below 2^-100: div_by would not be exact
+  if (a.v_dtype == BMX_K2B_F16) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc8[j] = 0.f;
-    for (int i = 0; i < kD; i += 8) {
+    for (int i = 0; i < NI; ++i) x[i] = half_bits_to_float(static_cast<const uint16_t*>(a.v)[row + 8 * i]);
+  } else {
+    if (a.v_dtype == BMX_K2B_BF16) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc8[j] = __builtin_fmaf(x[t][i + j], x[t][i + j], acc8[j]);
-    }
-    float ss = acc8[0];
+      for (int i = 0; i < NI; ++i)
+        x[i] = __uint_as_float((uint32_t)static_cast<const uint16_t*>(a.v)[row + 8 * i] << 16);
+    } else {
 #pragma unroll
-    for (int j = 1; j < 8; ++j) ss = ss + acc8[j];
-    {
-      const float nrm = fmaxf(__builtin_sqrtf(ss), 1e-12f);
-      const uint16_t nb = float_to_half_bits(nrm);
-      s_norm[t] = half_bits_to_float(nb);
-      *reinterpret_cast<uint16_t*>(page + a.L.vnorm + (h * kPT + t) * 2) = nb;
+      for (int i = 0; i < NI; ++i) x[i] = static_cast<const float*>(a.v)[row + 8 * i];
     }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) tiny |= (x[i] != 0.f) & (fabsf(x[i]) < 0x1p-100f);
   }
-  __syncthreads();
-  for (int e = tid; e < kPT * kD; e += 256) {
-    const int t = e / kD, c = e % kD;
-    const float u = x[t][c] / s_norm[t];
-    x[t][c] = sign_neg(a.v_sign_bits, c) ? -u : u;
+  float acc = 0.f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) acc = __builtin_fmaf(x[i], x[i], acc);
+  // the 8 lanes' sums, left to right, in every lane of the token
+  auto of_lane = [&](auto k) {   // lane k of each group of 8
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, acc), 0x18 | (decltype(k)::value << 5)));
+  };
+  const float s1 = of_lane(std::integral_constant<int, 1>{}), s2 = of_lane(std::integral_constant<int, 2>{}),
+              s3 = of_lane(std::integral_constant<int, 3>{}), s4 = of_lane(std::integral_constant<int, 4>{}),
+              s5 = of_lane(std::integral_constant<int, 5>{}), s6 = of_lane(std::integral_constant<int, 6>{}),
+              s7 = of_lane(std::integral_constant<int, 7>{});
+  float ss = of_lane(std::integral_constant<int, 0>{});
+  ss = ((((((ss + s1) + s2) + s3) + s4) + s5) + s6) + s7;
+  const uint16_t nb = float_to_half_bits(fmaxf(__builtin_sqrtf(ss), 1e-12f));
+  const float nrm = half_bits_to_float(nb);
+  uint8_t* page = append_page(a, __builtin_amdgcn_readfirstlane(pg));
+  if (j == 0) *reinterpret_cast<uint16_t*>(page + a.L.vnorm + (h * kPT + tok) * 2) = nb;
+  if (__all(nrm > 0.f && nrm < 65505.f && !tiny)) {
+    const float r = 1.0f / nrm;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x[i] = div_by(x[i], nrm, r);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x[i] = x[i] / nrm;
   }
-  __syncthreads();
-  // FWHT stages (i, i+hb) inside blocks of 2hb, as quant/hadamard.py:19-25
-  for (int hb = 1; hb < kD; hb <<= 1) {
-    for (int e = tid; e < kPT * kD / 2; e += 256) {
-      const int t = e / (kD / 2), pidx = e % (kD / 2);
-      const int i0 = (pidx / hb) * 2 * hb + (pidx % hb);
-      const float u = x[t][i0], w = x[t][i0 + hb];
-      x[t][i0] = u + w;
-      x[t][i0 + hb] = u - w;
-    }
-    __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NI; ++i)   // channel 8i + j: byte i & 3 of sign word i >> 2
+    x[i] = __uint_as_float(__float_as_uint(x[i]) ^ (((a.v_sign_bits[i >> 2] >> (8 * (i & 3) + j)) & 1u) << 31));
+  // FWHT stages (c, c + hb): the upper lane's partner minus its own
+  const float g1 = (j & 1) ? -1.f : 1.f, g2 = (j & 2) ? -1.f : 1.f, g4 = (j & 4) ? -1.f : 1.f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) x[i] = __builtin_fmaf(g1, x[i], xor_row16<1>(x[i]));
+#pragma unroll
+  for (int i = 0; i < NI; ++i) x[i] = __builtin_fmaf(g2, x[i], xor_row16<2>(x[i]));
+#pragma unroll
+  for (int i = 0; i < NI; ++i) x[i] = __builtin_fmaf(g4, x[i], xor_row16<4>(x[i]));
+#pragma unroll
+  for (int hb = 1; hb < NI; hb <<= 1)
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (!(i & hb)) {
+        const float u = x[i], w = x[i | hb];
+        x[i] = u + w;
+        x[i | hb] = u - w;
+      }
+  const float k0 = a.code_cuts[0], k1 = a.code_cuts[1], k2 = a.code_cuts[2];
+  const int t4 = tok & 3, q = tok >> 2;
+  uint32_t w[NI / 4];
+#pragma unroll
+  for (int k = 0; k < NI / 4; ++k) w[k] = 0u;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const uint32_t code = (uint32_t)(x[i] >= k0) + (uint32_t)(x[i] >= k1) + (uint32_t)(x[i] >= k2);
+    // recipe's page: dword 2 (i & 1) + (b >> 2), channel block b = i >> 1, byte
+    // b & 3; general page: dword i >> 2, byte i & 3
+    if (D == 128 && recipe) w[2 * (i & 1) + (i >> 3)] |= code << (8 * ((i >> 1) & 3));
+    else w[i >> 2] |= code << (8 * (i & 3));
   }
-  const float sqrt_d = 11.313708498984761f;  // fl32(sqrt(128)), applied as / then *
-  const float mid0 = (a.codebook[0] + a.codebook[1]) / 2.0f;
-  const float mid1 = (a.codebook[1] + a.codebook[2]) / 2.0f;
-  const float mid2 = (a.codebook[2] + a.codebook[3]) / 2.0f;
-  for (int e = tid; e < kPT * kD; e += 256) {
-    const int t = e / kD, c = e % kD;
-    const float r = (x[t][c] / sqrt_d) * sqrt_d;
-    code[t][c] = (uint8_t)((r > mid0) + (r > mid1) + (r > mid2));
+  // a byte holds the codes of 4 tokens: those of lanes ^ 8, ^ 16, ^ 24
+#pragma unroll
+  for (int k = 0; k < NI / 4; ++k) {
+    uint32_t v = w[k] << (2 * t4);
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);   // row rotation by 8: lane ^ 8
+    v |= (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x1F | (16 << 10));     // lane ^ 16
+    w[k] = v;
   }
-  __syncthreads();
-  if (tid < 128) {  // lane 16q+m, dword w: channel 16b + m (b = 4w + bb), token 4q + t at bit 8bb + 2t
-    const int lane = tid >> 1, w = tid & 1, q = lane >> 4, m = lane & 15;
-    uint32_t dword = 0;
-    for (int bb = 0; bb < 4; ++bb) {
-      const int c = 16 * (4 * w + bb) + m;
-      for (int t = 0; t < 4; ++t) dword |= (uint32_t)code[4 * q + t][c] << (8 * bb + 2 * t);
-    }
-    *reinterpret_cast<uint32_t*>(page + a.L.vcode + h * 512 + lane * 8 + w * 4) = dword;
+  if (D == 128 && recipe) {   // token t4's lane writes dword t4: lane 16q + m, m = 8 (t4 >> 1) + j, word t4 & 1
+    const uint32_t lo = (t4 & 1) ? w[1] : w[0], hi = (t4 & 1) ? w[NI / 4 - 1] : w[NI >= 12 ? 2 : 0];
+    *reinterpret_cast<uint32_t*>(page + a.L.vcode + h * 512 + (16 * q + 8 * (t4 >> 1) + j) * 8 + 4 * (t4 & 1)) =
+        (t4 & 2) ? hi : lo;
+  } else {                    // VCODE [h][4][d] bytes: token t4's lane writes bytes t4 of each dword
+    uint8_t* dst = page + a.L.vcode + (h * 4 + q) * D + j;
+#pragma unroll
+    for (int k = 0; k < NI / 4; ++k) dst[8 * (4 * k + t4)] = (uint8_t)(w[k] >> (8 * t4));
   }
 }
 
-// The value kernel alone, for pages whose layout has value sections only
-// (the spectral key path keeps its keys in pages of its own).
+// The recipe's page: workgroups [0, 2 h n) encode the residual of one 64-token
+// group of one head, the rest the values of 64 tokens of one head (8 waves x 8
+// tokens).  One launch for both: a commit of one codec page has 16 workgroups
+// of each, and they run side by side.  Measured at h_kv 8: 6.8 us for one codec
+// page at R 32 and 19.7 us for 63 at R 16; the two as kernels of their own, with
+// both residual operands from LDS and the FWHT's stages through LDS with a
+// barrier each, 21.7 + 7.5 and 27.1 + 27.1 us.
+template <int R>
+__global__ __launch_bounds__(512) void append_codes_kernel(const AppendKArgs a, int n_res) {
+  __shared__ ResidualLds<R, 16> s;
+  const int i = (int)blockIdx.x < n_res ? blockIdx.x : blockIdx.x - n_res;
+  const int u = i / a.h_kv, h = i - u * a.h_kv;
+  if ((int)blockIdx.x < n_res) {
+    encode_residual<R, 16, false>(a, s, u, h);
+  } else {
+    const int wave = threadIdx.x >> 6;
+    encode_values<128>(a, 4 * u + (wave >> 1), wave & 1, h, true);
+  }
+}
+
+// grid (residual groups of the call, h_kv), block 512 (general page).
+template <int R, int PER>
+__global__ __launch_bounds__(512) void gen_kres_kernel(const AppendKArgs a) {
+  __shared__ ResidualLds<R, PER> s;
+  encode_residual<R, PER, true>(a, s, blockIdx.x, blockIdx.y);
+}
+
+// grid (16-token pages of the call, h_kv), block 128: a wave for 8 tokens.
+template <int D>
+__global__ __launch_bounds__(128) void value_codes_kernel(const AppendKArgs a) {
+  encode_values<D>(a, blockIdx.x, threadIdx.x >> 6, blockIdx.y, !a.general);
+}
+
+// The smallest float x with (x / s) * s > mid, s = fl(sqrt(d)): the codes'
+// test as one compare (both operations are monotonic in x).  NaN (no such x)
+// where mid is not a number below infinity.
+static float code_cut(float mid, float s) {
+  if (!(mid < INFINITY)) return NAN;
+  auto above = [&](float x) {
+    volatile float q = x / s;
+    volatile float r = q * s;
+    return r > mid;
+  };
+  float x = std::max(mid, -3.0e38f);
+  for (int i = 0; i < 64 && above(x); ++i) x = std::nextafterf(x, -INFINITY);
+  for (int i = 0; i < 64 && !above(x); ++i) x = std::nextafterf(x, INFINITY);
+  return x;
+}
+
+void set_code_cuts(AppendKArgs& k, const float codebook[4], int d) {
+  const float s = std::sqrt((float)d);   // correctly rounded
+  for (int i = 0; i < 3; ++i) k.code_cuts[i] = code_cut((codebook[i] + codebook[i + 1]) / 2.0f, s);
+}
+
+// The values alone, for pages whose layout has value sections only (the
+// spectral key path keeps its keys in pages of its own).
 hipError_t launch_k2b_values(const AppendKArgs& a, int n_pages16, int h_kv, hipStream_t st) {
-  hipLaunchKernelGGL(k2b_v_kernel, dim3(n_pages16, h_kv), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(value_codes_kernel<128>, dim3(n_pages16, h_kv), dim3(128), 0, st, a);
   return hipGetLastError();
+}
+
+// Us of every page slot: the basis columns take C 64 bytes of LDS, above 64 KB
+// with the partial sums from C 1024 on (the limit is raised once).
+static hipError_t launch_us(const AppendKArgs& k, int n_slots, hipStream_t st) {
+  const size_t lds = (size_t)k.C * 16 * sizeof(float);
+  const bool vec = (reinterpret_cast<uintptr_t>(k.k_pre) & 15) == 0 && k.ksh % 8 == 0 && k.kst % 8 == 0;
+  const void* fn = vec ? (const void*)append_us_kernel<true> : (const void*)append_us_kernel<false>;
+  const hipError_t e = bmx_ensure_dynamic_lds(fn, lds);
+  if (e != hipSuccess) return e;
+  const dim3 grid(n_slots, k.R / 16);
+  if (vec) hipLaunchKernelGGL(append_us_kernel<true>, grid, dim3(256), lds, st, k);
+  else hipLaunchKernelGGL(append_us_kernel<false>, grid, dim3(256), lds, st, k);
+  return hipGetLastError();
+}
+
+template <int R>
+static void launch_gen_kres(const AppendKArgs& k, int per, dim3 grid, hipStream_t st) {
+  switch (per) {
+    case 1: hipLaunchKernelGGL((gen_kres_kernel<R, 1>), grid, dim3(512), 0, st, k); break;
+    case 2: hipLaunchKernelGGL((gen_kres_kernel<R, 2>), grid, dim3(512), 0, st, k); break;
+    case 4: hipLaunchKernelGGL((gen_kres_kernel<R, 4>), grid, dim3(512), 0, st, k); break;
+    case 8: hipLaunchKernelGGL((gen_kres_kernel<R, 8>), grid, dim3(512), 0, st, k); break;
+    case 16: hipLaunchKernelGGL((gen_kres_kernel<R, 16>), grid, dim3(512), 0, st, k); break;
+    default: hipLaunchKernelGGL((gen_kres_kernel<R, 32>), grid, dim3(512), 0, st, k); break;
+  }
 }
 
 }  // namespace bmx
@@ -249,18 +459,6 @@ using namespace bmx;
 static int afail(int code, const std::string& msg) {
   bmx_set_error(msg);
   return code;
-}
-
-// The Us kernel stages 16 key rows of C channels in LDS: above 64 KB (h_kv 16)
-// the launch needs the larger dynamic-LDS limit set once.
-template <int R>
-static hipError_t launch_us(const AppendKArgs& k, dim3 grid, size_t lds, hipStream_t st) {
-  if (lds > 65536) {
-    const hipError_t e = bmx_ensure_dynamic_lds((const void*)k2b_us_kernel<R>, lds);
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(k2b_us_kernel<R>, grid, dim3(256), lds, st, k);
-  return hipGetLastError();
 }
 
 extern "C" int bmx_k2b_append(const bmx_k2b_append_args* a, void* stream) {
@@ -280,23 +478,42 @@ extern "C" int bmx_k2b_append(const bmx_k2b_append_args* a, void* stream) {
     return afail(BMX_E_INVALID, "bmx_k2b_append: basis32 must be 16-byte aligned");
   if (a->v_dtype != BMX_K2B_F16 && a->v_dtype != BMX_K2B_F32 && a->v_dtype != BMX_K2B_BF16)
     return afail(BMX_E_INVALID, "bmx_k2b_append: v_dtype must be BMX_K2B_F16, _F32 or _BF16");
-  if (geo.general) return gen_append(a, (hipStream_t)stream);
   AppendKArgs k{};
-  k.h_kv = g.h_kv; k.R = g.rank; k.n_codec_pages = a->n_codec_pages;
+  k.h_kv = g.h_kv; k.R = geo.R; k.n_codec_pages = a->n_codec_pages;
+  k.C = geo.C(); k.log2d = __builtin_ctz((unsigned)geo.d); k.bits = geo.bits; k.general = geo.general;
   k.k_pre = a->k_pre; k.ksh = a->k_stride_h; k.kst = a->k_stride_t;
   k.v = a->v; k.vsh = a->v_stride_h; k.vst = a->v_stride_t; k.v_dtype = a->v_dtype;
   k.basis32 = a->basis32; k.basis16 = a->basis16; k.us_first = a->us_first;
   k.pages = a->pages; k.page_ids = a->page_ids; k.n_pool = a->n_pool_pages;
-  k.L = PageLayout::make(g.h_kv, g.rank);
-  for (int i = 0; i < 4; ++i) { k.codebook[i] = a->codebook[i]; k.v_sign_bits[i] = a->v_sign_bits[i]; }
+  if (geo.general) {
+    const GenLayout L = GenLayout::of(geo);
+    k.L.us = L.us; k.L.vnorm = L.vnorm; k.L.kscale = L.kscale; k.L.kres = L.kres; k.L.vcode = L.vcode;
+    k.L.bytes = L.bytes;
+  } else {
+    k.L = PageLayout::make(g.h_kv, g.rank);
+  }
+  for (int i = 0; i < 4; ++i) k.v_sign_bits[i] = a->v_sign_bits[i];
+  set_code_cuts(k, a->codebook, geo.d);
   hipStream_t st = (hipStream_t)stream;
-  const size_t us_lds = (size_t)kPT * (kD * g.h_kv + 2) * 2;
-  hipError_t le = g.rank == 32 ? launch_us<32>(k, dim3(a->n_codec_pages * 8), us_lds, st)
-                               : launch_us<16>(k, dim3(a->n_codec_pages * 8), us_lds, st);
-  if (le != hipSuccess) return afail(BMX_E_HIP, std::string("bmx_k2b_append: launch: ") + hipGetErrorString(le));
-  hipLaunchKernelGGL(k2b_kres_kernel, dim3(a->n_codec_pages * 2, g.h_kv), dim3(256), 0, st, k);
-  hipLaunchKernelGGL(k2b_v_kernel, dim3(a->n_codec_pages * 8, g.h_kv), dim3(256), 0, st, k);
-  hipError_t e = hipGetLastError();
+  const int slots = a->n_codec_pages * 8;
+  hipError_t e = launch_us(k, slots, st);
+  if (e != hipSuccess) return afail(BMX_E_HIP, std::string("bmx_k2b_append: launch: ") + hipGetErrorString(e));
+  if (!geo.general) {
+    const int n_res = a->n_codec_pages * 2 * g.h_kv;   // workgroups of the residual, and as many of the values
+    if (geo.R == 32) hipLaunchKernelGGL(append_codes_kernel<32>, dim3(2 * n_res), dim3(512), 0, st, k, n_res);
+    else hipLaunchKernelGGL(append_codes_kernel<16>, dim3(2 * n_res), dim3(512), 0, st, k, n_res);
+  } else {
+    const dim3 kgrid(a->n_codec_pages * (kCodec / geo.group), geo.h), vgrid(slots, geo.h);
+    const int per = geo.group * geo.d / 512;
+    if (geo.R == 16) launch_gen_kres<16>(k, per, kgrid, st);
+    else if (geo.R == 32) launch_gen_kres<32>(k, per, kgrid, st);
+    else if (geo.R == 64) launch_gen_kres<64>(k, per, kgrid, st);
+    else launch_gen_kres<128>(k, per, kgrid, st);
+    if (geo.d == 32) hipLaunchKernelGGL(value_codes_kernel<32>, vgrid, dim3(128), 0, st, k);
+    else if (geo.d == 64) hipLaunchKernelGGL(value_codes_kernel<64>, vgrid, dim3(128), 0, st, k);
+    else hipLaunchKernelGGL(value_codes_kernel<128>, vgrid, dim3(128), 0, st, k);
+  }
+  e = hipGetLastError();
   if (e != hipSuccess) return afail(BMX_E_HIP, std::string("bmx_k2b_append: launch: ") + hipGetErrorString(e));
   return BMX_OK;
 }

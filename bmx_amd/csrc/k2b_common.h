@@ -262,9 +262,10 @@ __device__ __forceinline__ void dq_store_tile(const DqTile16<DT>& tl, void* out,
   for (int u = 0; u < 4; ++u) dst[u] = src[u];
 }
 
-// Arguments of the k2b write kernels (k2b_append.hip).
+// Arguments of the k2b write kernels (k2b_append.hip), either page format.
 struct AppendKArgs {
   int h_kv, R, n_codec_pages, n_pool;
+  int C, log2d, bits, general;   // channels, log2(head_dim), key bits, general page
   const uint16_t* k_pre;
   int64_t ksh, kst;
   const void* v;
@@ -276,12 +277,14 @@ struct AppendKArgs {
   uint8_t* pages;
   const int32_t* page_ids;
   PageLayout L;
-  float codebook[4];
+  float code_cuts[3];            // set_code_cuts: a value's code counts the cuts it reaches
   uint32_t v_sign_bits[4];
 };
 
-// k2b_v_kernel over n_pages16 16-token pages of h_kv heads: norms and codes
-// into the VNORM and VCODE sections of a.L (k2b_append.hip).
+// The code thresholds of a codebook at head_dim d (k2b_append.hip).
+void set_code_cuts(AppendKArgs& k, const float codebook[4], int d);
+// Norms and codes of n_pages16 16-token pages of h_kv heads (head_dim 128) into
+// the VNORM and VCODE sections of a.L (k2b_append.hip).
 hipError_t launch_k2b_values(const AppendKArgs& a, int n_pages16, int h_kv, hipStream_t st);
 
 // Values of one 16-token page of one head into the wave's staging tile: the

@@ -64,10 +64,9 @@ struct GenLayout {
   static GenLayout of(const Geo& g) { return make(g.h, g.R, g.d, g.group, g.bits); }
 };
 
-// Entry points on the general page (k2b_general.hip), called by bmx_k2b_append,
+// Entry points on the general page (k2b_general.hip), called by
 // bmx_k2b_decode(_noalloc), bmx_k2b_decode_workspace_bytes and bmx_k2b_dequant
 // after their common argument checks; the geometry-specific checks are theirs.
-int gen_append(const bmx_k2b_append_args* a, hipStream_t st);
 std::string gen_decode_check(const bmx_k2b_decode_args* a);
 size_t gen_decode_workspace(const bmx_k2b_decode_args* a);
 int gen_decode(const bmx_k2b_decode_args* a, hipStream_t st, void* ws, size_t ws_cap, const std::string& name);

@@ -1,11 +1,7 @@
 // The k2b path on the general page (include/bmx_k2b.h): head_dim 32, 64 or
 // 128, rank 16..128, residual group 16..128 tokens, 2..4-bit keys, gfx950.
 //
-// Write (quantize-on-append), three launches per call as for the recipe's page:
-//   gen_us_kernel    Us = M * basis32 (or the first codec page's SVD factor), fp16
-//   gen_kres_kernel  R = M - Us16 * basis16^T, per-channel RTN over group tokens
-//   gen_v_kernel     per (token, head): fp16 norm, sign flip, FWHT, Lloyd codes
-// Read:
+// The read side (k2b_append.hip writes the pages):
 //   gen_split_kernel one workgroup per (split, head, sequence): every 16-token
 //                    page of the split rebuilt on MFMA (K^T = basis * Us^T),
 //                    residual and RoPE in registers (cos and sin of HF's fp32
@@ -18,9 +14,7 @@
 // Reference semantics: cache/packed_streaming.py:475-580 and 957-1060,
 // cache/codecs.py:616-649, 677-695, 786-796, quant/rtn.py:23-44,
 // quant/hadamard.py:12-33, cache/triton_dequant_attention.py:1232-1368.
-// Element-wise write steps follow the reference's operation order (divide,
-// round-half-even, divide-then-multiply by sqrt(d)); this file is built without
-// floating-point contraction.
+// This file is built without floating-point contraction.
 
 #include <algorithm>
 #include <string>
@@ -29,233 +23,6 @@
 #include "k2b_general.h"
 
 namespace bmx {
-
-struct GenAppendArgs {
-  GenLayout L;
-  const uint16_t* k_pre;
-  int64_t ksh, kst;
-  const void* v;
-  int64_t vsh, vst;
-  int v_dtype;
-  const float* basis32;
-  const uint16_t* basis16;
-  const float* us_first;
-  float codebook[4];
-  uint32_t v_sign_bits[4];
-  uint8_t* pages;
-  int32_t n_pool;
-  const int32_t* page_ids;   // [n_codec_pages * 8]
-};
-
-__device__ __forceinline__ uint8_t* gen_page(const GenAppendArgs& a, int slot) {
-  return a.pages + clamp_page(a.page_ids[slot], a.n_pool) * (int64_t)a.L.bytes;
-}
-
-// grid (n_codec_pages * 8), block 256 = 4 waves, one 16-token page each.
-// Us[t][r] = sum_c M[t][c] basis32[c][r] in fp32 (the reference's M @ V): the
-// page's 16 key rows staged in LDS, wave w sums channels [w C/4, (w+1) C/4) in
-// order, lane (t = lane & 15, rq = lane >> 4) owns ranks rq R/4 .. + R/4, and
-// the four partial sums are added in wave order.  The first codec page of a
-// sequence takes its SVD factor instead.
-template <int R>
-__global__ __launch_bounds__(256) void gen_us_kernel(const GenAppendArgs a) {
-  constexpr int RQ = R / 4;
-  extern __shared__ uint16_t s_m[];          // [kPT][C + 2] fp16 key rows
-  __shared__ float s_part[4][kPT][R + 1];
-  const int pg = blockIdx.x, cp = pg / 8, pl = pg % 8;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int C = a.L.C, D = a.L.d, ld = C + 2;
-  uint8_t* page = gen_page(a, pg);
-  uint16_t* us = reinterpret_cast<uint16_t*>(page + a.L.us);
-  if (a.us_first != nullptr && cp == 0) {
-    for (int e = tid; e < kPT * R; e += 256) us[e] = float_to_half_bits(a.us_first[pl * kPT * R + e]);
-    return;
-  }
-  for (int e = tid; e < kPT * C; e += 256) {
-    const int t = e / C, c = e % C;
-    s_m[t * ld + c] = a.k_pre[(c / D) * a.ksh + (int64_t)(pg * kPT + t) * a.kst + (c % D)];
-  }
-  __syncthreads();
-  const int t = lane & 15, rq = lane >> 4;
-  float acc[RQ];
-#pragma unroll
-  for (int k = 0; k < RQ; ++k) acc[k] = 0.f;
-  const int c0 = wave * (C / 4), c1 = c0 + C / 4;
-  for (int c = c0; c < c1; ++c) {
-    const float m = half_bits_to_float(s_m[t * ld + c]);
-    const float4* b = reinterpret_cast<const float4*>(a.basis32 + (int64_t)c * R + rq * RQ);
-#pragma unroll
-    for (int k4 = 0; k4 < RQ / 4; ++k4) {
-      const float4 bv = b[k4];
-      acc[4 * k4 + 0] = __builtin_fmaf(m, bv.x, acc[4 * k4 + 0]);
-      acc[4 * k4 + 1] = __builtin_fmaf(m, bv.y, acc[4 * k4 + 1]);
-      acc[4 * k4 + 2] = __builtin_fmaf(m, bv.z, acc[4 * k4 + 2]);
-      acc[4 * k4 + 3] = __builtin_fmaf(m, bv.w, acc[4 * k4 + 3]);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < RQ; ++k) s_part[wave][t][rq * RQ + k] = acc[k];
-  __syncthreads();
-  for (int e = tid; e < kPT * R; e += 256) {
-    const int tt = e / R, r = e % R;
-    const float v = ((s_part[0][tt][r] + s_part[1][tt][r]) + s_part[2][tt][r]) + s_part[3][tt][r];
-    us[e] = float_to_half_bits(v);
-  }
-}
-
-// grid (residual groups of the call, h_kv), block 256: the group's tokens x
-// the head's d channels.  Thread (channel j = tid % d, part tid / d) takes
-// tokens part, part + 256/d, ...: L = sum_r Us16[t][r] basis16[c][r] (ranks in
-// order), R = M - L; the channel's scale is max |R| over the group / qmax and
-// its codes clamp(rint(R / scale), -qmax - 1, qmax).  Dynamic LDS: the
-// group's Us16 rows and the head's basis16 rows (fp16, exact), then the codes.
-__global__ __launch_bounds__(256) void gen_kres_kernel(const GenAppendArgs a) {
-  const GenLayout& L = a.L;
-  const int gi = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-  const int D = L.d, R = L.R, NG = L.group, C = L.C;
-  const int gpp = kCodec / NG;                      // groups per codec page
-  const int cp = gi / gpp, g_in = gi % gpp;
-  const int slot0 = cp * 8 + g_in * (NG / kPT);     // first 16-token page slot of the group
-  extern __shared__ uint16_t s_dyn[];
-  uint16_t* s_us = s_dyn;                           // [NG][R]
-  uint16_t* s_b = s_us + NG * R;                    // [D][R]
-  int8_t* s_code = reinterpret_cast<int8_t*>(s_b + D * R);   // [NG][D]
-  __shared__ float s_amax[8][128];
-  for (int e = tid; e < NG * R; e += 256) {
-    const int t = e / R, r = e % R;
-    const uint8_t* page = gen_page(a, slot0 + t / kPT);
-    s_us[e] = *reinterpret_cast<const uint16_t*>(page + L.us + ((t % kPT) * R + r) * 2);
-  }
-  for (int e = tid; e < D * R; e += 256) s_b[e] = a.basis16[(int64_t)(h * D) * R + e];
-  __syncthreads();
-  const int j = tid % D, part = tid / D, parts = 256 / D, per = NG / parts;
-  const int qmax = (1 << (L.bits - 1)) - 1;
-  float res[64];   // per <= 64 (d >= 32 and group <= 128): fixed bounds keep it in registers
-  float amax = 0.f;
-#pragma unroll
-  for (int k = 0; k < 64; ++k) {
-    if (k >= per) break;
-    const int t = part + parts * k;
-    const int tg = cp * kCodec + g_in * NG + t;     // token within the call
-    float Lv = 0.f;
-    for (int r = 0; r < R; ++r)
-      Lv = __builtin_fmaf(half_bits_to_float(s_us[t * R + r]), half_bits_to_float(s_b[j * R + r]), Lv);
-    const float m = half_bits_to_float(a.k_pre[h * a.ksh + (int64_t)tg * a.kst + j]);
-    res[k] = m - Lv;
-    amax = fmaxf(amax, fabsf(res[k]));
-  }
-  s_amax[part][j] = amax;
-  __syncthreads();
-  float mx = s_amax[0][j];
-  for (int p = 1; p < parts; ++p) mx = fmaxf(mx, s_amax[p][j]);
-  const float scale = fmaxf(mx, 1e-12f) / (float)qmax;
-#pragma unroll
-  for (int k = 0; k < 64; ++k) {
-    if (k >= per) break;
-    float cq = rintf(res[k] / scale);
-    cq = fminf(fmaxf(cq, (float)(-qmax - 1)), (float)qmax);
-    s_code[(part + parts * k) * D + j] = (int8_t)cq;
-  }
-  if (part == 0) {
-    const int c = h * D + j, slot = c / L.per_slot, off = c % L.per_slot;
-    *reinterpret_cast<uint16_t*>(gen_page(a, slot0 + slot) + L.kscale + off * 2) = float_to_half_bits(scale);
-  }
-  __syncthreads();
-  // KRES: 8 channels (4 bytes) of one token per item, offset-binary nibbles
-  const int off = 1 << (L.bits - 1);
-  for (int e = tid; e < NG * (D / 8); e += 256) {
-    const int t = e / (D / 8), j8 = e % (D / 8);
-    uint32_t w = 0u;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) w |= (uint32_t)(s_code[t * D + 8 * j8 + i] + off) << (4 * i);
-    uint8_t* page = gen_page(a, slot0 + t / kPT);
-    *reinterpret_cast<uint32_t*>(page + L.kres + (h * kPT + t % kPT) * (D / 2) + 4 * j8) = w;
-  }
-}
-
-// grid (16-token pages of the call, h_kv), block 256: the page's 16 value rows
-// of one head.
-__global__ __launch_bounds__(256) void gen_v_kernel(const GenAppendArgs a) {
-  const GenLayout& L = a.L;
-  const int pg = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, D = L.d;
-  __shared__ float x[kPT][128];
-  __shared__ float s_norm[kPT];
-  __shared__ uint8_t code[kPT][128];
-  uint8_t* page = gen_page(a, pg);
-  for (int e = tid; e < kPT * D; e += 256) {
-    const int t = e / D, c = e % D;
-    const int64_t i = h * a.vsh + (int64_t)(pg * kPT + t) * a.vst + c;
-    float val;
-    if (a.v_dtype == BMX_K2B_F32)
-      val = static_cast<const float*>(a.v)[i];
-    else if (a.v_dtype == BMX_K2B_BF16)
-      val = __uint_as_float((uint32_t)static_cast<const uint16_t*>(a.v)[i] << 16);
-    else
-      val = half_bits_to_float(static_cast<const uint16_t*>(a.v)[i]);
-    x[t][c] = val;
-  }
-  __syncthreads();
-  // norms in the order torch's CPU 2-norm reduces a row (8 strided FMA
-  // accumulators, a left-to-right sum of them, a correctly rounded sqrt)
-  if (tid < kPT) {
-    const int t = tid;
-    float acc8[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) acc8[k] = 0.f;
-    for (int i = 0; i < D; i += 8) {
-#pragma unroll
-      for (int k = 0; k < 8; ++k) acc8[k] = __builtin_fmaf(x[t][i + k], x[t][i + k], acc8[k]);
-    }
-    float ss = acc8[0];
-#pragma unroll
-    for (int k = 1; k < 8; ++k) ss = ss + acc8[k];
-    const float nrm = fmaxf(__builtin_sqrtf(ss), 1e-12f);
-    const uint16_t nb = float_to_half_bits(nrm);
-    s_norm[t] = half_bits_to_float(nb);
-    *reinterpret_cast<uint16_t*>(page + L.vnorm + (h * kPT + t) * 2) = nb;
-  }
-  __syncthreads();
-  for (int e = tid; e < kPT * D; e += 256) {
-    const int t = e / D, c = e % D;
-    const float u = x[t][c] / s_norm[t];
-    x[t][c] = sign_neg(a.v_sign_bits, c) ? -u : u;
-  }
-  __syncthreads();
-  for (int hb = 1; hb < D; hb <<= 1) {   // FWHT stages as quant/hadamard.py:19-25
-    for (int e = tid; e < kPT * D / 2; e += 256) {
-      const int t = e / (D / 2), p = e % (D / 2);
-      const int i0 = (p / hb) * 2 * hb + (p % hb);
-      const float u = x[t][i0], w = x[t][i0 + hb];
-      x[t][i0] = u + w;
-      x[t][i0 + hb] = u - w;
-    }
-    __syncthreads();
-  }
-  const float sqrt_d = __builtin_sqrtf((float)D);   // fl32(sqrt(d)), applied as / then *
-  const float mid0 = (a.codebook[0] + a.codebook[1]) / 2.0f;
-  const float mid1 = (a.codebook[1] + a.codebook[2]) / 2.0f;
-  const float mid2 = (a.codebook[2] + a.codebook[3]) / 2.0f;
-  for (int e = tid; e < kPT * D; e += 256) {
-    const int t = e / D, c = e % D;
-    const float r = (x[t][c] / sqrt_d) * sqrt_d;
-    code[t][c] = (uint8_t)((r > mid0) + (r > mid1) + (r > mid2));
-  }
-  __syncthreads();
-  // VCODE [h][4][d]: byte (a, j) holds tokens 4a .. 4a + 3 of channel j; 4 channels per item
-  for (int e = tid; e < D; e += 256) {
-    const int aq = e / (D / 4), j4 = e % (D / 4);
-    uint32_t w = 0u;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int j = 4 * j4 + i;
-      uint32_t byte = 0u;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) byte |= (uint32_t)code[4 * aq + t][j] << (2 * t);
-      w |= byte << (8 * i);
-    }
-    *reinterpret_cast<uint32_t*>(page + L.vcode + (h * 4 + aq) * D + 4 * j4) = w;
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Read side.  MFMA 16x16x16 f16 fragments (lane l = 16 qd + n): A holds
@@ -818,40 +585,6 @@ void gen_plan(const bmx_k2b_decode_args* a, const Geo& g, int* n_split, int* pps
 }  // namespace
 
 namespace bmx {
-
-int gen_append(const bmx_k2b_append_args* a, hipStream_t st) {
-  const Geo g = Geo::from(a->geom);
-  const std::string why = g.check();
-  if (!why.empty()) return gfail(BMX_E_INVALID, "bmx_k2b_append: " + why);
-  GenAppendArgs k{};
-  k.L = GenLayout::of(g);
-  k.k_pre = a->k_pre; k.ksh = a->k_stride_h; k.kst = a->k_stride_t;
-  k.v = a->v; k.vsh = a->v_stride_h; k.vst = a->v_stride_t; k.v_dtype = a->v_dtype;
-  k.basis32 = a->basis32; k.basis16 = a->basis16; k.us_first = a->us_first;
-  for (int i = 0; i < 4; ++i) { k.codebook[i] = a->codebook[i]; k.v_sign_bits[i] = a->v_sign_bits[i]; }
-  k.pages = a->pages; k.n_pool = a->n_pool_pages; k.page_ids = a->page_ids;
-  const int np = a->n_codec_pages * 8;
-  const size_t us_lds = (size_t)kPT * (g.C() + 2) * 2;
-  hipError_t e = hipSuccess;
-#define BMX_GEN_US(R_)                                                                          \
-  if (g.R == R_) {                                                                              \
-    if (us_lds > 65536) e = bmx_ensure_dynamic_lds((const void*)gen_us_kernel<R_>, us_lds);      \
-    if (e == hipSuccess) hipLaunchKernelGGL(gen_us_kernel<R_>, dim3(np), dim3(256), us_lds, st, k); \
-  }
-  BMX_GEN_US(16) BMX_GEN_US(32) BMX_GEN_US(64) BMX_GEN_US(128)
-#undef BMX_GEN_US
-  if (e != hipSuccess) return gfail(BMX_E_HIP, std::string("bmx_k2b_append: LDS limit: ") + hipGetErrorString(e));
-  const size_t kres_lds = (size_t)(g.group * g.R + g.d * g.R) * 2 + (size_t)g.group * g.d;
-  if (kres_lds > 65536) {
-    e = bmx_ensure_dynamic_lds((const void*)gen_kres_kernel, kres_lds);
-    if (e != hipSuccess) return gfail(BMX_E_HIP, std::string("bmx_k2b_append: LDS limit: ") + hipGetErrorString(e));
-  }
-  hipLaunchKernelGGL(gen_kres_kernel, dim3(a->n_codec_pages * (kCodec / g.group), g.h), dim3(256), kres_lds, st, k);
-  hipLaunchKernelGGL(gen_v_kernel, dim3(np, g.h), dim3(256), 0, st, k);
-  e = hipGetLastError();
-  if (e != hipSuccess) return gfail(BMX_E_HIP, std::string("bmx_k2b_append: launch: ") + hipGetErrorString(e));
-  return BMX_OK;
-}
 
 size_t gen_decode_workspace(const bmx_k2b_decode_args* a) {
   const Geo g = Geo::from(a->geom);

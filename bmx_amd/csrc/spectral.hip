@@ -1915,7 +1915,8 @@ extern "C" int32_t bmx_spectral_append(const bmx_spectral_append_args* a, void* 
     v.h_kv = a->L.h_kv; v.n_pool = a->n_v_pool;
     v.v = a->v; v.vsh = a->v_sh; v.vst = a->v_st; v.v_dtype = a->v_dtype;
     v.pages = a->v_pages; v.page_ids = a->v_page_ids; v.L = value_layout(a->L.h_kv);
-    for (int i = 0; i < 4; ++i) { v.codebook[i] = a->v_codebook[i]; v.v_sign_bits[i] = a->v_sign_bits[i]; }
+    for (int i = 0; i < 4; ++i) v.v_sign_bits[i] = a->v_sign_bits[i];
+    set_code_cuts(v, a->v_codebook, kD);
     e = launch_k2b_values(v, 4 * a->n_groups, a->L.h_kv, st);
   }
   if (e != hipSuccess) {
