@@ -165,6 +165,39 @@ __device__ __forceinline__ float4_t load_q4(const void* base, int64_t idx, int i
                   __builtin_bit_cast(float, r.y << 16), __builtin_bit_cast(float, r.y & 0xffff0000u)};
 }
 
+// Four query elements as they lie in memory, loaded without a branch on the
+// dtype: 8 bytes at element idx, and for fp32 the next 8 (16-bit dtypes: the
+// same 8 again).  load_q4 converts inside its branch, so a run of its calls
+// waits for each load before the next is issued; these are all in flight
+// together, and cvt_q4 converts them once they are needed.
+struct RawQ4 {
+  uint2 a, b;
+};
+__device__ __forceinline__ RawQ4 load_raw_q4(const void* base, int64_t idx, int io) {
+  const char* p = static_cast<const char*>(base) + (idx << (io == kIoF32 ? 2 : 1));
+  return {*reinterpret_cast<const uint2*>(p), *reinterpret_cast<const uint2*>(p + (io == kIoF32 ? 8 : 0))};
+}
+template <int N>
+__device__ __forceinline__ void cvt_q4(const RawQ4 (&r)[N], int io, float4_t (&out)[N]) {
+  if (io == kIoF32) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      out[i] = float4_t{__uint_as_float(r[i].a.x), __uint_as_float(r[i].a.y), __uint_as_float(r[i].b.x),
+                        __uint_as_float(r[i].b.y)};
+  } else if (io == kIoF16) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const half2_t lo = as_h2(r[i].a.x), hi = as_h2(r[i].a.y);
+      out[i] = float4_t{(float)lo[0], (float)lo[1], (float)hi[0], (float)hi[1]};
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      out[i] = float4_t{__uint_as_float(r[i].a.x << 16), __uint_as_float(r[i].a.x & 0xffff0000u),
+                        __uint_as_float(r[i].a.y << 16), __uint_as_float(r[i].a.y & 0xffff0000u)};
+  }
+}
+
 __device__ __forceinline__ uint32_t bf16_bits(float v) {   // round to nearest even, NaN kept
   uint32_t u = __builtin_bit_cast(uint32_t, v);
   u = (u & 0x7fffffffu) > 0x7f800000u ? (u | 0x00400000u) : u + 0x7fffu + ((u >> 16) & 1u);
@@ -271,7 +304,6 @@ __host__ __device__ __forceinline__ size_t partial_bytes(size_t rows, size_t spl
 constexpr int kCmbWaves = 4;
 constexpr int kCmbThreads = 64 * kCmbWaves;
 constexpr int kChunk = 16;                  // channels per merge unit
-constexpr int kChunks = kD / kChunk;
 constexpr int kCmbSplits = 4;               // split blocks per wave per pass
 constexpr int kCmbTokens = 2;               // window-token blocks per wave per pass
 
@@ -282,7 +314,7 @@ struct CombineKArgs {
   int max_packed_len;
   void* out;               // [B][h_kv][G][128] in io_dtype
   int io_dtype;
-  const uint16_t* ws_acc;   // partial records (store_partial_record)
+  const void* ws_acc;       // partial records (store_partial_record; fp32 on the general page)
   const float* ws_ml;
   const float* ws_win;
   const uint16_t* v_tail;
@@ -300,6 +332,17 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_row(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
+
+// v_mov_b32_dpp: lanes enabled by BANK (4-lane banks of each 16-lane row) take
+// src from the DPP-selected lane, the others keep old.
+template <int CTRL, int BANK = 0xF>
+__device__ __forceinline__ float dpp(float old, float src) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old),
+                                                               __builtin_bit_cast(int, src), CTRL, 0xF,
+                                                               BANK, false));
+}
+constexpr int kRowShr = 0x110;  // + n: lane i of a row reads lane i - n
+constexpr int kRowRor = 0x120;  // + n: rotate within the row
 
 // All-reduce over the 16 lanes of a row with DPP (quad xor 1, quad xor 2,
 // half-row mirror, row mirror): every lane gets the same value.
@@ -330,14 +373,16 @@ __device__ __forceinline__ float part_weight(float mi, float M) {
 // kTok: window-token blocks per wave per pass: kCmbTokens (128 tokens per
 // pass), or 4 for windows of more than 128 rows (up to 255 between commits),
 // so that the window is one pass, one memory round trip.
-template <bool kRotated, int kTok>
+// kDim: head_dim; Rec: the records' element (uint16_t: fp16 bits; float: the
+// general page's fp32 records, whose empty attention -- no token at all -- is 0).
+template <bool kRotated, int kTok, int kDim = kD, class Rec = uint16_t>
 __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs a) {
   const int ch = blockIdx.x, r = blockIdx.y, b = blockIdx.z;
   const int h = r / a.G;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, p = lane & 15, c4 = lane >> 4;
   const int S_slots = a.max_splits;
   const int64_t row = (int64_t)b * a.h_kv * a.G + r;   // (b, h, g) row
-  const uint16_t* accb = a.ws_acc + (row * kChunks + ch) * (int64_t)S_slots * kChunk + 4 * c4;
+  const Rec* accb = static_cast<const Rec*>(a.ws_acc) + (row * (kDim / kChunk) + ch) * (int64_t)S_slots * kChunk + 4 * c4;
   const float* mlb = a.ws_ml + row * S_slots * 2;
   const float* swb = a.ws_win + row * a.tail_cap;
   const uint16_t* vb = a.v_tail + b * a.ts_b + h * a.ts_h + kChunk * ch + 4 * c4;
@@ -358,9 +403,13 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
     for (int u = 0; u < kCmbSplits; ++u) {
       const int i = min(elem(j0, u), S - 1);
       ml[u] = *reinterpret_cast<const f2_t*>(mlb + 2 * (int64_t)i);
-      const uint2 r = *reinterpret_cast<const uint2*>(accb + (int64_t)i * kChunk);
-      const half2_t lo = as_h2(r.x), hi = as_h2(r.y);
-      pv[u] = float4_t{(float)lo[0], (float)lo[1], (float)hi[0], (float)hi[1]};
+      if constexpr (sizeof(Rec) == 4) {
+        pv[u] = *reinterpret_cast<const float4_t*>(accb + (int64_t)i * kChunk);
+      } else {
+        const uint2 r = *reinterpret_cast<const uint2*>(accb + (int64_t)i * kChunk);
+        const half2_t lo = as_h2(r.x), hi = as_h2(r.y);
+        pv[u] = float4_t{(float)lo[0], (float)lo[1], (float)hi[0], (float)hi[1]};
+      }
     }
   };
   auto load_tokens = [&](int t0, int t_end) {   // t_end >= 1
@@ -511,22 +560,23 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
   if (p == 0) {
     const float M = fmaxf(Mp, Mt);
     const float wp = part_weight(Mp, M), wt = part_weight(Mt, M);
-    const float inv = 1.0f / (lp * wp + lt * wt);
+    const float den = lp * wp + lt * wt, inv = 1.0f / den;
     float4_t o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = (y[i] * wp + z[i] * wt) * inv;
-    store_o4(a.out, row * kD + kChunk * ch + 4 * c4, o, a.io_dtype);
+    if (sizeof(Rec) == 4 && !(den > 0.f)) o = float4_t{0.f, 0.f, 0.f, 0.f};
+    store_o4(a.out, row * kDim + kChunk * ch + 4 * c4, o, a.io_dtype);
   }
 }
 
 // The merge launch: the window in one pass when it holds more than 128 rows.
-template <bool kRotated>
+template <bool kRotated, int kDim = kD, class Rec = uint16_t>
 inline void launch_combine(const CombineKArgs& c, int rows, int batch, hipStream_t st) {
-  const dim3 grid(kChunks, rows, batch);
+  const dim3 grid(kDim / kChunk, rows, batch);
   if (c.tail_cap > 16 * kCmbWaves * kCmbTokens)
-    hipLaunchKernelGGL((combine_kernel<kRotated, 4>), grid, dim3(kCmbThreads), 0, st, c);
+    hipLaunchKernelGGL((combine_kernel<kRotated, 4, kDim, Rec>), grid, dim3(kCmbThreads), 0, st, c);
   else
-    hipLaunchKernelGGL((combine_kernel<kRotated, kCmbTokens>), grid, dim3(kCmbThreads), 0, st, c);
+    hipLaunchKernelGGL((combine_kernel<kRotated, kCmbTokens, kDim, Rec>), grid, dim3(kCmbThreads), 0, st, c);
 }
 
 }  // namespace bmx

@@ -120,17 +120,6 @@ struct DecodeKArgs {
   float* ws_win;          // [B][h_kv][G][tail_cap] window scores, base 2
 };
 
-// v_mov_b32_dpp: lanes enabled by BANK (4-lane banks of each 16-lane row) take
-// src from the DPP-selected lane, the others keep old.
-template <int CTRL, int BANK = 0xF>
-__device__ __forceinline__ float dpp(float old, float src) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old),
-                                                               __builtin_bit_cast(int, src), CTRL, 0xF,
-                                                               BANK, false));
-}
-constexpr int kRowShr = 0x110;  // + n: lane i of a row reads lane i - n
-constexpr int kRowRor = 0x120;  // + n: rotate within the row
-
 // x from the DPP-selected lane, every lane written (foldable into a DPP ALU op).
 template <int CTRL>
 __device__ __forceinline__ float dpp_all(float x) {

@@ -2,14 +2,14 @@
 // 128, rank 16..128, residual group 16..128 tokens, 2..4-bit keys, gfx950.
 //
 // The read side (k2b_append.hip writes the pages):
-//   gen_split_kernel one workgroup per (split, head, sequence): every 16-token
-//                    page of the split rebuilt on MFMA (K^T = basis * Us^T),
-//                    residual and RoPE in registers (cos and sin of HF's fp32
-//                    angle times rope_scaling, rounded to fp16: the
-//                    reference's shared tables), scores K^T Q^T on MFMA,
-//                    online softmax, P V on MFMA in the rotated value domain
-//   gen_merge_kernel one workgroup per (query, head, sequence): the splits'
-//                    partials, the inverse Hadamard, the recent window
+//   gen_split_kernel one workgroup of 8 waves per (split, head block, sequence),
+//                    a wave per KV head (or several per head when there are
+//                    fewer heads than waves), 4 pages at a time: RoPE tables
+//                    shared by the heads in LDS, keys rebuilt on MFMA (K^T =
+//                    basis * Us^T), residual and rotation in registers, scores
+//                    K^T Q^T on MFMA, online softmax, V^T P^T on MFMA in the
+//                    rotated value domain, the inverse Hadamard at the end
+//   combine_kernel   (decode_shared.h) merges the splits and the recent window
 //   gen_dequant_kernel  dense keys and values of committed pages (prefill)
 // Reference semantics: cache/packed_streaming.py:475-580 and 957-1060,
 // cache/codecs.py:616-649, 677-695, 786-796, quant/rtn.py:23-44,
@@ -25,16 +25,10 @@
 namespace bmx {
 
 // ---------------------------------------------------------------------------
-// Read side.  MFMA 16x16x16 f16 fragments (lane l = 16 qd + n): A holds
+// Dequant.  MFMA 16x16x16 f16 fragments (lane l = 16 qd + n): A holds
 // A[n][4qd .. 4qd+3], B holds B[4qd .. 4qd+3][n], the result D[4qd + e][n].
 //   K^T tile rt (channels 16rt ..): A = basis rows 16rt + n, ranks 16ks + 4qd ..
 //     (LDS), B = Us[token n][16ks + 4qd ..] -> lane: K[16rt + 4qd + e][token n]
-//   S^T = K^T Q^T: A = that tile (token n, channels 16rt + 4qd + e), B = query
-//     n's channels 16rt + 4qd + e, both as fp16 high and low parts
-//     -> lane: score of token 4qd + e for query n
-//   O = P V: A = those weights (query n, tokens 4qd + e), B = value level times
-//     norm of token 4qd + e, channel n + 16ct (both high + low parts)
-//     -> lane: O[query 4qd + e][n + 16ct]
 // RoPE pairs channels j and j + d/2: tiles rt and rt + d/32 of the same lane.
 // ---------------------------------------------------------------------------
 struct GenReadArgs {
@@ -49,30 +43,6 @@ struct GenReadArgs {
   float level[4];
   uint32_t v_sign_bits[4];
 };
-
-struct GenDecodeArgs {
-  GenReadArgs r;
-  int G, n_split, pps;             // splits per sequence, 16-token pages per split
-  const void* q;
-  int io_dtype;
-  const int32_t* packed_len;
-  int max_packed_len;
-  float qscale;                    // sm_scale * log2(e): scores in base 2
-  float* ws_acc;                   // [B][h][G][n_split][d] unnormalised sums (rotated values)
-  float* ws_ml;                    // [B][h][G][n_split][2] (max, sum)
-  // the merge
-  void* out;
-  const uint16_t* k_tail;
-  const uint16_t* v_tail;
-  int64_t ts_b, ts_h, ts_t;
-  int tail_cap, tail_bf16;
-  const int32_t* tail_len;
-  WinNew nw;
-};
-
-__device__ __forceinline__ half4_t gen_h4(float4_t v) {
-  return half4_t{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-}
 
 __device__ __forceinline__ const uint8_t* gen_read_page(const GenReadArgs& a, int b, int p) {
   const int32_t pid = a.page_table ? a.page_table[(int64_t)b * a.max_pages + p] : b * a.max_pages + p;
@@ -118,13 +88,7 @@ __device__ __forceinline__ void gen_keys(const GenReadArgs& a, const uint8_t* pg
 
 // RoPE of the lane's keys at position pos: mode 1 exact fp32 cos/sin, mode 2
 // the fp16-rounded tables (cos and sin times rope_scaling, then fp16).
-// kFast: cos/sin of HF's fp32 angle fl(pos * inv_freq) from its fraction of a
-// revolution (the product scaled by 1/2pi in double, its fraction rounded to
-// fp32) and the hardware sin/cos of revolutions, ~1e-6 absolute: the decode's
-// tables are rounded to fp16 after it (the library's sincosf takes the long
-// argument reduction for the angles of long contexts and was the decode's
-// bound).  Without kFast, sincosf of the fp32 angle.
-template <int D, bool kFast>
+template <int D>
 __device__ __forceinline__ void gen_rope(const GenReadArgs& a, float4_t kt[D / 16], int pos, int qd, int mode) {
   constexpr int NP = D / 32;
 #pragma unroll
@@ -133,14 +97,7 @@ __device__ __forceinline__ void gen_rope(const GenReadArgs& a, float4_t kt[D / 1
     for (int e = 0; e < 4; ++e) {
       const float ang = (float)pos * a.inv_freq[16 * rt + 4 * qd + e];
       float sn, cs;
-      if constexpr (kFast) {
-        const double rev = (double)ang * 0.15915494309189535;
-        const float fr = (float)(rev - floor(rev));
-        cs = __builtin_amdgcn_cosf(fr);
-        sn = __builtin_amdgcn_sinf(fr);
-      } else {
-        sincosf(ang, &sn, &cs);
-      }
+      sincosf(ang, &sn, &cs);
       cs = cs * a.rope_scaling;
       sn = sn * a.rope_scaling;
       if (mode == 2) {
@@ -153,331 +110,593 @@ __device__ __forceinline__ void gen_rope(const GenReadArgs& a, float4_t kt[D / 1
     }
 }
 
-template <int D, int R>
-__global__ __launch_bounds__(256) void gen_split_kernel(const GenDecodeArgs a) {
-  constexpr int NT = D / 16, LDB = R + 4;
-  const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, qd = lane >> 4;
-  const int H = a.r.L.h, G = a.G;
-  // the basis rows during the page loop, the waves' partial sums after it
-  constexpr int kBBytes = D * LDB * 2, kOBytes = 4 * 16 * (D + 1) * 4;
-  __shared__ __align__(16) uint8_t s_buf[kBBytes > kOBytes ? kBBytes : kOBytes];
-  __shared__ float s_m[4][16], s_l[4][16];
-  uint16_t* s_B = reinterpret_cast<uint16_t*>(s_buf);
-  float (*s_o)[16][D + 1] = reinterpret_cast<float (*)[16][D + 1]>(s_buf);
-  const uint16_t* basis = a.r.basis + (int64_t)b * a.r.basis_stride + (int64_t)(h * D) * R;
-  for (int e = tid; e < D * R; e += 256) s_B[(e / R) * LDB + e % R] = basis[e];
-  // query n's channels 16ks + 4qd .. as fp16 high and low parts (scaled to base 2)
-  half4_t qh[NT], ql[NT];
+// ---------------------------------------------------------------------------
+// Decode.  Fragments of the 16x16x32 f16 MFMA (lane l = 16 qd + n): A holds
+// A[n][8qd .. 8qd+7], B holds B[8qd .. 8qd+7][n], the result D[4qd + e][n].
+//   K^T tile rt: A = the basis row of the channel that row n stands for, ranks
+//     32ks + 8qd .., B = Us[token n][32ks + 8qd ..] -> lane: channel of row
+//     4qd + e, token n.  Row 4qd + e of tile rt < d/32 stands for channel
+//     qd d/8 + 4rt + e, of tile rt + d/32 for that channel + d/2: a lane's
+//     channels are two runs of d/8, so its codes, scales and table entries are
+//     contiguous, and both channels of a RoPE pair are in one lane
+//   S^T = K^T Q^T: the keys as fp16 high and low parts (kh, kl), the queries
+//     too (qh, ql): one product of (kh, kl) against (qh, qh) per tile and one of
+//     (kh, kh') against (ql, ql') per tile pair: kl ql is below 2^-22
+//     -> lane: score of token 4qd + e for query n
+//   V^T P^T: A = the levels (fp16 high and low parts) of channel n d/16 + ct,
+//     tokens 4qd .. 4qd+3 (one code byte through an LDS table), B = the lane's own
+//     P norm as high and low parts: (lh, lh) against (ph, pl) per page and
+//     (ll, ll') against (ph, ph') per page pair
+//     -> lane: channel (4qd + e) d/16 + ct for query n
+// G queries fill G of the 16 columns; pages are compacted SW columns apart (as
+// k2b_decode_split_kernel does), so the softmax runs once per 16/SW pages.
+//
+// What bounds it: VALU issue and the fixed latency of two launches.  A page of
+// one head takes ~135 VALU (residual 48, rotation 32, high and low parts 32)
+// and, a quarter of its quad's softmax and products, ~45 more at d 64; the
+// HBM floor of 32,640 tokens at d 64, rank 16, h_kv 8 is 2.6 us.  Measured there
+// (G 4, 128-row window): split 17.6 + merge 4.5 us, 20.6 us a call; a workgroup
+// per (split, head) with a page at a time per wave, the rotation remade per head
+// and page (22 of them, f64 included, per RoPE pair) and a merge workgroup per
+// query took 31.6 + 8.5 us, 37.9 us a call.  d 128, rank 64: 92 -> 39 us a call.
+// Kept in 32 bits as before: keys, weights and partial sums (fp16 pairs on MFMA).
+// ---------------------------------------------------------------------------
+struct GenDecodeArgs {
+  GenReadArgs r;
+  int G, n_split, hpb, wph;        // workgroups of a sequence and head block, heads of a block, waves of a head
+  int win_tiles, win_wgs;          // 16-token tiles of the window, workgroups a sequence has for them alone
+  int div32;                       // (n_split + 1) * quads < 2^32
+  float inv_per_slot;              // 1 / L.per_slot
+  int b0;                          // the call's sequence that block z = 0 serves (the pointers start there)
+  const void* q;
+  int io_dtype;
+  const int32_t* packed_len;
+  int max_packed_len;
+  float qscale;                    // sm_scale * log2(e): scores in base 2
+  float* ws_acc;                   // [B][h][G][d/16][n_split wph][16] fp32 records (means over the split)
+  float* ws_ml;                    // [B][h][G][n_split wph][2] (max, sum)
+  float* ws_win;                   // [B][h][G][tail_cap] window scores, base 2
+  const uint16_t* k_tail;
+  int64_t ts_b, ts_h, ts_t;
+  int tail_cap, tail_bf16;
+  WinNew nw;
+};
+
+constexpr int kGenQuad = 4;        // pages a wave takes at a time
+constexpr int kGenTables = 4;      // RoPE tables (64 positions each) in LDS
+constexpr int kGenIds = 64;        // page ids held per lane vector
+template <int D>
+constexpr int gen_cs_row() { return D / 2 + 4; }   // dwords per position row of a table (rows 4 banks apart)
+template <int D>
+constexpr size_t gen_lds() { return (size_t)kGenTables * 64 * gen_cs_row<D>() * 4; }
+// 8 waves a workgroup (2 per SIMD), or 4 where the basis and query fragments need
+// more than the 256 registers that leaves a wave
+constexpr int gen_waves(int D, int R) { return D == 128 || R == 128 ? 4 : 8; }
+
+// N bytes at p (16, 8, 4 or 2) as dwords
+template <int N>
+struct GenBytes {
+  uint32_t w[(N + 3) / 4];
+  __device__ __forceinline__ void load(const uint8_t* p) {
+    if constexpr (N == 16) {
+      const uint4 v = *reinterpret_cast<const uint4*>(p);
+      w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+    } else if constexpr (N == 8) {
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
+      w[0] = v.x; w[1] = v.y;
+    } else if constexpr (N == 4) {
+      w[0] = *reinterpret_cast<const uint32_t*>(p);
+    } else {
+      w[0] = *reinterpret_cast<const uint16_t*>(p);
+    }
+  }
+};
+
+__device__ __forceinline__ half2_t gen_rtz(float x, float y) {
+  return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(x, y));
+}
+
+// x and y as fp16 high parts (towards zero) and the fp16 low parts that remain
+// (x = h + l to 2^-21).  m1: -1 in a register the compiler cannot see through,
+// so that x - h reads the fp16 h in place (v_fma_mix_f32; exact), with no
+// conversion instruction.
+__device__ __forceinline__ void gen_split2(float x, float y, float m1, uint32_t& hi, uint32_t& lo) {
+  const half2_t h = gen_rtz(x, y);
+  hi = as_u32(h);
+  lo = as_u32(gen_rtz(__builtin_fmaf((float)h[0], m1, x), __builtin_fmaf((float)h[1], m1, y)));
+}
+
+// One 16-token tile of one head's recent window against its G queries, in
+// fp32: lane (token n, channel quarter qd).  Rows given apart are also stored
+// into the window buffer.
+template <int D>
+__device__ __forceinline__ void gen_window_tile(const GenDecodeArgs& a, int b, int h, int j, int n, int qd) {
+  constexpr int NQ = D / 16;   // 4-channel pieces of the lane's quarter
+  const int H = a.r.L.h, t = 16 * j + n, i_new = fresh_row(a.nw, t);
+  const int64_t tb = (int64_t)b * a.ts_b + (int64_t)h * a.ts_h;
+  const uint16_t* row = (i_new >= 0 ? a.nw.k + (int64_t)b * a.nw.sb + (int64_t)h * a.nw.sh + (int64_t)i_new * a.nw.st
+                                    : a.k_tail + tb + (int64_t)(t < a.tail_cap ? t : 0) * a.ts_t) + qd * (D / 4);
+  uint2 kv[NQ];
+#pragma unroll
+  for (int c = 0; c < NQ; ++c) kv[c] = *reinterpret_cast<const uint2*>(row + 4 * c);
+  const bool bf = __builtin_amdgcn_readfirstlane(a.tail_bf16) != 0;
+  const int64_t r0 = ((int64_t)b * H + h) * a.G;
+  constexpr int GB = D == 128 ? 2 : 4;   // queries whose loads are in flight with the tile's
+  RawQ4 qr[GB][NQ];
+  auto load_q = [&](int g0) {
+#pragma unroll
+    for (int i = 0; i < GB; ++i)
+#pragma unroll
+      for (int c = 0; c < NQ; ++c)
+        qr[i][c] = load_raw_q4(a.q, (r0 + min(g0 + i, a.G - 1)) * D + qd * (D / 4) + 4 * c, a.io_dtype);
+  };
+  load_q(0);
+  if (i_new >= 0) {
+    uint16_t* dst = a.nw.k_dst + tb + (int64_t)t * a.ts_t + qd * (D / 4);
+#pragma unroll
+    for (int c = 0; c < NQ; ++c) *reinterpret_cast<uint2*>(dst + 4 * c) = kv[c];
+  }
+  for (int g0 = 0; g0 < a.G; g0 += GB) {
+    if (g0 > 0) load_q(g0);
+#pragma unroll
+    for (int i = 0; i < GB; ++i) {
+      float s = 0.f;
+      float4_t qv[NQ];
+      cvt_q4(qr[i], a.io_dtype, qv);
+#pragma unroll
+      for (int c = 0; c < NQ; ++c) {
+        const uint2 r = kv[c];
+        const float4_t x = bf ? float4_t{__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u),
+                                         __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u)}
+                              : float4_t{half_bits_to_float(r.x & 0xffff), half_bits_to_float(r.x >> 16),
+                                         half_bits_to_float(r.y & 0xffff), half_bits_to_float(r.y >> 16)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_fmaf(qv[c][e] * a.qscale, x[e], s);
+      }
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
+      if (qd == 0 && t < a.tail_cap && g0 + i < a.G) a.ws_win[(r0 + g0 + i) * a.tail_cap + t] = s;
+    }
+  }
+}
+
+template <int D, int R, int SW>
+__global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const GenDecodeArgs a) {
+  constexpr int NWV = gen_waves(D, R), NT = D / 16, NP = NT / 2, NK = R >= 32 ? R / 32 : 1;
+  constexpr int KQ = R >= 32 ? 8 : 4;            // ranks per lane of one K^T product
+  constexpr int NSLOT = 16 / SW, NCR = kGenQuad / NSLOT;
+  constexpr int RUN = D / 8;                     // channels of a lane's run
+  constexpr int CSROW = gen_cs_row<D>();
+  constexpr int PF = D == 128 ? 2 : 4;           // pages whose key data is in flight or in use
+  typedef _Float16 hvec_t __attribute__((ext_vector_type(KQ)));
+  extern __shared__ __attribute__((aligned(16))) uint32_t s_cs[];   // [tables][64][CSROW]: fp16 (cos, sin)
+  // the 4 levels of a code byte (tokens 4a .. 4a + 3): fp16 high parts twice (the
+  // product's operand as it is), low parts
+  __shared__ uint4 s_lvh[256];
+  __shared__ uint2 s_lvl[256];
+  // the scalar arguments of the prologue requested at once: one round trip
+  asm volatile("" ::"s"(a.r.pages), "s"(a.r.page_table), "s"(a.r.max_pages), "s"(a.r.n_pool), "s"(a.r.basis),
+               "s"(a.r.basis_stride), "s"(a.r.rope_scaling), "s"(a.G), "s"(a.n_split), "s"(a.hpb), "s"(a.wph),
+               "s"(a.div32), "s"(a.inv_per_slot), "s"(a.b0), "s"(a.q), "s"(a.io_dtype), "s"(a.packed_len),
+               "s"(a.max_packed_len), "s"(a.qscale));
+  asm volatile("" ::"s"(a.r.L.us), "s"(a.r.L.vnorm), "s"(a.r.L.kscale), "s"(a.r.L.kres), "s"(a.r.L.vcode),
+               "s"(a.r.L.bytes), "s"(a.r.L.h), "s"(a.r.L.bits), "s"(a.r.L.slots), "s"(a.r.L.per_slot),
+               "s"(a.r.level[0]), "s"(a.r.level[1]), "s"(a.r.level[2]), "s"(a.r.level[3]));
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int n = lane & 15, qd = lane >> 4;
+  const GenLayout& L = a.r.L;
+  const int split = blockIdx.x, b = blockIdx.z, G = a.G;
+  // the window's (16-token tile, head) pairs, dealt over workgroups and waves:
+  // over the sequence's own workgroups at their end, or over win_wgs more that do
+  // nothing else
+  auto window_pairs = [&](int wg, int n) {
+    const int n_wg = n * gridDim.y, n_pairs = a.win_tiles * L.h;
+    for (int p = wg + n * blockIdx.y + wave * n_wg; p < n_pairs; p += NWV * n_wg) {
+      const int j = p / L.h;
+      gen_window_tile<D>(a, b, p - j * L.h, j, lane & 15, qd);
+    }
+  };
+  if (split >= a.n_split) {
+    window_pairs(split - a.n_split, a.win_wgs);
+    return;
+  }
+  const float freq = a.r.inv_freq[tid & (D / 2 - 1)];   // the RoPE frequency this thread makes table entries of
+  const int len_raw = a.packed_len[b];
+  const int sub = wave / a.hpb, h_own = blockIdx.y * a.hpb + wave % a.hpb;
+  const bool active = sub < a.wph && h_own < L.h;
+  const int h = active ? h_own : 0;
+  // ---- the basis rows and the query, before anything waits for the length
+  hvec_t bw[NT][NK];
+  half8_t qhh[NT], qll[NP];                      // (qh, qh) of each tile, (ql, ql') of each tile pair
+  RawQ4 qx[NT];
+  if (a.max_packed_len > 0) {
+    const uint16_t* basis = a.r.basis + (int64_t)b * a.r.basis_stride;
+    auto row = [&](int rt) {
+      return basis + (int64_t)(h * D + (n >> 2) * RUN + 4 * (rt % NP) + (n & 3) + (rt / NP) * (D / 2)) * R + KQ * qd;
+    };
+    if ((reinterpret_cast<uintptr_t>(basis) & 15) == 0) {
+#pragma unroll
+      for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+        for (int ks = 0; ks < NK; ++ks) bw[rt][ks] = *reinterpret_cast<const hvec_t*>(row(rt) + 4 * KQ * ks);
+    } else {
+#pragma unroll
+      for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+        for (int ks = 0; ks < NK; ++ks)
+#pragma unroll
+          for (int i = 0; i < KQ; ++i) bw[rt][ks][i] = __builtin_bit_cast(_Float16, row(rt)[4 * KQ * ks + i]);
+    }
+    const int64_t qrow = (((int64_t)b * L.h + h) * G + (n < G ? n : 0)) * D;
+#pragma unroll
+    for (int rt = 0; rt < NT; ++rt)
+      qx[rt] = load_raw_q4(a.q, qrow + RUN * qd + 4 * (rt % NP) + (rt / NP) * (D / 2), a.io_dtype);
+  }
+  // the workgroup's quads, first of the host's bound of the length (so that the
+  // first pages are requested without a wait for the device length)
+  int n_pages, q0, q1;
+  auto set_range = [&](int len) {
+    n_pages = len / kPT;
+    const int n_quads = (n_pages + kGenQuad - 1) / kGenQuad;
+    if (a.div32) {   // every product fits 32 bits
+      q0 = (int)((uint32_t)split * (uint32_t)n_quads / (uint32_t)a.n_split);
+      q1 = (int)(((uint32_t)split + 1u) * (uint32_t)n_quads / (uint32_t)a.n_split);
+    } else {
+      q0 = (int)((int64_t)split * n_quads / a.n_split);
+      q1 = (int)((int64_t)(split + 1) * n_quads / a.n_split);
+    }
+    q0 = __builtin_amdgcn_readfirstlane(q0);
+    q1 = __builtin_amdgcn_readfirstlane(q1);
+  };
+  set_range(a.max_packed_len);
+
+  // ---- page ids, 64 from an 8-page boundary at or before the wave's next quad
+  // (a residual group of up to 128 tokens lies within 8 pages)
+  int id_base = 0, idv = 0;
+  auto load_ids = [&](int quad) {
+    id_base = (kGenQuad * quad) & ~7;
+    const int p = min(id_base + lane, max(a.r.max_pages - 1, 0));
+    idv = a.r.page_table ? a.r.page_table[(int64_t)b * a.r.max_pages + p] : (b + a.b0) * a.r.max_pages + p;
+    idv = (int)clamp_page(idv, a.r.n_pool);
+  };
+  auto page_of = [&](int p) -> const uint8_t* {   // uniform p
+    return a.r.pages + (int64_t)__builtin_amdgcn_readlane(idv, p - id_base) * L.bytes;
+  };
+  auto page_of_lane = [&](int p) -> const uint8_t* {   // p per lane
+    return a.r.pages + (int64_t)__shfl(idv, p - id_base) * L.bytes;
+  };
+  // ---- the lane's scales: channels h d + RUN qd .. and + d/2, in the page
+  // slot of the residual group that holds them
+  const int c_lo = h * D + RUN * qd, c_hi = c_lo + D / 2;
+  const int slot_lo = (int)(((float)c_lo + 0.5f) * a.inv_per_slot), slot_hi = (int)(((float)c_hi + 0.5f) * a.inv_per_slot);
+  const int off_lo = L.kscale + 2 * (c_lo - slot_lo * L.per_slot), off_hi = L.kscale + 2 * (c_hi - slot_hi * L.per_slot);
+  const int kres_off = L.kres + (h * kPT + n) * (D / 2) + (RUN / 2) * qd, vcode_off = L.vcode + (h * 4 + qd) * D + NT * n;
+  struct Key {
+    hvec_t us[NK];
+    GenBytes<RUN / 2> lo, hi;
+    GenBytes<2 * RUN < 16 ? 2 * RUN : 16> slo[(2 * RUN + 15) / 16], shi[(2 * RUN + 15) / 16];
+  };
+  Key key[PF];
+  GenBytes<NT> vc[kGenQuad];
+  half4_t vn[NCR];
+  auto last_page = [&](int p) { return min(p, n_pages - 1); };
+  auto load_key = [&](Key& k, int p_any) {
+    const int p = last_page(p_any), p0 = p & ~(L.slots - 1);
+    const uint8_t* pg = page_of(p);
+#pragma unroll
+    for (int ks = 0; ks < NK; ++ks)
+      k.us[ks] = *reinterpret_cast<const hvec_t*>(pg + L.us + (n * R + 4 * KQ * ks + KQ * qd) * 2);
+    k.lo.load(pg + kres_off);
+    k.hi.load(pg + kres_off + D / 4);
+    const uint8_t* gl = page_of_lane(p0 + slot_lo) + off_lo;
+    const uint8_t* gh = page_of_lane(p0 + slot_hi) + off_hi;
+#pragma unroll
+    for (int i = 0; i < (2 * RUN + 15) / 16; ++i) {
+      k.slo[i].load(gl + 16 * i);
+      k.shi[i].load(gh + 16 * i);
+    }
+  };
+  const int my_slot = NSLOT > 1 ? n / SW : 0;   // page slot of this lane after compaction
+  auto load_values = [&](int quad) {
+#pragma unroll
+    for (int pp = 0; pp < kGenQuad; ++pp) vc[pp].load(page_of(last_page(kGenQuad * quad + pp)) + vcode_off);
+#pragma unroll
+    for (int r = 0; r < NCR; ++r)
+      vn[r] = *reinterpret_cast<const half4_t*>(page_of_lane(last_page(kGenQuad * quad + r * NSLOT + my_slot)) +
+                                                L.vnorm + (h * kPT + 4 * qd) * 2);
+  };
+
+  // ---- the wave's first quad in flight
+  int qi;                                        // the wave's quads: q0 + sub, + wph, ...
+  auto load_first = [&]() {
+    qi = q0 + sub;
+    if (active && qi < q1) {
+      load_ids(qi);
+#pragma unroll
+      for (int i = 0; i < PF; ++i) load_key(key[i], kGenQuad * qi + i);
+      load_values(qi);
+    }
+  };
+  load_first();
+  for (int i = tid; i < 256; i += 64 * NWV) {
+    uint32_t hi[2] = {0u, 0u}, lo[2] = {0u, 0u};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const float x = level4((i >> (2 * t)) & 3, a.r.level[0], a.r.level[1], a.r.level[2], a.r.level[3]);
+      const _Float16 xh = (_Float16)x;
+      hi[t >> 1] |= half_bits(xh) << (16 * (t & 1));
+      lo[t >> 1] |= half_bits((_Float16)(x - (float)xh)) << (16 * (t & 1));
+    }
+    s_lvh[i] = make_uint4(hi[0], hi[1], hi[0], hi[1]);
+    s_lvl[i] = make_uint2(lo[0], lo[1]);
+  }
   {
     const float sc = n < G ? a.qscale : 0.f;
-    const int64_t qrow = (((int64_t)b * H + h) * G + (n < G ? n : 0)) * D;
+    float4_t qf[NT];
+    cvt_q4(qx, a.io_dtype, qf);
 #pragma unroll
-    for (int ks = 0; ks < NT; ++ks) {
-      const float4_t x = load_q4(a.q, qrow + 16 * ks + 4 * qd, a.io_dtype) * sc;
-      qh[ks] = gen_h4(x);
-      ql[ks] = gen_h4(x - float4_t{(float)qh[ks][0], (float)qh[ks][1], (float)qh[ks][2], (float)qh[ks][3]});
-    }
-  }
-  const int n_tok = min(max(a.packed_len[b], 0), a.max_packed_len);
-  const int n_pages = n_tok / kPT;
-  const int p_begin = split * a.pps, p_end = min(p_begin + a.pps, n_pages);
-  __syncthreads();
-  float m_run = -INFINITY, l_part = 0.f;
-  float4_t o[NT];
-#pragma unroll
-  for (int ct = 0; ct < NT; ++ct) o[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
-  for (int p = p_begin + wave; p < p_end; p += 4) {
-    const uint8_t* pg = gen_read_page(a.r, b, p);
-    const GenLayout& L = a.r.L;
-    const half4_t vn = *reinterpret_cast<const half4_t*>(pg + L.vnorm + (h * kPT + 4 * qd) * 2);
-    uint32_t vc[NT];
-#pragma unroll
-    for (int ct = 0; ct < NT; ++ct) vc[ct] = pg[L.vcode + (h * 4 + qd) * D + n + 16 * ct];
-    float4_t kt[NT];
-    gen_keys<D, R>(a.r, pg, s_B, b, p, h, n, qd, kt);
-    gen_rope<D, true>(a.r, kt, p * kPT + n, qd, 2);   // the reference's shared fp16 tables
-    // keys and queries as fp16 high + low parts: the three products that
-    // matter carry both to about 2^-22
-    float4_t st = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < NT; ++ks) {
-      const half4_t kh = gen_h4(kt[ks]);
-      const half4_t kl = gen_h4(kt[ks] - float4_t{(float)kh[0], (float)kh[1], (float)kh[2], (float)kh[3]});
-      st = __builtin_amdgcn_mfma_f32_16x16x16f16(kh, qh[ks], st, 0, 0, 0);
-      st = __builtin_amdgcn_mfma_f32_16x16x16f16(kh, ql[ks], st, 0, 0, 0);
-      st = __builtin_amdgcn_mfma_f32_16x16x16f16(kl, qh[ks], st, 0, 0, 0);
-    }
-    // online softmax of query n over the page's 16 tokens (4 per lane)
-    float mloc = fmaxf(fmaxf(st[0], st[1]), fmaxf(st[2], st[3]));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
-    const float m_new = fmaxf(m_run, mloc);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    float4_t pw;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) pw[e] = __builtin_amdgcn_exp2f(st[e] - m_new);
-    l_part = l_part * alpha + ((pw[0] + pw[1]) + (pw[2] + pw[3]));
-    m_run = m_new;
-    // the output rows are queries 4qd + e: their rescale factors from lanes 4qd + e
-    float4_t al;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) al[e] = __shfl(alpha, 4 * qd + e);
-    const half4_t ph = gen_h4(pw);
-    const half4_t pl = gen_h4(pw - float4_t{(float)ph[0], (float)ph[1], (float)ph[2], (float)ph[3]});
-#pragma unroll
-    for (int ct = 0; ct < NT; ++ct) {
-      half4_t vh, vl;   // norm times level, fp16 high + low parts
+    for (int rt = 0; rt < NT; ++rt) {
+      const float4_t x = qf[rt] * sc;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x = (float)vn[e] * a.r.level[(vc[ct] >> (2 * e)) & 3u];
-        vh[e] = (_Float16)x;
-        vl[e] = (_Float16)(x - (float)vh[e]);
+        const _Float16 xh = (_Float16)x[e];
+        qhh[rt][e] = qhh[rt][4 + e] = xh;
+        qll[rt % NP][4 * (rt / NP) + e] = (_Float16)(x[e] - (float)xh);
       }
-      o[ct] *= al;
-      o[ct] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, vh, o[ct], 0, 0, 0);
-      o[ct] = __builtin_amdgcn_mfma_f32_16x16x16f16(pl, vh, o[ct], 0, 0, 0);
-      o[ct] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, vl, o[ct], 0, 0, 0);
     }
   }
-  l_part += __shfl_xor(l_part, 16);
-  l_part += __shfl_xor(l_part, 32);
-  __syncthreads();   // every wave is done with the basis rows
-  if (qd == 0) {
-    s_m[wave][n] = m_run;
-    s_l[wave][n] = l_part;
+  float4_t acc[NT];
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) acc[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  const int len = __builtin_amdgcn_readfirstlane(min(max(len_raw, 0), a.max_packed_len));
+  if (len != a.max_packed_len) {                 // a shorter sequence: its own quads
+    set_range(len);
+    load_first();
   }
+  // nibble e of a half word: its mask, the exponent field of 2^(23 - 4e) and
+  // that power plus the codes' offset (in registers: one AND-OR a code)
+  uint32_t nib_m[4], nib_e[4];
+  float nib_b[4], m1 = -1.0f, zero = -0.0f;   // m1, zero: see gen_split2
+  asm volatile("" : "+s"(m1), "+s"(zero));
 #pragma unroll
-  for (int ct = 0; ct < NT; ++ct)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s_o[wave][4 * qd + e][n + 16 * ct] = o[ct][e];
-  __syncthreads();
-  const int64_t rows = ((int64_t)b * H + h) * G;
-  for (int it = tid; it < G * D; it += 256) {
-    const int g = it / D, c = it % D;
-    float M = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, s_m[w][g]);
-    float acc = 0.f, l = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float wt = s_m[w][g] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[w][g] - M);
-      acc += wt * s_o[w][g][c];
-      l += wt * s_l[w][g];
-    }
-    const int64_t slot = (rows + g) * a.n_split + split;
-    a.ws_acc[slot * D + c] = acc;
-    if (c == 0) {
-      a.ws_ml[2 * slot] = M;
-      a.ws_ml[2 * slot + 1] = l;
-    }
+  for (int e = 0; e < 4; ++e) {
+    nib_m[e] = 15u << (4 * e);
+    nib_e[e] = 0x4B000000u - (0x02000000u * e);
+    nib_b[e] = (float)((8388608 >> (4 * e)) + (1 << (L.bits - 1)));
+    asm volatile("" : "+v"(nib_m[e]));
+    asm volatile("" : "+s"(nib_e[e]));
   }
-}
 
-__device__ __forceinline__ void gen_store_io(void* base, int64_t idx, float v, int io) {
-  if (io == kIoF32) {
-    reinterpret_cast<float*>(base)[idx] = v;
-  } else if (io == kIoF16) {
-    reinterpret_cast<uint16_t*>(base)[idx] = float_to_half_bits(v);
-  } else {
-    reinterpret_cast<uint16_t*>(base)[idx] = (uint16_t)bf16_bits(v);
-  }
-}
-
-// Sum over the 128 threads of v (every thread gets the result); s_red holds 2.
-__device__ __forceinline__ float gen_block_sum(float v, float* s_red) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return s_red[0] + s_red[1];
-}
-
-__device__ __forceinline__ float gen_block_max(float v, float* s_red) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return fmaxf(s_red[0], s_red[1]);
-}
-
-// grid (G, h_kv, B), block 128: output row (b, h, g).  The splits' partials
-// merge by the split softmax's weights, the inverse value rotation (H_d, the
-// codec's signs, 1/d) turns the sum into values, and the recent window
-// (scored here; rows given apart read from there and copied into the window
-// buffer by query 0's workgroup) joins with its own weight.  Thread (part,
-// c4) takes 4 channels of splits / window rows part, part + P, ...  Every
-// first-pass load of the four phases (the split maxima and sums, the
-// thread's splits' partial sums, its window row's key, its window value rows)
-// is issued before any of them is used, so the phases share one memory round
-// trip; splits and window rows beyond the first pass are loaded in later
-// passes.
-template <int D>
-__global__ __launch_bounds__(128) void gen_merge_kernel(const GenDecodeArgs a) {
-  constexpr int NC4 = D / 4, P = 128 / NC4;   // channel quads, row parts
-  constexpr int kMS = 64 / P;                 // first-pass splits per thread: 64 splits
-  constexpr int kMV = (D == 128 ? 64 : 128) / P;   // first-pass window value rows per thread
-  const int g = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
-  const int H = a.r.L.h, G = a.G, S = a.n_split;
-  const int c4 = tid % NC4, part = tid / NC4;
-  __shared__ float s_x[D], s_q[D], s_red[2];
-  __shared__ float4_t s_part[P][NC4];
-  __shared__ float s_s[4096];
-  const int64_t row = ((int64_t)b * H + h) * G + g;
-  const float2* ml = reinterpret_cast<const float2*>(a.ws_ml) + row * S;
-  const float* accr = a.ws_acc + row * S * D + 4 * c4;
-  const bool wbf = __builtin_amdgcn_readfirstlane(a.tail_bf16) != 0;
-  const int64_t tb = (int64_t)b * a.ts_b + (int64_t)h * a.ts_h;
-  const int64_t nb = (int64_t)b * a.nw.sb + (int64_t)h * a.nw.sh;
-  auto wrow = [&](const uint16_t* fresh, const uint16_t* buf, int t) {
-    const int i = fresh_row(a.nw, t);
-    return i >= 0 ? fresh + nb + (int64_t)i * a.nw.st : buf + tb + (int64_t)t * a.ts_t;
-  };
-  auto cvt4 = [&](uint2 r) {   // 4 window elements as fp32
-    return wbf ? float4_t{__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u),
-                          __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u)}
-               : float4_t{half_bits_to_float(r.x & 0xffff), half_bits_to_float(r.x >> 16),
-                          half_bits_to_float(r.y & 0xffff), half_bits_to_float(r.y >> 16)};
-  };
-  const int Tc = a.tail_cap;   // the host's bound of the window
-  // ---- every first-pass load at once
-  float4_t qx = {0.f, 0.f, 0.f, 0.f};
-  if (tid < D) qx = load_q4(a.q, row * D + (tid & ~3), a.io_dtype);
-  const float2 mlv = ml[min(tid, S - 1)];
-  float msp[kMS];
-  float4_t accv[kMS];
-#pragma unroll
-  for (int k = 0; k < kMS; ++k) {
-    const int sc = min(part + P * k, S - 1);
-    msp[k] = ml[sc].x;
-    accv[k] = *reinterpret_cast<const float4_t*>(accr + (int64_t)sc * D);
-  }
-  uint2 kv[NC4], vv[kMV];
-  if (Tc > 0) {
-    const uint16_t* kr = wrow(a.nw.k, a.k_tail, min(tid, Tc - 1));
-#pragma unroll
-    for (int c = 0; c < NC4; ++c) kv[c] = *reinterpret_cast<const uint2*>(kr + 4 * c);
-#pragma unroll
-    for (int k = 0; k < kMV; ++k)
-      vv[k] = *reinterpret_cast<const uint2*>(wrow(a.nw.v, a.v_tail, min(part + P * k, Tc - 1)) + 4 * c4);
-  }
-  const int T = a.tail_len ? min(max(a.tail_len[b], 0), Tc) : a.nw.T;
-  if (tid < D) s_q[tid] = qx[tid & 3] * a.qscale;   // published by the block max's barriers
-
-  // ---- packed partials: the max, then weighted sums
-  float mx = tid < S ? mlv.x : -INFINITY;
-  for (int s2 = tid + 128; s2 < S; s2 += 128) mx = fmaxf(mx, ml[s2].x);
-  const float Mp = gen_block_max(mx, s_red);
-  float lp = 0.f;
-  float4_t acc = {0.f, 0.f, 0.f, 0.f};
-  if (Mp != -INFINITY) {
-    if (tid < S && mlv.x != -INFINITY) lp = __builtin_amdgcn_exp2f(mlv.x - Mp) * mlv.y;
-    for (int s2 = tid + 128; s2 < S; s2 += 128) {
-      const float2 v = ml[s2];
-      lp += v.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(v.x - Mp) * v.y;
-    }
-#pragma unroll
-    for (int k = 0; k < kMS; ++k) {
-      const bool ok = part + P * k < S && msp[k] != -INFINITY;
-      const float w = ok ? __builtin_amdgcn_exp2f(msp[k] - Mp) : 0.f;
-      acc += ok ? w * accv[k] : float4_t{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll 4
-    for (int s2 = part + P * kMS; s2 < S; s2 += P) {
-      const float m = ml[s2].x;
-      const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - Mp);
-      acc += w * *reinterpret_cast<const float4_t*>(accr + (int64_t)s2 * D);
-    }
-  }
-  const float Lp = gen_block_sum(lp, s_red);
-  s_part[part][c4] = acc;
-  __syncthreads();
-  if (tid < NC4) {
-    float4_t t = s_part[0][tid];
-    for (int q = 1; q < P; ++q) t += s_part[q][tid];
-    *reinterpret_cast<float4_t*>(&s_x[4 * tid]) = t;
-  }
-  __syncthreads();
-  for (int hb = 1; hb < D; hb <<= 1) {   // unnormalised H_d, Sylvester order
-    float u = 0.f, v = 0.f;
-    int i0 = 0;
-    if (tid < D / 2) {
-      i0 = (tid / hb) * 2 * hb + (tid % hb);
-      u = s_x[i0];
-      v = s_x[i0 + hb];
+  for (int qt = q0; qt < q1; qt += kGenTables) {
+    const int nt = min(kGenTables, q1 - qt);
+    if (qt != q0) __syncthreads();               // every wave is done with the previous tables
+    // (cos, sin) of HF's fp32 angle fl(pos * inv_freq) from its fraction of a
+    // revolution (the product scaled by 1/2pi in double, its fraction rounded
+    // to fp32) and the hardware sin/cos of revolutions, ~1e-6 absolute, times
+    // rope_scaling, rounded to fp16: the reference's shared tables
+    {
+      const int j = tid & (D / 2 - 1);
+      for (int p = tid / (D / 2); p < 64 * nt; p += 64 * NWV / (D / 2)) {
+        const float ang = (float)(64 * qt + p) * freq;
+        const double rev = (double)ang * 0.15915494309189535;
+        const float fr = (float)(rev - floor(rev));
+        const half2_t v = {(_Float16)fp32_rounded(__builtin_amdgcn_cosf(fr) * a.r.rope_scaling),
+                           (_Float16)fp32_rounded(__builtin_amdgcn_sinf(fr) * a.r.rope_scaling)};
+        s_cs[p * CSROW + j] = as_u32(v);
+      }
     }
     __syncthreads();
-    if (tid < D / 2) {
-      s_x[i0] = u + v;
-      s_x[i0 + hb] = u - v;
+    if (!active) continue;
+    for (; qi < qt + nt; qi += a.wph) {
+      const int qn = qi + a.wph;                 // the wave's next quad
+      const bool more = qn < q1;
+      const int p0 = kGenQuad * qi;
+      float4_t st[kGenQuad];
+#pragma unroll
+      for (int pp = 0; pp < kGenQuad; ++pp) {
+        Key& k = key[pp % PF];
+        float4_t kt[NT];
+        const float4_t z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt) {
+          kt[rt] = z;
+#pragma unroll
+          for (int ks = 0; ks < NK; ++ks) {
+            if constexpr (R >= 32) kt[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bw[rt][ks], k.us[ks], kt[rt], 0, 0, 0);
+            else kt[rt] = __builtin_amdgcn_mfma_f32_16x16x16f16(bw[rt][ks], k.us[ks], kt[rt], 0, 0, 0);
+          }
+        }
+        // residual code times scale: the nibble at bit 4k of a half word under
+        // the exponent of 2^(23 - 4k) reads as 2^(23 - 4k) + code, exactly
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int i = 4 * (rt % NP) + e;     // position in the run
+            const uint32_t w = rt < NP ? k.lo.w[i / 8] : k.hi.w[i / 8];
+            const uint32_t sw = rt < NP ? k.slo[i / 8].w[(i % 8) / 2] : k.shi[i / 8].w[(i % 8) / 2];
+            const float c = __uint_as_float(((i % 8 < 4 ? w : w >> 16) & nib_m[e]) | nib_e[e]) - nib_b[e];
+            kt[rt][e] = __builtin_fmaf((float)as_h2(sw)[i & 1], c, kt[rt][e]);
+          }
+        // RoPE and the high and low parts, a tile pair at a time
+        const uint32_t* cs = s_cs + ((qi - qt) * 64 + pp * kPT + n) * CSROW + RUN * qd;
+        float4_t s = z;
+#pragma unroll
+        for (int rt = 0; rt < NP; ++rt) {
+          const uint4 cv = *reinterpret_cast<const uint4*>(cs + 4 * rt);
+          const uint32_t cw[4] = {cv.x, cv.y, cv.z, cv.w};
+          float xr[4], yr[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const half2_t c2 = as_h2(cw[e]);
+            const float x = kt[rt][e], y = kt[rt + NP][e];
+            xr[e] = __builtin_fmaf(-y, (float)c2[1], __builtin_fmaf(x, (float)c2[0], zero));
+            yr[e] = __builtin_fmaf(x, (float)c2[1], __builtin_fmaf(y, (float)c2[0], zero));
+          }
+          union { uint32_t w[4]; half8_t v; } kx, ky, kh;
+          gen_split2(xr[0], xr[1], m1, kx.w[0], kx.w[2]);
+          gen_split2(xr[2], xr[3], m1, kx.w[1], kx.w[3]);
+          gen_split2(yr[0], yr[1], m1, ky.w[0], ky.w[2]);
+          gen_split2(yr[2], yr[3], m1, ky.w[1], ky.w[3]);
+          kh.w[0] = kx.w[0]; kh.w[1] = kx.w[1]; kh.w[2] = ky.w[0]; kh.w[3] = ky.w[1];
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kx.v, qhh[rt], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(ky.v, qhh[rt + NP], s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh.v, qll[rt], s, 0, 0, 0);
+        }
+        if (p0 + pp >= n_pages) s = float4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        st[pp] = s;
+        // the page's registers take the page PF further on
+        const int quad_n = pp + PF < kGenQuad ? qi : qn, p_n = kGenQuad * quad_n + (pp + PF) % kGenQuad;
+        if (quad_n == qi || more) {
+          if (quad_n != qi && kGenQuad * qn + kGenQuad > id_base + kGenIds) load_ids(qn);
+          load_key(k, p_n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // ---- compaction: page r NSLOT + s to columns [s SW, (s + 1) SW)
+      float4_t cr[NCR];
+#pragma unroll
+      for (int r = 0; r < NCR; ++r) {
+        cr[r] = st[r * NSLOT];
+        if constexpr (NSLOT == 4) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            cr[r][i] = dpp<kRowShr + 4, 0x2>(cr[r][i], st[r * NSLOT + 1][i]);
+            cr[r][i] = dpp<kRowShr + 8, 0x4>(cr[r][i], st[r * NSLOT + 2][i]);
+            cr[r][i] = dpp<kRowShr + 12, 0x8>(cr[r][i], st[r * NSLOT + 3][i]);
+          }
+        } else if constexpr (NSLOT == 2) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) cr[r][i] = dpp<kRowShr + 8, 0xC>(cr[r][i], st[r * NSLOT + 1][i]);
+        }
+      }
+      // ---- online softmax (one running max per query, the accumulator rescaled
+      // only when some max grows)
+      float mx = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < NCR; ++r) mx = fmaxf(mx, fmaxf(fmaxf(cr[r][0], cr[r][1]), fmaxf(cr[r][2], cr[r][3])));
+      if (__any(mx > m_run)) {
+        if constexpr (NSLOT == 4) mx = fmaxf(mx, dpp_row<kRowRor + 4>(mx));
+        if constexpr (NSLOT >= 2) mx = fmaxf(mx, dpp_row<kRowRor + 8>(mx));
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) acc[ct] *= alpha;
+        m_run = m_new;
+      }
+      uint2 ph[NCR], pl[NCR];
+#pragma unroll
+      for (int r = 0; r < NCR; ++r) {
+        float x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float p = __builtin_amdgcn_exp2f(cr[r][i] - m_run);
+          l_run += p;
+          x[i] = p * (float)vn[r][i];
+        }
+        gen_split2(x[0], x[1], m1, ph[r].x, pl[r].x);
+        gen_split2(x[2], x[3], m1, ph[r].y, pl[r].y);
+      }
+      // ---- V^T P^T, two pages at a time
+#pragma unroll
+      for (int u = 0; u < kGenQuad / 2; ++u) {
+        const int pa = 2 * u, pb = 2 * u + 1;
+        const bool on_a = NSLOT == 1 || my_slot == pa % NSLOT, on_b = NSLOT == 1 || my_slot == pb % NSLOT;
+        const uint2 z2 = make_uint2(0u, 0u);
+        const uint2 ha = on_a ? ph[pa / NSLOT] : z2, la = on_a ? pl[pa / NSLOT] : z2;
+        const uint2 hb = on_b ? ph[pb / NSLOT] : z2, lb = on_b ? pl[pb / NSLOT] : z2;
+        union U { uint4 e; half8_t v; };
+        U ba, bb, bl;
+        ba.e = make_uint4(ha.x, ha.y, la.x, la.y);
+        bb.e = make_uint4(hb.x, hb.y, lb.x, lb.y);
+        bl.e = make_uint4(ha.x, ha.y, hb.x, hb.y);
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) {
+          const uint32_t ia = (vc[pa].w[ct / 4] >> (8 * (ct % 4))) & 0xFFu;
+          const uint32_t ib = (vc[pb].w[ct / 4] >> (8 * (ct % 4))) & 0xFFu;
+          U ua, ub, ul;
+          ua.e = s_lvh[ia];
+          ub.e = s_lvh[ib];
+          const uint2 xa = s_lvl[ia], xb = s_lvl[ib];
+          ul.e = make_uint4(xa.x, xa.y, xb.x, xb.y);
+          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ua.v, ba.v, acc[ct], 0, 0, 0);
+          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ub.v, bb.v, acc[ct], 0, 0, 0);
+          acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ul.v, bl.v, acc[ct], 0, 0, 0);
+        }
+      }
+      if (more) load_values(qn);
     }
-    __syncthreads();
   }
-  float op = 0.f;
-  if (tid < D) {
-    op = s_x[tid] / (float)D;
-    if (sign_neg(a.r.v_sign_bits, tid)) op = -op;
-  }
-  // ---- the recent window: scores, one row per thread (its first from kv)
-  auto score = [&](const uint2 (&k4)[NC4]) {
-    float sc = 0.f;
+
+  if (a.win_wgs == 0) window_pairs(split, a.n_split);
+  if (!active) return;
+  // ---- fold the page slots, then the inverse Hadamard of channel
+  // (4qd + e) NT + ct: ct and e in registers, qd across the rows; signs, 1/d
+  if constexpr (NSLOT == 4) {
 #pragma unroll
-    for (int c = 0; c < NC4; ++c) {
-      const float4_t x = cvt4(k4[c]);
+    for (int ct = 0; ct < NT; ++ct)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sc = __builtin_fmaf(s_q[4 * c + e], x[e], sc);
-    }
-    return sc;
-  };
-  float mw = -INFINITY;
-  if (tid < T) {
-    const float sc = score(kv);
-    s_s[tid] = sc;
-    mw = sc;
+      for (int i = 0; i < 4; ++i) acc[ct][i] += dpp_row<kRowRor + 4>(acc[ct][i]);
+    l_run += dpp_row<kRowRor + 4>(l_run);
   }
-  for (int t = tid + 128; t < T; t += 128) {
-    const uint16_t* kr = wrow(a.nw.k, a.k_tail, t);
-    uint2 k4[NC4];
+  if constexpr (NSLOT >= 2) {
 #pragma unroll
-    for (int c = 0; c < NC4; ++c) k4[c] = *reinterpret_cast<const uint2*>(kr + 4 * c);
-    const float sc = score(k4);
-    s_s[t] = sc;
-    mw = fmaxf(mw, sc);
-  }
-  mw = gen_block_max(mw, s_red);   // its barriers also publish s_s
-  float lw = 0.f;
-  for (int t = tid; t < T; t += 128) lw += __builtin_amdgcn_exp2f(s_s[t] - mw);
-  float4_t ow = {0.f, 0.f, 0.f, 0.f};
+    for (int ct = 0; ct < NT; ++ct)
 #pragma unroll
-  for (int k = 0; k < kMV; ++k) {
-    const int t = part + P * k;
-    if (t < T) ow += __builtin_amdgcn_exp2f(s_s[t] - mw) * cvt4(vv[k]);
+      for (int i = 0; i < 4; ++i) acc[ct][i] += dpp_row<kRowRor + 8>(acc[ct][i]);
+    l_run += dpp_row<kRowRor + 8>(l_run);
   }
-#pragma unroll 4
-  for (int t = part + P * kMV; t < T; t += P)
-    ow += __builtin_amdgcn_exp2f(s_s[t] - mw) * cvt4(*reinterpret_cast<const uint2*>(wrow(a.nw.v, a.v_tail, t) + 4 * c4));
-  const float Lw = gen_block_sum(lw, s_red);
-  s_part[part][c4] = ow;
-  if (g == 0 && a.nw.n > 0) {   // rows given apart into the window buffer
-    for (int e = tid; e < a.nw.n * D; e += 128) {
-      const int t = a.nw.T - a.nw.n + e / D, c = e % D;
-      const int64_t src = nb + (int64_t)(e / D) * a.nw.st + c, dst = tb + (int64_t)t * a.ts_t + c;
-      a.nw.k_dst[dst] = a.nw.k[src];
-      a.nw.v_dst[dst] = a.nw.v[src];
-    }
+  l_run += __shfl_xor(l_run, 16);
+  l_run += __shfl_xor(l_run, 32);
+#pragma unroll
+  for (int hb = 1; hb < NT; hb <<= 1)
+#pragma unroll
+    for (int ct = 0; ct < NT; ++ct)
+      if (!(ct & hb)) {
+        const float4_t u = acc[ct], w = acc[ct | hb];
+        acc[ct] = u + w;
+        acc[ct | hb] = u - w;
+      }
+#pragma unroll
+  for (int ct = 0; ct < NT; ++ct) {
+#pragma unroll
+    for (int hb = 1; hb < 4; hb <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!(e & hb)) {
+          const float u = acc[ct][e], w = acc[ct][e | hb];
+          acc[ct][e] = u + w;
+          acc[ct][e | hb] = u - w;
+        }
+#pragma unroll
+    for (int rb = 1; rb < 4; rb <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float o = __shfl_xor(acc[ct][e], 16 * rb);
+        acc[ct][e] = (qd & rb) ? o - acc[ct][e] : acc[ct][e] + o;
+      }
   }
-  __syncthreads();
-  if (tid < D) {
-    float owc = 0.f;
-    for (int q = 0; q < P; ++q) owc += s_part[q][tid / 4][tid % 4];
-    const float M = fmaxf(Mp, mw);
-    const float wp = Mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(Mp - M);
-    const float ww = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
-    const float den = wp * Lp + ww * Lw;
-    gen_store_io(a.out, row * D + tid, den > 0.f ? (wp * op + ww * owc) / den : 0.f, a.io_dtype);
+  if (n >= G) return;
+  const float inv = l_run > 0.f ? 1.0f / ((float)D * l_run) : 0.f;
+  const int S = a.n_split * a.wph, slot = split * a.wph + sub;
+  const int64_t row = ((int64_t)b * L.h + h) * G + n;
+  float* rec = a.ws_acc + row * D * S + slot * 16;   // chunk k at + 16 k S
+#pragma unroll
+  for (int i = 0; i < D / 4; i += 4) {               // channels qd d/4 + i .. + 3
+    float4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = acc[(i + e) % NT][(i + e) / NT] * inv;
+    const int c = qd * (D / 4) + i;
+    const uint32_t sg = a.r.v_sign_bits[c >> 5] >> (c & 31);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (sg >> e) & 1u ? -o[e] : o[e];
+    *reinterpret_cast<float4_t*>(rec + (int64_t)(c >> 4) * 16 * S + (c & 15)) = o;
   }
+  if (qd == 0) *reinterpret_cast<float2*>(a.ws_ml + (row * S + slot) * 2) = make_float2(m_run, l_run);
 }
 
 // Dense keys and values of committed pages: grid (pages, h_kv), block 64.
@@ -502,7 +721,7 @@ __global__ __launch_bounds__(64) void gen_dequant_kernel(const GenDequantArgs a)
   const uint8_t* pg = gen_read_page(a.r, 0, p);
   float4_t kt[NT];
   gen_keys<D, R>(a.r, pg, s_B, 0, p, h, n, qd, kt);
-  if (a.apply_rope) gen_rope<D, false>(a.r, kt, a.pos0 + p * kPT + n, qd, a.apply_rope);
+  if (a.apply_rope) gen_rope<D>(a.r, kt, a.pos0 + p * kPT + n, qd, a.apply_rope);
   const int64_t krow = ((int64_t)h * a.out_rows + p * kPT + n) * D;
 #pragma unroll
   for (int rt = 0; rt < NT; ++rt)
@@ -564,34 +783,54 @@ void fill_read(GenReadArgs& r, const Geo& g) {
   r.L = GenLayout::of(g);
 }
 
-// splits per sequence and 16-token pages per split
-void gen_plan(const bmx_k2b_decode_args* a, const Geo& g, int* n_split, int* pps) {
-  const int pages = a->max_packed_len / kPT;
-  if (pages == 0) {
-    *n_split = 1;
-    *pps = 1;
-    return;
+// The decode grid of a sequence: n_split workgroups (its 4-page quads dealt
+// evenly) x head blocks of hpb heads, wph waves per head.  One workgroup per CU
+// over the batch; a wave per head, or several where there are fewer heads than
+// waves, each with its own partial slot.  A range with fewer quads than CUs
+// spreads its heads over more blocks (a wave alone on its SIMD takes a quad in
+// about half the time), and where CUs are still idle the window's tiles get
+// workgroups of their own (d 64, 2,048 tokens and a 128-row window: 17.1 us a call
+// with neither, 15.8 with the window apart, 12.6 with both).  The sequences are launched `chunk` at
+// a time, so that the workspace stays within kGenWorkspace whatever the batch.
+constexpr size_t kGenWorkspace = 24u << 20;   // one sequence takes at most 21.5 MB (16 heads x 16 queries, d 128)
+
+struct GenPlan {
+  int chunk, n_split, hpb, blocks, wph, win_tiles, win_wgs;
+  size_t bytes;
+  int slots() const { return n_split * wph; }
+};
+
+GenPlan gen_plan(const bmx_k2b_decode_args* a, const Geo& g) {
+  GenPlan p;
+  const int nw = gen_waves(g.d, g.R), cus = bmx_device_cu_count();
+  const int quads = std::max(1, (a->max_packed_len / kPT + kGenQuad - 1) / kGenQuad);
+  p.win_tiles = ((a->tail_len ? a->tail_cap : a->tail_len_value) + 15) / 16;
+  p.chunk = a->batch;
+  for (;; p.chunk = (p.chunk + 1) / 2) {
+    p.blocks = (g.h + nw - 1) / nw;
+    const int win_pairs = p.win_tiles * g.h;
+    while (a->split_tokens == 0 && 2 * p.blocks <= g.h &&
+           (int64_t)p.chunk * (2 * p.blocks * (int64_t)quads + (win_pairs + 3) / 4) <= cus)
+      p.blocks *= 2;
+    p.hpb = (g.h + p.blocks - 1) / p.blocks;
+    const int per_seq = cus / (p.chunk * p.blocks);
+    p.n_split = a->split_tokens > 0 ? (a->max_packed_len + a->split_tokens - 1) / a->split_tokens : per_seq;
+    p.n_split = std::max(1, std::min(p.n_split, quads));
+    p.wph = std::max(1, std::min(nw / p.hpb, (quads + p.n_split - 1) / p.n_split));
+    // as many as give every (tile, head) pair a wave, 4 pairs a workgroup if there is room, else none
+    const int spare = a->split_tokens > 0 ? 0 : per_seq - p.n_split;
+    p.win_wgs = std::min(spare, (win_pairs + 4 * p.blocks - 1) / (4 * p.blocks));
+    if (p.win_wgs * p.blocks * nw < win_pairs) p.win_wgs = 0;
+    p.bytes = (size_t)p.chunk * g.h * g.G * ((size_t)p.slots() * (g.d + 2) + a->tail_cap) * sizeof(float);
+    if (p.chunk == 1 || p.bytes <= kGenWorkspace) return p;
   }
-  int per = a->split_tokens > 0 ? a->split_tokens / kPT : 0;
-  if (per == 0) {
-    const int target = 2 * bmx_device_cu_count();
-    const int per_seq = std::max(1, (target + a->batch * g.h - 1) / (a->batch * g.h));
-    per = std::max(4, (pages + per_seq - 1) / per_seq);
-  }
-  *pps = per;
-  *n_split = (pages + per - 1) / per;
 }
 
 }  // namespace
 
 namespace bmx {
 
-size_t gen_decode_workspace(const bmx_k2b_decode_args* a) {
-  const Geo g = Geo::from(a->geom);
-  int n_split, pps;
-  gen_plan(a, g, &n_split, &pps);
-  return (size_t)a->batch * g.h * g.G * n_split * (g.d + 2) * sizeof(float);
-}
+size_t gen_decode_workspace(const bmx_k2b_decode_args* a) { return gen_plan(a, Geo::from(a->geom)).bytes; }
 
 std::string gen_decode_check(const bmx_k2b_decode_args* a) {
   const Geo g = Geo::from(a->geom);
@@ -602,55 +841,91 @@ std::string gen_decode_check(const bmx_k2b_decode_args* a) {
   return "";
 }
 
+template <int D, int R>
+static hipError_t gen_launch_split(const GenDecodeArgs& k, dim3 grid, hipStream_t st) {
+  auto go = [&](auto sw) {
+    constexpr int SW = decltype(sw)::value;
+    const hipError_t e = bmx_ensure_dynamic_lds((const void*)gen_split_kernel<D, R, SW>, gen_lds<D>());
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((gen_split_kernel<D, R, SW>), grid, dim3(64 * gen_waves(D, R)), gen_lds<D>(), st, k);
+    return hipGetLastError();
+  };
+  if (k.G <= 4) return go(std::integral_constant<int, 4>{});
+  if (k.G <= 8) return go(std::integral_constant<int, 8>{});
+  return go(std::integral_constant<int, 16>{});
+}
+
 int gen_decode(const bmx_k2b_decode_args* a, hipStream_t st, void* ws, size_t ws_cap, const std::string& name) {
   const Geo g = Geo::from(a->geom);
-  int n_split, pps;
-  gen_plan(a, g, &n_split, &pps);
-  const size_t need = gen_decode_workspace(a);
-  if (!ws || ws_cap < need)
+  const GenPlan p = gen_plan(a, g);
+  if (!ws || ws_cap < p.bytes)
     return gfail(BMX_E_WORKSPACE, name + ": workspace missing or smaller than bmx_k2b_decode_workspace_bytes()");
   GenDecodeArgs k{};
   fill_read(k.r, g);
-  k.r.pages = a->pages; k.r.page_table = a->page_table; k.r.max_pages = a->max_pages;
+  k.r.pages = a->pages; k.r.max_pages = a->max_pages;
   k.r.n_pool = a->n_pool_pages > 0 ? a->n_pool_pages : 1;
-  k.r.basis = a->basis; k.r.basis_stride = a->basis_stride;
+  k.r.basis_stride = a->basis_stride;
   for (int j = 0; j < 64; ++j) k.r.inv_freq[j] = a->inv_freq[j];
   k.r.rope_scaling = a->rope_scaling;
   for (int j = 0; j < 4; ++j) { k.r.level[j] = a->codebook[j]; k.r.v_sign_bits[j] = a->v_sign_bits[j]; }
-  k.G = g.G; k.n_split = n_split; k.pps = pps;
-  k.q = a->q; k.io_dtype = a->io_dtype;
-  k.packed_len = a->packed_len; k.max_packed_len = a->max_packed_len;
+  k.G = g.G; k.n_split = p.n_split; k.hpb = p.hpb; k.wph = p.wph;
+  k.win_tiles = p.win_tiles; k.win_wgs = p.win_wgs;
+  k.div32 = ((uint64_t)p.n_split + 1) * (a->max_packed_len / 64 + 1) < (1ull << 32);
+  k.inv_per_slot = 1.0f / (float)k.r.L.per_slot;
+  k.io_dtype = a->io_dtype;
+  k.max_packed_len = a->max_packed_len;
   k.qscale = a->sm_scale * 1.4426950408889634f;
-  const size_t rows = (size_t)a->batch * g.h * g.G * n_split;
+  const int hg = g.h * g.G;
+  const size_t recs = (size_t)p.chunk * hg * p.slots();
   k.ws_acc = (float*)ws;
-  k.ws_ml = k.ws_acc + rows * g.d;
-  k.out = a->out;
-  k.k_tail = a->k_tail; k.v_tail = a->v_tail;
+  k.ws_ml = k.ws_acc + recs * g.d;
+  k.ws_win = k.ws_ml + recs * 2;
   k.ts_b = a->tail_stride_b; k.ts_h = a->tail_stride_h; k.ts_t = a->tail_stride_t;
   k.tail_cap = a->tail_cap; k.tail_bf16 = a->tail_dtype == BMX_K2B_TAIL_BF16;
-  k.tail_len = a->tail_len;
-  k.nw.k = a->new_k; k.nw.v = a->new_v;
   k.nw.sb = a->new_stride_b; k.nw.sh = a->new_stride_h; k.nw.st = a->new_stride_t;
   k.nw.n = a->n_new;
   k.nw.T = a->tail_len ? -1 : a->tail_len_value;
-  k.nw.k_dst = const_cast<uint16_t*>(a->k_tail);
-  k.nw.v_dst = const_cast<uint16_t*>(a->v_tail);
-  const dim3 grid(n_split, g.h, a->batch);
-#define BMX_GEN_SPLIT(D_, R_) hipLaunchKernelGGL((gen_split_kernel<D_, R_>), grid, dim3(256), 0, st, k)
-  BMX_GEN_DISPATCH(g.d, g.R, BMX_GEN_SPLIT)
+  CombineKArgs c{};
+  c.h_kv = g.h; c.G = g.G; c.max_splits = p.slots(); c.tail_cap = a->tail_cap;
+  c.io_dtype = a->io_dtype;
+  c.ws_acc = k.ws_acc; c.ws_ml = k.ws_ml; c.ws_win = k.ws_win;
+  c.ts_b = k.ts_b; c.ts_h = k.ts_h; c.ts_t = k.ts_t; c.tail_bf16 = k.tail_bf16;
+  c.packed_scale = 1.0f;
+  c.max_packed_len = a->max_packed_len;
+  const int64_t io_bytes = a->io_dtype == BMX_K2B_IO_F32 ? 4 : 2;
+  for (int b0 = 0; b0 < a->batch; b0 += p.chunk) {
+    const int nb = std::min(p.chunk, a->batch - b0);
+    auto at = [&](const uint16_t* x, int64_t stride) { return x ? x + b0 * stride : nullptr; };
+    k.b0 = b0;
+    k.r.page_table = a->page_table ? a->page_table + (int64_t)b0 * a->max_pages : nullptr;
+    k.r.basis = at(a->basis, a->basis_stride);
+    k.q = (const char*)a->q + b0 * (int64_t)hg * g.d * io_bytes;
+    c.out = (char*)a->out + b0 * (int64_t)hg * g.d * io_bytes;
+    k.packed_len = c.packed_len = a->packed_len + b0;
+    k.k_tail = at(a->k_tail, a->tail_stride_b);
+    c.v_tail = at(a->v_tail, a->tail_stride_b);
+    c.tail_len = a->tail_len ? a->tail_len + b0 : nullptr;
+    k.nw.k = at(a->new_k, a->new_stride_b);
+    k.nw.v = at(a->new_v, a->new_stride_b);
+    k.nw.k_dst = const_cast<uint16_t*>(k.k_tail);
+    k.nw.v_dst = const_cast<uint16_t*>(c.v_tail);
+    c.nw = k.nw;
+    const dim3 grid(p.n_split + p.win_wgs, p.blocks, nb);
+    hipError_t e = hipSuccess;
+#define BMX_GEN_SPLIT(D_, R_) e = gen_launch_split<D_, R_>(k, grid, st)
+    BMX_GEN_DISPATCH(g.d, g.R, BMX_GEN_SPLIT)
 #undef BMX_GEN_SPLIT
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return gfail(BMX_E_HIP, name + ": split kernel launch: " + hipGetErrorString(e));
-  if (a->split_end_event) {
-    e = hipEventRecord((hipEvent_t)a->split_end_event, st);
-    if (e != hipSuccess) return gfail(BMX_E_HIP, name + ": hipEventRecord: " + hipGetErrorString(e));
+    if (e != hipSuccess) return gfail(BMX_E_HIP, name + ": split kernel launch: " + hipGetErrorString(e));
+    if (a->split_end_event) {
+      e = hipEventRecord((hipEvent_t)a->split_end_event, st);
+      if (e != hipSuccess) return gfail(BMX_E_HIP, name + ": hipEventRecord: " + hipGetErrorString(e));
+    }
+    if (g.d == 32) launch_combine<false, 32, float>(c, hg, nb, st);
+    else if (g.d == 64) launch_combine<false, 64, float>(c, hg, nb, st);
+    else launch_combine<false, 128, float>(c, hg, nb, st);
+    e = hipGetLastError();
+    if (e != hipSuccess) return gfail(BMX_E_HIP, name + ": merge kernel launch: " + hipGetErrorString(e));
   }
-  const dim3 mgrid(g.G, g.h, a->batch);
-  if (g.d == 32) hipLaunchKernelGGL(gen_merge_kernel<32>, mgrid, dim3(128), 0, st, k);
-  else if (g.d == 64) hipLaunchKernelGGL(gen_merge_kernel<64>, mgrid, dim3(128), 0, st, k);
-  else hipLaunchKernelGGL(gen_merge_kernel<128>, mgrid, dim3(128), 0, st, k);
-  e = hipGetLastError();
-  if (e != hipSuccess) return gfail(BMX_E_HIP, name + ": merge kernel launch: " + hipGetErrorString(e));
   return BMX_OK;
 }
 
