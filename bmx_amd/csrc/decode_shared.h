@@ -3,6 +3,8 @@
 // merge kernel that combines the split partials with the window.
 #pragma once
 
+#include <algorithm>
+
 #include "k2b_common.h"
 
 namespace bmx {
@@ -151,31 +153,33 @@ __device__ __forceinline__ void score_win_tile(const A& a, int b, int h, int j, 
 
 // Query and output elements of a decode call in its I/O dtype: 0 = fp32,
 // 1 = fp16, 2 = bf16 (BMX_K2B_IO_*; the model's own dtype, so a decode step
-// needs no conversion kernel).  Four consecutive elements from element idx.
+// needs no conversion kernel).
 constexpr int kIoF32 = 0, kIoF16 = 1, kIoBF16 = 2;
 
-__device__ __forceinline__ float4_t load_q4(const void* base, int64_t idx, int io) {
-  if (io == kIoF32) return *reinterpret_cast<const float4_t*>(reinterpret_cast<const float*>(base) + idx);
-  const uint2 r = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(base) + idx);
-  if (io == kIoF16) {
-    const half2_t lo = as_h2(r.x), hi = as_h2(r.y);
-    return float4_t{(float)lo[0], (float)lo[1], (float)hi[0], (float)hi[1]};
-  }
-  return float4_t{__builtin_bit_cast(float, r.x << 16), __builtin_bit_cast(float, r.x & 0xffff0000u),
-                  __builtin_bit_cast(float, r.y << 16), __builtin_bit_cast(float, r.y & 0xffff0000u)};
-}
-
-// Four query elements as they lie in memory, loaded without a branch on the
-// dtype: 8 bytes at element idx, and for fp32 the next 8 (16-bit dtypes: the
-// same 8 again).  load_q4 converts inside its branch, so a run of its calls
-// waits for each load before the next is issued; these are all in flight
-// together, and cvt_q4 converts them once they are needed.
+// Four query elements as they lie in memory: 8 bytes at the element, and for
+// fp32 the next 8.  A load and its conversion inside a branch on the dtype makes
+// a run of them wait for each load before the next is issued; load_q4 issues the
+// loads of N pieces (at element idx(i)) together, and cvt_q4 converts them once
+// they are needed.  Measured on a k2b call of 256 tokens (rank 16, fp16, the
+// window on workgroups of its own): 12.1 us; with the second 8 bytes loaded (and
+// unused) for 16-bit dtypes too 12.8: the prologue's loads are bound by their
+// number.  Masking the loads of lanes past the G query rows: 2 % slower.
 struct RawQ4 {
   uint2 a, b;
 };
-__device__ __forceinline__ RawQ4 load_raw_q4(const void* base, int64_t idx, int io) {
-  const char* p = static_cast<const char*>(base) + (idx << (io == kIoF32 ? 2 : 1));
-  return {*reinterpret_cast<const uint2*>(p), *reinterpret_cast<const uint2*>(p + (io == kIoF32 ? 8 : 0))};
+template <int N, class Idx>
+__device__ __forceinline__ void load_q4(const void* base, int io, Idx idx, RawQ4 (&r)[N]) {
+  const char* p = static_cast<const char*>(base);
+  const int sh = io == kIoF32 ? 2 : 1;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    r[i].a = *reinterpret_cast<const uint2*>(p + ((int64_t)idx(i) << sh));
+    r[i].b = make_uint2(0u, 0u);
+  }
+  if (io == kIoF32) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i].b = *reinterpret_cast<const uint2*>(p + ((int64_t)idx(i) << sh) + 8);
+  }
 }
 template <int N>
 __device__ __forceinline__ void cvt_q4(const RawQ4 (&r)[N], int io, float4_t (&out)[N]) {
@@ -257,6 +261,84 @@ __device__ __forceinline__ void window_fragments(const float4_t qraw[8], float s
         qh[bb][2 * i + e] = __builtin_bit_cast(_Float16, (uint16_t)hb);
         ql[bb][2 * i + e] = __builtin_bit_cast(_Float16, (uint16_t)bf16_bits(x - __uint_as_float(hb << 16)));
       }
+}
+
+// The recent window is scored in (16-token tile, head) pairs, pair
+// p = tile * h_kv + head on workgroup p mod n_wg, a workgroup's k-th pair on its
+// wave k mod nw.  Each pair is one memory round trip: the head's query rows and
+// the tile's rows together.
+template <class A>
+__device__ __forceinline__ void score_win_pairs(const A& a, float qscale, int b, int wg, int n_wg, int wave, int nw,
+                                                int n, int q) {
+  const int n_pairs = a.win_tiles * a.h_kv;
+  for (int p = wg + wave * n_wg; p < n_pairs; p += nw * n_wg) {
+    const int j = p / a.h_kv, hh = p - j * a.h_kv;
+    const int64_t qrow = (((int64_t)b * a.h_kv + hh) * a.G + (n < a.G ? n : 0)) * kD;
+    const int64_t tb = (int64_t)b * a.ts_b + (int64_t)hh * a.ts_h;
+    RawQ4 qr[8];
+    load_q4(a.q, a.io_dtype, [&](int u) { return qrow + 16 * (u & 3) + 4 * q + 64 * (u >> 2); }, qr);
+    uint2 kw[8];
+    load_win_tile(a, tb, j, n, q, kw, (int64_t)b * a.nw.sb + (int64_t)hh * a.nw.sh);
+    float4_t qraw[8];
+    cvt_q4(qr, a.io_dtype, qraw);
+    half8_t qh[4], ql[4];
+    window_fragments(qraw, n < a.G ? qscale : 0.0f, a.tail_bf16, qh, ql);
+    score_win_tile(a, b, hh, j, n, q, kw, qh, ql, tb);
+  }
+}
+
+// The window's pairs of a split kernel's workgroup, at its end: those of the
+// window's own workgroups (split >= S), or, where it has none, dealt over the
+// splits on waves 0-3 (of the two waves of a SIMD, w and w + 4, these end their
+// groups first).  One call for both, so that the kernel holds its code once.
+template <class A>
+__device__ __forceinline__ void score_window(const A& a, float qscale, int b, int split, int S, int wave, int waves,
+                                             int n, int q) {
+  const bool apart = a.win_wgs != 0;
+  if (apart ? split < S : wave >= 4) return;
+  score_win_pairs(a, qscale, b, apart ? split - S + a.win_wgs * (int)blockIdx.z : split,
+                  apart ? a.win_wgs * (int)gridDim.z : S, wave, apart ? waves : 4, n, q);
+}
+
+// The split grid of a call (k2b and RTN): S splits of a sequence, its heads in
+// `blocks` blocks of hpb (grid z), and win_wgs workgroups (grid x, after the
+// splits) that score the window and do nothing else.
+//   S: one workgroup per CU over the batch, or what split_tokens asks for; at
+//     most one per 64-token group.
+//   blocks: a range with few groups leaves CUs idle while the 8 waves of a
+//     workgroup, two per SIMD, share its issue slots; its heads are spread over
+//     2, 4 or 8 workgroups as long as all of them, and the window's, have a CU.
+//   win_wgs: as many as give every (tile, head) pair a wave, 4 pairs a workgroup
+//     where there is room; none where there is not enough: the splits then score
+//     the window after their groups, and, where they are fewer than its tiles,
+//     are as many as those (one per CU at most).
+// Measured, us a call at h_kv 8, G 4 (with neither, and with both): k2b rank 16,
+// 256 tokens and a 60-row window 17.4 -> 12.1 (the query loads together in both:
+// see load_q4); 8,576 tokens, bf16, a 161-row window (no room to spread) 17.7 ->
+// 15.5; RTN 128 tokens 16.9 -> 12.4.
+// Everything follows from the bounds (max_len, tail_cap), not from a call's own
+// window length, so a bound call's workspace fits it at any length.
+struct SplitPlan {
+  int S, blocks, hpb, win_wgs;
+};
+inline SplitPlan plan_splits(int batch, int h_kv, int groups, int max_len, int split_tokens, int tail_cap, int cus) {
+  SplitPlan p;
+  const int per_seq = std::max(1, cus / batch);
+  const int tiles = (tail_cap + 15) / 16, pairs = tiles * h_kv;
+  p.S = split_tokens > 0 ? (max_len + split_tokens - 1) / split_tokens : per_seq;
+  p.S = std::max(1, std::min(p.S, groups));
+  p.blocks = 1;
+  p.win_wgs = 0;
+  if (split_tokens == 0) {
+    while (2 * p.blocks <= h_kv && (int64_t)batch * (2 * p.blocks * (int64_t)p.S + (pairs + 3) / 4) <= cus)
+      p.blocks *= 2;
+    const int spare = per_seq / p.blocks - p.S;
+    p.win_wgs = std::max(0, std::min(spare, (pairs + 4 * p.blocks - 1) / (4 * p.blocks)));
+    if (p.win_wgs * p.blocks * 8 < pairs) p.win_wgs = 0;
+  }
+  if (p.win_wgs == 0 && p.S < tiles) p.S = std::min(tiles, std::max(p.S, per_seq));
+  p.hpb = (h_kv + p.blocks - 1) / p.blocks;
+  return p;
 }
 
 // ---------------------------------------------------------------------------

@@ -37,12 +37,14 @@
 //   * at the end, the accumulator is half un-rotated in registers: the
 //     128-point Hadamard factors as H8 (over the 16-channel chunks) x H16
 //     (within a chunk), and the split kernel applies H8;
-//   * the workgroups that own a 16-token tile of the fp16 recent window score
-//     it on MFMA (decode_shared.h) after their group loop, on waves 0-3: of
-//     the two waves of a SIMD (w, w + 4) the older wins issue arbitration and
-//     ends its groups ~2 us before the younger, so the tiles fill that slack
-//     instead of delaying the workgroup's first group; the two waves of a
-//     SIMD also take turns at the higher issue priority page by page.
+//   * the recent window is scored in (16-token tile, head) pairs on MFMA
+//     (decode_shared.h): by workgroups that do nothing else where CUs are idle,
+//     else by the splits after their groups, on waves 0-3: of the two waves of a
+//     SIMD (w, w + 4) the older wins issue arbitration and ends its groups ~2 us
+//     before the younger, so the tiles fill that slack; the two waves of a SIMD
+//     also take turns at the higher issue priority page by page;
+//   * a range of few groups spreads its heads over several workgroups (grid z),
+//     a wave with a head then alone on its SIMD or nearly so (plan_splits).
 //
 // combine_kernel<true> (decode_shared.h): one wave per (16-channel chunk,
 // query head, sequence) merges the packed partials of its chunk (base-2 LSE),
@@ -92,6 +94,9 @@ struct DecodeKArgs {
   uint32_t div_magic;
   int div_sh1, div_sh2, div_ok;
   int io_dtype;
+  int hpb;             // heads per workgroup (blockIdx.z: the head block)
+  int win_tiles;       // 16-token tiles of the window that are scored
+  int win_wgs;         // workgroups of a sequence for the window alone, after its max_splits (0: none)
   float qscale_rope;   // sm_scale * log2(e) * rope_scaling (the cos/sin table is unscaled)
   uint32_t level_hi[4];   // fp16 bits of the value levels as used by the MFMA:
                           // hi_c = kappa * codebook_c + mu (+ < 1e-6 relative)
@@ -171,30 +176,6 @@ __device__ __forceinline__ void store_partial(const DecodeKArgs& a, int b, int s
                          m_run, l_run);
 }
 
-// The recent window is scored in (16-token tile, head) pairs: pair
-// p = tile * h_kv + head goes to split p mod S, and a split's k-th pair to
-// its wave k mod nw (after the group loop: waves 0-3, which end their groups
-// first; in a split with no packed tokens: any wave).  Each pair is one
-// memory round trip (the head's query rows and the tile's rows together), so
-// a wave that owns one pair ends one round trip after its groups.
-__device__ __forceinline__ void score_win_pairs(const DecodeKArgs& a, int b, int split, int S, int wave, int nw,
-                                                int n, int q) {
-  const int n_pairs = ((a.tail_cap + 15) >> 4) * a.h_kv;
-  for (int p = split + wave * S; p < n_pairs; p += nw * S) {
-    const int j = p / a.h_kv, hh = p - j * a.h_kv;
-    const int64_t qrow = (((int64_t)b * a.h_kv + hh) * a.G + (n < a.G ? n : 0)) * kD;
-    const int64_t tb = (int64_t)b * a.ts_b + (int64_t)hh * a.ts_h;
-    float4_t qraw[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) qraw[u] = load_q4(a.q, qrow + 16 * (u & 3) + 4 * q + 64 * (u >> 2), a.io_dtype);
-    uint2 kw[8];
-    load_win_tile(a, tb, j, n, q, kw, (int64_t)b * a.nw.sb + (int64_t)hh * a.nw.sh);
-    half8_t qh[4], ql[4];
-    window_fragments(qraw, n < a.G ? a.qscale_rope : 0.0f, a.tail_bf16, qh, ql);
-    score_win_tile(a, b, hh, j, n, q, kw, qh, ql, tb);
-  }
-}
-
 // R: key rank (16 or 32).  SW: query slot width (G rounded up to 4, 8 or 16);
 // the 16 score columns of a page hold 16/SW pages after compaction.
 template <int R, int SW, bool CONTIG>
@@ -221,15 +202,17 @@ __global__ __launch_bounds__(kThreads) void k2b_decode_split_kernel(const Decode
   // prologue's branches
   asm volatile("" ::"s"(a.h_kv), "s"(a.G), "s"(a.max_splits), "s"(a.max_pages), "s"(a.max_packed_len),
                "s"(a.n_pool), "s"(a.shared_bytes), "s"(a.cs_bufs), "s"(a.balanced), "s"(a.n_seq),
-               "s"(a.div_magic), "s"(a.div_sh1), "s"(a.div_sh2), "s"(a.div_ok), "s"(a.io_dtype));
+               "s"(a.div_magic), "s"(a.div_sh1), "s"(a.div_sh2), "s"(a.div_ok), "s"(a.io_dtype), "s"(a.hpb),
+               "s"(a.win_wgs));
   asm volatile("" ::"s"(a.q), "s"(a.pages), "s"(a.page_table), "s"(a.packed_len), "s"(a.basis),
                "s"(a.basis_stride), "s"(a.L.bytes), "s"(a.L.kres), "s"(a.L.vcode));
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int n = lane & 15;   // token within page (K side) / score column (softmax side)
   const int q = lane >> 4;   // quarter
-  const bool active = wave < a.h_kv;
-  const int h = active ? wave : 0;
+  const int h_own = blockIdx.z * a.hpb + wave;   // heads of block z: hpb z .. + hpb - 1
+  const bool active = wave < a.hpb && h_own < a.h_kv;
+  const int h = active ? h_own : 0;
   // this workgroup's sequence b, split and the sequence's split count S: the
   // grid's (x, y), or, for a ragged batch, the workgroup's place in the
   // length-proportional shares of the flat grid (read from the lengths)
@@ -245,6 +228,9 @@ __global__ __launch_bounds__(kThreads) void k2b_decode_split_kernel(const Decode
     S = __shfl(share, b);
     len_known = __shfl(len_l, b);
   }
+
+  do {   // left at once by a workgroup for the window alone
+  if (split >= S) break;
 
   // ---- every load that depends only on the arguments is issued first, the
   // page-table read first of all, and nothing is used before the first group's
@@ -304,11 +290,10 @@ __global__ __launch_bounds__(kThreads) void k2b_decode_split_kernel(const Decode
 #pragma unroll
   for (int bt = 0; bt < 8; ++bt)
     vh[bt] = *reinterpret_cast<const hvec_t*>(basis + (int64_t)(h * kD + 16 * bt + n) * R + KQ * q);
-  float4_t qraw[8];   // q_n[16bb + 4q .. +3] (u = bb) and [.. + 64] (u = 4 + bb)
+  RawQ4 qr[8];   // q_n[16bb + 4q .. +3] (u = bb) and [.. + 64] (u = 4 + bb)
   {
     const int64_t qrow = (((int64_t)b * a.h_kv + h) * a.G + (n < a.G ? n : 0)) * kD;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) qraw[u] = load_q4(a.q, qrow + 16 * (u & 3) + 4 * q + 64 * (u >> 2), a.io_dtype);
+    load_q4(a.q, a.io_dtype, [&](int u) { return qrow + 16 * (u & 3) + 4 * q + 64 * (u >> 2); }, qr);
   }
   // dynamic LDS: the cos/sin tables, then the prefix ring
   const int cs_bufs = a.cs_bufs;
@@ -449,6 +434,8 @@ __global__ __launch_bounds__(kThreads) void k2b_decode_split_kernel(const Decode
   // query fragments (qf: the MFMA B operand of the packed pages; the low parts
   // are unused here: the window tiles remake both after the loop)
   half8_t qf[4], qlo[4];
+  float4_t qraw[8];
+  cvt_q4(qr, a.io_dtype, qraw);
   query_fragments(qraw, (n < a.G) ? a.qscale_rope : 0.0f, qf, qlo);
 
   store_prefix(pre, 0);
@@ -664,9 +651,6 @@ __global__ __launch_bounds__(kThreads) void k2b_decode_split_kernel(const Decode
       }
     }
   }
-  // the window pairs this workgroup owns, on waves 0-3: of the two waves of a
-  // SIMD (w, w + 4) these finish their groups first
-  if (wave < 4) score_win_pairs(a, b, split, S, wave, 4, n, q);
   if (active) {
     // fold the page slots: column s*SW + g -> g
     if constexpr (NSLOT == 4) {
@@ -687,6 +671,8 @@ __global__ __launch_bounds__(kThreads) void k2b_decode_split_kernel(const Decode
     }
     store_partial(a, b, split, h, n, q, acc, m_run, l_run, w_run);
   }
+  } while (false);
+  score_window(a, a.qscale_rope, b, split, S, wave, kWaves, n, q);
 }
 
 }  // namespace bmx
@@ -695,10 +681,6 @@ using namespace bmx;
 
 static int device_cu_count() { return bmx_device_cu_count(); }
 
-// Workgroups per sequence: one wave of workgroups over the device's CUs (one
-// 8-wave workgroup per CU), or as many as split_tokens asks for; never more
-// than the sequence has 64-token groups, except that the recent window's
-// 16-token score tiles get a workgroup each, up to one per CU.
 // A ragged batch (2..64 sequences, no split_tokens, two CUs or more per
 // sequence) runs balanced: one flat wave of workgroups over the CUs, each
 // sequence a share proportional to its length (batch_shares); the partial
@@ -708,20 +690,11 @@ static bool balanced_batch(const bmx_k2b_decode_args* a) {
          device_cu_count() >= 2 * a->batch;
 }
 
-// Partial slots per row (the split count of a sequence, at most).
-static int choose_splits(const bmx_k2b_decode_args* a) {
-  if (balanced_batch(a)) return device_cu_count() - a->batch + 1;
-  const int units = (a->max_packed_len + kGroup - 1) / kGroup;
-  const int per_seq = std::max(1, device_cu_count() / a->batch);
-  int S;
-  if (a->split_tokens > 0)
-    S = (a->max_packed_len + a->split_tokens - 1) / a->split_tokens;
-  else
-    S = per_seq;
-  if (S > units) S = units;
-  const int tiles = (a->tail_cap + 15) / 16;
-  if (S < tiles) S = std::min(tiles, std::max(S, per_seq));
-  return S < 1 ? 1 : S;
+// The grid of a call; S is also the partial slots per row.
+static SplitPlan split_plan(const bmx_k2b_decode_args* a) {
+  if (balanced_batch(a)) return {device_cu_count() - a->batch + 1, 1, a->geom.h_kv, 0};
+  return plan_splits(a->batch, a->geom.h_kv, (a->max_packed_len + kGroup - 1) / kGroup, a->max_packed_len,
+                     a->split_tokens, a->tail_cap, device_cu_count());
 }
 
 // Workspace: split partial records [B][h_kv][G][8][S][16] fp16, then (max,
@@ -734,7 +707,7 @@ static size_t ws_bytes(const bmx_k2b_decode_args* a, int splits) {
 extern "C" size_t bmx_k2b_decode_workspace_bytes(const bmx_k2b_decode_args* a) {
   if (!a || a->batch < 1) return 0;
   if (Geo::from(a->geom).general) return gen_decode_workspace(a);
-  return ws_bytes(a, choose_splits(a));
+  return ws_bytes(a, split_plan(a).S);
 }
 
 // ---------------------------------------------------------------------------
@@ -997,7 +970,8 @@ static int decode_launch(const bmx_k2b_decode_args* a, void* stream, void* ws, s
   const bmx_k2b_geom& g = a->geom;
   if (const int rc = check_decode_args(a, name)) return rc;
   if (Geo::from(g).general) return gen_decode(a, (hipStream_t)stream, ws, ws_cap, name);
-  const int max_splits = choose_splits(a);
+  const SplitPlan plan = split_plan(a);
+  const int max_splits = plan.S;
   const size_t need = ws_bytes(a, max_splits);
   if (max_splits > 8192)
     return fail(BMX_E_INVALID, name + ": more than 8192 splits; use a larger split_tokens");
@@ -1013,6 +987,8 @@ static int decode_launch(const bmx_k2b_decode_args* a, void* stream, void* ws, s
 
   DecodeKArgs k{};
   k.h_kv = g.h_kv; k.G = g.n_q_groups;
+  k.hpb = plan.hpb; k.win_tiles = ((a->tail_len ? a->tail_cap : a->tail_len_value) + 15) / 16;
+  k.win_wgs = plan.win_wgs;
   k.max_splits = max_splits; k.max_pages = a->max_pages;
   k.max_packed_len = a->max_packed_len; k.n_pool = a->n_pool_pages > 0 ? a->n_pool_pages : 1;
   k.L = PageLayout::make(g.h_kv, g.rank);
@@ -1071,7 +1047,7 @@ static int decode_launch(const bmx_k2b_decode_args* a, void* stream, void* ws, s
     k.div_ok = (uint64_t)d * (groups + 1) < (1ull << 32) ? 1 : 0;
   }
   const size_t smem = (size_t)k.cs_bufs * kCsBuf * 4 + (size_t)kRingSlots * kGroupPages * k.shared_bytes;
-  const dim3 grid = balanced ? dim3(n_wg, 1) : dim3(max_splits, a->batch);
+  const dim3 grid = balanced ? dim3(n_wg, 1) : dim3(max_splits + plan.win_wgs, a->batch, plan.blocks);
   hipError_t e = g.rank == 32 ? launch_split<32>(k, grid, smem, st)
                               : launch_split<16>(k, grid, smem, st);
   if (e != hipSuccess)

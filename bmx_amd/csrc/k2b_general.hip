@@ -222,13 +222,10 @@ __device__ __forceinline__ void gen_window_tile(const GenDecodeArgs& a, int b, i
   const bool bf = __builtin_amdgcn_readfirstlane(a.tail_bf16) != 0;
   const int64_t r0 = ((int64_t)b * H + h) * a.G;
   constexpr int GB = D == 128 ? 2 : 4;   // queries whose loads are in flight with the tile's
-  RawQ4 qr[GB][NQ];
+  RawQ4 qr[GB * NQ];
   auto load_q = [&](int g0) {
-#pragma unroll
-    for (int i = 0; i < GB; ++i)
-#pragma unroll
-      for (int c = 0; c < NQ; ++c)
-        qr[i][c] = load_raw_q4(a.q, (r0 + min(g0 + i, a.G - 1)) * D + qd * (D / 4) + 4 * c, a.io_dtype);
+    load_q4(a.q, a.io_dtype,
+            [&](int k) { return (r0 + min(g0 + k / NQ, a.G - 1)) * D + qd * (D / 4) + 4 * (k % NQ); }, qr);
   };
   load_q(0);
   if (i_new >= 0) {
@@ -238,11 +235,11 @@ __device__ __forceinline__ void gen_window_tile(const GenDecodeArgs& a, int b, i
   }
   for (int g0 = 0; g0 < a.G; g0 += GB) {
     if (g0 > 0) load_q(g0);
+    float4_t qv[GB * NQ];
+    cvt_q4(qr, a.io_dtype, qv);
 #pragma unroll
     for (int i = 0; i < GB; ++i) {
       float s = 0.f;
-      float4_t qv[NQ];
-      cvt_q4(qr[i], a.io_dtype, qv);
 #pragma unroll
       for (int c = 0; c < NQ; ++c) {
         const uint2 r = kv[c];
@@ -251,7 +248,7 @@ __device__ __forceinline__ void gen_window_tile(const GenDecodeArgs& a, int b, i
                               : float4_t{half_bits_to_float(r.x & 0xffff), half_bits_to_float(r.x >> 16),
                                          half_bits_to_float(r.y & 0xffff), half_bits_to_float(r.y >> 16)};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s = __builtin_fmaf(qv[c][e] * a.qscale, x[e], s);
+        for (int e = 0; e < 4; ++e) s = __builtin_fmaf(qv[i * NQ + c][e] * a.qscale, x[e], s);
       }
       s += __shfl_xor(s, 16);
       s += __shfl_xor(s, 32);
@@ -328,9 +325,7 @@ __global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const G
           for (int i = 0; i < KQ; ++i) bw[rt][ks][i] = __builtin_bit_cast(_Float16, row(rt)[4 * KQ * ks + i]);
     }
     const int64_t qrow = (((int64_t)b * L.h + h) * G + (n < G ? n : 0)) * D;
-#pragma unroll
-    for (int rt = 0; rt < NT; ++rt)
-      qx[rt] = load_raw_q4(a.q, qrow + RUN * qd + 4 * (rt % NP) + (rt / NP) * (D / 2), a.io_dtype);
+    load_q4(a.q, a.io_dtype, [&](int rt) { return qrow + RUN * qd + 4 * (rt % NP) + (rt / NP) * (D / 2); }, qx);
   }
   // the workgroup's quads, first of the host's bound of the length (so that the
   // first pages are requested without a wait for the device length)
@@ -795,7 +790,7 @@ void fill_read(GenReadArgs& r, const Geo& g) {
 constexpr size_t kGenWorkspace = 24u << 20;   // one sequence takes at most 21.5 MB (16 heads x 16 queries, d 128)
 
 struct GenPlan {
-  int chunk, n_split, hpb, blocks, wph, win_tiles, win_wgs;
+  int chunk, n_split, hpb, blocks, wph, win_wgs;
   size_t bytes;
   int slots() const { return n_split * wph; }
 };
@@ -804,11 +799,10 @@ GenPlan gen_plan(const bmx_k2b_decode_args* a, const Geo& g) {
   GenPlan p;
   const int nw = gen_waves(g.d, g.R), cus = bmx_device_cu_count();
   const int quads = std::max(1, (a->max_packed_len / kPT + kGenQuad - 1) / kGenQuad);
-  p.win_tiles = ((a->tail_len ? a->tail_cap : a->tail_len_value) + 15) / 16;
+  const int win_pairs = (a->tail_cap + 15) / 16 * g.h;   // the bound: a bound call's plan holds at any length
   p.chunk = a->batch;
   for (;; p.chunk = (p.chunk + 1) / 2) {
     p.blocks = (g.h + nw - 1) / nw;
-    const int win_pairs = p.win_tiles * g.h;
     while (a->split_tokens == 0 && 2 * p.blocks <= g.h &&
            (int64_t)p.chunk * (2 * p.blocks * (int64_t)quads + (win_pairs + 3) / 4) <= cus)
       p.blocks *= 2;
@@ -869,7 +863,8 @@ int gen_decode(const bmx_k2b_decode_args* a, hipStream_t st, void* ws, size_t ws
   k.r.rope_scaling = a->rope_scaling;
   for (int j = 0; j < 4; ++j) { k.r.level[j] = a->codebook[j]; k.r.v_sign_bits[j] = a->v_sign_bits[j]; }
   k.G = g.G; k.n_split = p.n_split; k.hpb = p.hpb; k.wph = p.wph;
-  k.win_tiles = p.win_tiles; k.win_wgs = p.win_wgs;
+  k.win_tiles = ((a->tail_len ? a->tail_cap : a->tail_len_value) + 15) / 16;
+  k.win_wgs = p.win_wgs;
   k.div32 = ((uint64_t)p.n_split + 1) * (a->max_packed_len / 64 + 1) < (1ull << 32);
   k.inv_per_slot = 1.0f / (float)k.r.L.per_slot;
   k.io_dtype = a->io_dtype;

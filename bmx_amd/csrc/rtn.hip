@@ -246,6 +246,7 @@ __global__ __launch_bounds__(256) void rtn_dequant_kernel(const RtnDequantKArgs 
 struct RtnDecodeKArgs {
   int h_kv, G, max_splits, max_pages, max_packed_len, n_pool;
   int gk, gv;
+  int hpb, win_tiles, win_wgs;   // plan_splits (decode_shared.h)
   int prefix_bytes;    // scale bytes of one page (KSCALE + VSCALE), multiple of 16
   const void* q;       // [B][h_kv][G][128] in io_dtype
   int io_dtype;
@@ -319,35 +320,6 @@ __device__ __forceinline__ void rtn_store_partial(const RtnDecodeKArgs& a, int b
                          m_run, l_run);
 }
 
-// the lane's query in the RoPE pair order of the window tiles (decode_shared.h)
-__device__ __forceinline__ void rtn_window_fragments(const RtnDecodeKArgs& a, int b, int h, int n, int q,
-                                                     half8_t qh[4], half8_t ql[4]) {
-  const int64_t qrow = (((int64_t)b * a.h_kv + h) * a.G + (n < a.G ? n : 0)) * kD;
-  float4_t qraw[8];
-#pragma unroll
-  for (int u = 0; u < 8; ++u) qraw[u] = load_q4(a.q, qrow + 16 * (u & 3) + 4 * q + 64 * (u >> 2), a.io_dtype);
-  window_fragments(qraw, n < a.G ? a.qscale : 0.0f, a.tail_bf16, qh, ql);
-}
-
-// A workgroup with no packed tokens: its window tiles and an empty partial.
-__device__ __noinline__ void rtn_empty_range(const RtnDecodeKArgs& a, int b, int split, int h, int n, int q) {
-  const int n_tiles = (a.tail_cap + 15) >> 4;
-  if (split < n_tiles) {
-    half8_t qh[4], ql[4];
-    rtn_window_fragments(a, b, h, n, q, qh, ql);
-    const int64_t tail_base = (int64_t)b * a.ts_b + (int64_t)h * a.ts_h;
-    for (int j = split; j < n_tiles; j += a.max_splits) {
-      uint2 kw[8];
-      load_win_tile(a, tail_base, j, n, q, kw, (int64_t)b * a.nw.sb + (int64_t)h * a.nw.sh);
-      score_win_tile(a, b, h, j, n, q, kw, qh, ql, tail_base);
-    }
-  }
-  float4_t zero[8];
-#pragma unroll
-  for (int bt = 0; bt < 8; ++bt) zero[bt] = float4_t{0.f, 0.f, 0.f, 0.f};
-  rtn_store_partial(a, b, split, h, n, q, zero, -INFINITY, 0.f);
-}
-
 // SW: query slot width (G rounded up to 4, 8 or 16); the 16 score columns of a
 // page hold 16 / SW pages after compaction.  NGK: key scale groups per token
 // (128 / k_group) of token-arm keys, 0 for channel-arm keys.
@@ -365,9 +337,12 @@ __global__ __launch_bounds__(kRThreads) void rtn_decode_split_kernel(const RtnDe
   const int wave = tid >> 6, lane = tid & 63;
   const int n = lane & 15, q = lane >> 4;
   const int split = blockIdx.x, b = blockIdx.y;
-  const bool active = wave < a.h_kv;
-  const int h = active ? wave : 0;
+  const int h_own = blockIdx.z * a.hpb + wave;   // heads of block z: hpb z .. + hpb - 1
+  const bool active = wave < a.hpb && h_own < a.h_kv;
+  const int h = active ? h_own : 0;
   const int S = a.max_splits;
+  do {   // left at once by a workgroup for the window alone
+  if (split >= S) break;
   const int len_spec = a.max_packed_len & ~(kRGroup - 1);
   auto range = [&](int L, int& r0, int& r1) {
     const int NG = L / kRGroup;
@@ -385,14 +360,11 @@ __global__ __launch_bounds__(kRThreads) void rtn_decode_split_kernel(const RtnDe
   const int pid_raw = load_ids_raw(0, (g1 - g0) * kRGroupPages);
   const int len_raw = a.packed_len[b];
   // the lane's query: channels 32bb + 8q + j (bb < 4, j < 8) of query n
-  float4_t qraw[8];
+  RawQ4 qr[8];
   {
     const int64_t qrow = (((int64_t)b * a.h_kv + h) * a.G + (n < a.G ? n : 0)) * kD;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) qraw[u] = load_q4(a.q, qrow + 32 * (u >> 1) + 8 * q + 4 * (u & 1), a.io_dtype);
+    load_q4(a.q, a.io_dtype, [&](int u) { return qrow + 32 * (u >> 1) + 8 * q + 4 * (u & 1); }, qr);
   }
-  const int n_win_tiles = (a.tail_cap + 15) >> 4;
-  const int64_t tail_base = (int64_t)b * a.ts_b + (int64_t)h * a.ts_h;
 
   int pidv = (int)clamp_page(pid_raw, a.n_pool);
   // uniform values in scalar registers: the group loop's bookkeeping is scalar work
@@ -404,10 +376,12 @@ __global__ __launch_bounds__(kRThreads) void rtn_decode_split_kernel(const RtnDe
   g0 = __builtin_amdgcn_readfirstlane(g0);
   g1 = __builtin_amdgcn_readfirstlane(g1);
   const int n_groups = g1 - g0;
-  if (n_groups == 0) {
-    if (active)
-      rtn_empty_range(*(const RtnDecodeKArgs*)__builtin_amdgcn_kernarg_segment_ptr(), b, split, h, n, q);
-    return;
+  if (n_groups == 0) {   // no packed tokens: an empty partial
+    float4_t zero[8];
+#pragma unroll
+    for (int bt = 0; bt < 8; ++bt) zero[bt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (active) rtn_store_partial(a, b, split, h, n, q, zero, -INFINITY, 0.f);
+    break;
   }
   auto load_ids = [&](int first, int count) { return (int)clamp_page(load_ids_raw(first, count), a.n_pool); };
   const int pb = a.L.bytes;
@@ -487,6 +461,8 @@ __global__ __launch_bounds__(kRThreads) void rtn_decode_split_kernel(const RtnDe
   half8_t qh[4], ql[4];
   {
     const float sc = n < a.G ? a.qscale : 0.0f;
+    float4_t qraw[8];
+    cvt_q4(qr, a.io_dtype, qraw);
 #pragma unroll
     for (int bb = 0; bb < 4; ++bb)
 #pragma unroll
@@ -497,16 +473,6 @@ __global__ __launch_bounds__(kRThreads) void rtn_decode_split_kernel(const RtnDe
         qh[bb][jp] = xh;
         ql[bb][jp] = (_Float16)(x - (float)xh);
       }
-  }
-  // the window tiles of this workgroup (their rows after the first group's pages)
-  if (active && split < n_win_tiles) {
-    half8_t wh[4], wl[4];
-    rtn_window_fragments(a, b, h, n, q, wh, wl);
-    for (int j = split; j < n_win_tiles; j += S) {
-      uint2 kw[8];
-      load_win_tile(a, tail_base, j, n, q, kw, (int64_t)b * a.nw.sb + (int64_t)h * a.nw.sh);
-      score_win_tile(a, b, h, j, n, q, kw, wh, wl, tail_base);
-    }
   }
   store_prefix(pre, 0);
   store_prefix(pre1, 1);
@@ -739,6 +705,8 @@ __global__ __launch_bounds__(kRThreads) void rtn_decode_split_kernel(const RtnDe
     }
     rtn_store_partial(a, b, split, h, n, q, acc, m_run, l_run);
   }
+  } while (false);
+  score_window(a, a.qscale, b, split, S, wave, kRWaves, n, q);
 }
 
 }  // namespace bmx
@@ -826,19 +794,9 @@ extern "C" int bmx_rtn_dequant(const bmx_rtn_dequant_args* a, void* stream) {
   return BMX_OK;
 }
 
-static int rtn_cu_count() { return bmx_device_cu_count(); }
-
-// as for k2b: one workgroup per CU over the batch (or split_tokens), never more
-// than the 64-token groups, and at least one per 16-token window tile (up to
-// one per CU)
-static int rtn_choose_splits(const bmx_rtn_decode_args* a) {
-  const int units = (a->max_packed_len + kRGroup - 1) / kRGroup;
-  const int per_seq = std::max(1, rtn_cu_count() / a->batch);
-  int S = a->split_tokens > 0 ? (a->max_packed_len + a->split_tokens - 1) / a->split_tokens : per_seq;
-  if (S > units) S = units;
-  const int tiles = (a->tail_cap + 15) / 16;
-  if (S < tiles) S = std::min(tiles, std::max(S, per_seq));
-  return S < 1 ? 1 : S;
+static SplitPlan rtn_split_plan(const bmx_rtn_decode_args* a) {
+  return plan_splits(a->batch, a->geom.h_kv, (a->max_packed_len + kRGroup - 1) / kRGroup, a->max_packed_len,
+                     a->split_tokens, a->tail_cap, bmx_device_cu_count());
 }
 
 static size_t rtn_ws_bytes(const bmx_rtn_decode_args* a, int splits) {
@@ -848,7 +806,7 @@ static size_t rtn_ws_bytes(const bmx_rtn_decode_args* a, int splits) {
 
 extern "C" size_t bmx_rtn_decode_workspace_bytes(const bmx_rtn_decode_args* a) {
   if (!a || a->batch < 1) return 0;
-  return rtn_ws_bytes(a, rtn_choose_splits(a));
+  return rtn_ws_bytes(a, rtn_split_plan(a).S);
 }
 
 template <int SW, bool kNT>
@@ -914,7 +872,8 @@ extern "C" int bmx_rtn_decode(const bmx_rtn_decode_args* a, void* stream) {
     return rfail(BMX_E_INVALID, "bmx_rtn_decode: k_tail/v_tail must be non-NULL when tail_cap > 0");
   if (a->tail_cap > 0 && (a->tail_stride_t % 8 != 0 || a->tail_stride_h % 8 != 0 || a->tail_stride_b % 8 != 0))
     return rfail(BMX_E_INVALID, "bmx_rtn_decode: tail strides must be multiples of 8 elements");
-  const int S = rtn_choose_splits(a);
+  const SplitPlan plan = rtn_split_plan(a);
+  const int S = plan.S;
   if (S > 8192) return rfail(BMX_E_INVALID, "bmx_rtn_decode: more than 8192 splits; use a larger split_tokens");
   const size_t need = rtn_ws_bytes(a, S);
   if (!a->workspace || a->workspace_bytes < need)
@@ -927,6 +886,8 @@ extern "C" int bmx_rtn_decode(const bmx_rtn_decode_args* a, void* stream) {
   hipStream_t st = (hipStream_t)stream;
 
   RtnDecodeKArgs k{};
+  k.hpb = plan.hpb; k.win_wgs = plan.win_wgs;
+  k.win_tiles = ((a->tail_len ? a->tail_cap : a->tail_len_value) + 15) / 16;
   k.h_kv = g.h_kv; k.G = g.n_q_groups; k.max_splits = S; k.max_pages = a->max_pages;
   k.max_packed_len = a->max_packed_len; k.n_pool = a->n_pool_pages > 0 ? a->n_pool_pages : 1;
   k.gk = g.k_group; k.gv = g.v_group;
@@ -944,7 +905,7 @@ extern "C" int bmx_rtn_decode(const bmx_rtn_decode_args* a, void* stream) {
   k.nw.T = a->tail_len ? -1 : a->tail_len_value;
   k.nw.k_dst = const_cast<uint16_t*>(a->k_tail);
   k.nw.v_dst = const_cast<uint16_t*>(a->v_tail);
-  dim3 grid(S, a->batch);
+  const dim3 grid(S + plan.win_wgs, a->batch, plan.blocks);
   const int ngk = g.k_arm == BMX_RTN_CHANNEL ? 0 : kD / g.k_group;
   const bool nt = (int64_t)a->batch * (a->max_packed_len / kPT) * k.L.bytes >= kRNtBytes;
   if (g.n_q_groups <= 4)
