@@ -14,7 +14,6 @@
 
 namespace bmx {
 
-constexpr int kSpCh = 64;                          // key channels staged per pass
 constexpr int kSpMaxSlices = BMX_SPECTRAL_MAX_CPAD / 8;
 
 __device__ __forceinline__ int sp_width(int b) { return b == 2 ? 2 : (b <= 4 ? 4 : 8); }
@@ -81,6 +80,7 @@ __device__ __forceinline__ float sp_load(const void* base, int64_t i, int dtype)
 }
 
 struct SpEncodeKArgs {
+  int n_blocks;      // encode workgroups (column blocks x groups); the rest of the grid encodes full-C values
   int C, c_pad, n_pool, k_dtype, page_bytes;
   const void* k;
   int64_t ksh, kst;
@@ -90,152 +90,6 @@ struct SpEncodeKArgs {
   const int32_t* page_ids;
   const float* lq;   // the Lloyd levels, or nullptr (rtn payload)
 };
-
-// grid (ceil(c_pad / 64), n_groups), block 512: wave w of block x
-// accumulates Y[t][j] for tokens 8w .. 8w + 7 of group y and page column
-// 64x + j (lane j) over the C channels, staged 64 at a time through LDS with
-// the chunk's enc rows (every product and sum rounded on its own, channels in
-// order); then wave 0's lane j takes column 64x + j's 64 values from LDS for
-// the step (max|Y| / qmax and 10 rounds of <Y, Q> / <Q, Q>; for the Lloyd
-// payload the sample deviation and 3 rounds of <Y, l> / <l, l>) and its
-// codes, and the block's 8 slices are assembled in LDS and written with dword
-// stores.
-template <bool kLloyd>
-__global__ __launch_bounds__(512) void spectral_encode_kernel(const SpEncodeKArgs a) {
-  __shared__ __align__(16) float s_m[kGroup][kSpCh + 4];   // the chunk's keys: [token][channel] (row pad 4: measured faster than 1)
-  __shared__ float s_e[kSpCh][64];           // the chunk's enc rows: [channel][column]
-  __shared__ float s_y[kGroup][65];          // Y: [token][column]
-  __shared__ uint32_t s_code[8 * kGroup * 8 / 4];   // 8 slices of at most 512 bytes
-  __shared__ float s_lv[kLloyd ? kLqLevels : 1], s_mid[kLloyd ? kLqLevels : 1];   // levels, midpoints
-  __shared__ float s_l[kLloyd ? kGroup : 1][65];      // Lloyd: the level of each (token, column)
-  __shared__ uint8_t s_cd[kLloyd ? kGroup : 1][64];   // Lloyd: the final level indices
-  __shared__ float s_sc[64];                          // Lloyd: each column's current step
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int j = blockIdx.x * 64 + lane, g = blockIdx.y;
-  const bool active = j < a.c_pad;
-  constexpr bool lloyd = kLloyd;
-  if (lloyd)
-    for (int i = tid; i < kLqLevels; i += 512) s_lv[i] = a.lq[i];
-  float y[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) y[t] = 0.f;
-  // the next chunk's keys and enc rows are loaded into registers while the
-  // current one is summed
-  float mreg[8], ereg[8];
-  auto load_chunk = [&](int c0) {
-    const int c = c0 + lane, h = c >> 7, d = c & (kD - 1);
-#pragma unroll
-    for (int t = 0; t < 8; ++t)
-      mreg[t] = sp_load(a.k, h * a.ksh + (int64_t)(g * kGroup + 8 * wave + t) * a.kst + d, a.k_dtype);
-#pragma unroll
-    for (int r = 0; r < 8; ++r)
-      ereg[r] = active ? a.encp[(int64_t)(c0 + 8 * wave + r) * a.c_pad + j] : 0.f;
-  };
-  load_chunk(0);
-  for (int c0 = 0; c0 < a.C; c0 += kSpCh) {
-    __syncthreads();   // the previous chunk read
-#pragma unroll
-    for (int t = 0; t < 8; ++t) s_m[8 * wave + t][lane] = mreg[t];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) s_e[8 * wave + r][lane] = ereg[r];
-    __syncthreads();
-    if (c0 + kSpCh < a.C) load_chunk(c0 + kSpCh);
-    // channels in order (16-byte reads of 4 channels measured slower)
-#pragma unroll 4
-    for (int cc = 0; cc < kSpCh; ++cc) {
-      const float e = s_e[cc][lane];
-#pragma unroll
-      for (int t = 0; t < 8; ++t) y[t] = __fadd_rn(y[t], __fmul_rn(s_m[8 * wave + t][cc], e));
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < 8; ++t) s_y[8 * wave + t][lane] = y[t];
-  // midpoints (l_i + l_{i+1}) / 2 within each tier (the slot after a tier's
-  // last level is never read); s_lv was written before the chunk loop's barriers
-  if (lloyd)
-    for (int i = tid; i + 1 < kLqLevels; i += 512) s_mid[i] = (s_lv[i] + s_lv[i + 1]) * 0.5f;
-  __syncthreads();
-  const int s = j >> 3, k = j & 7;
-  const uint32_t tab = active ? (uint32_t)a.slice_tab[s] : 0u;
-  const int b = active ? (int)(tab >> 24) : 2, w = sp_width(b);
-  const float qmax = (float)((1 << (b - 1)) - 1);
-  const float* lv = s_lv + (kLloyd ? lq_off(b) : 0);
-  const float* mid = s_mid + (kLloyd ? lq_off(b) : 0);
-  float scale = 1e-12f;
-  if constexpr (kLloyd) {
-    // the starting step in wave 0 (lane = column), then 4 rounds: every wave
-    // finds the level indices of 8 tokens (binary searches in parallel), and
-    // for the 3 refits wave 0 sums <Y, l> and <l, l> left to right
-    if (wave == 0) {
-      double sum = 0.0;
-      for (int t = 0; t < kGroup; ++t) sum += (double)s_y[t][lane];
-      const double mean = sum / 64.0;
-      double ss = 0.0;
-      for (int t = 0; t < kGroup; ++t) {
-        const double d = (double)s_y[t][lane] - mean;
-        ss += d * d;
-      }
-      s_sc[lane] = fmaxf((float)__dsqrt_rn(ss / 63.0), 1e-12f);
-    }
-    for (int r = 0; r <= 3; ++r) {
-      __syncthreads();   // the step written; the previous round's levels read
-      const float sc = s_sc[lane];
-      for (int t = wave; t < kGroup; t += 8) {
-        const int c = lq_index(mid, b, s_y[t][lane] / sc);
-        if (r < 3) s_l[t][lane] = lv[c];
-        else s_cd[t][lane] = (uint8_t)c;
-      }
-      if (r == 3) break;
-      __syncthreads();
-      if (wave == 0) {
-        float num = 0.f, den = 0.f;
-        for (int t = 0; t < kGroup; ++t) {
-          const float yv = s_y[t][lane], l = s_l[t][lane];
-          num = __fadd_rn(num, __fmul_rn(yv, l));
-          den = __fadd_rn(den, __fmul_rn(l, l));
-        }
-        s_sc[lane] = fmaxf(num / fmaxf(den, 1e-12f), 1e-12f);
-      }
-    }
-    scale = s_sc[lane];
-  } else if (active && wave == 0) {
-    float amax = 0.f;
-    for (int t = 0; t < kGroup; ++t) amax = fmaxf(amax, fabsf(s_y[t][lane]));
-    scale = fmaxf(amax, 1e-12f) / qmax;
-    for (int it = 0; it < 10; ++it) {
-      float num = 0.f, den = 0.f;
-      for (int t = 0; t < kGroup; ++t) {
-        const float yv = s_y[t][lane];
-        const float qv = fminf(fmaxf(rintf(yv / scale), -qmax - 1.f), qmax);
-        num = __fadd_rn(num, __fmul_rn(yv, qv));
-        den = __fadd_rn(den, __fmul_rn(qv, qv));
-      }
-      scale = fmaxf(num / fmaxf(den, 1e-12f), 1e-12f);
-    }
-  }
-  // the block's slices are contiguous in the page: [base, end)
-  const int n_sl = a.c_pad >> 3, s_first = blockIdx.x * 8, s_last = min(s_first + 8, n_sl) - 1;
-  const uint32_t tab0 = (uint32_t)a.slice_tab[s_first], tabl = (uint32_t)a.slice_tab[s_last];
-  const int base = (int)(tab0 & 0xFFFFFFu);
-  const int n_words = ((int)(tabl & 0xFFFFFFu) + kGroup * sp_width((int)(tabl >> 24)) - base) >> 2;
-  for (int i = tid; i < n_words; i += 512) s_code[i] = 0u;
-  __syncthreads();
-  if (active && wave == 0) {
-    const int bit0 = ((int)(tab & 0xFFFFFFu) - base) * 8 + k * w;
-    const uint32_t bias = 1u << (b - 1);
-    for (int t = 0; t < kGroup; ++t) {
-      const float qv = fminf(fmaxf(rintf(s_y[t][lane] / scale), -qmax - 1.f), qmax);
-      const uint32_t stored = lloyd ? (uint32_t)s_cd[kLloyd ? t : 0][lane] : (uint32_t)((int)qv + (int)bias);
-      const int bit = bit0 + t * w * 8;
-      atomicOr(&s_code[bit >> 5], stored << (bit & 31));
-    }
-  }
-  __syncthreads();
-  uint8_t* page = a.pages + clamp_page(a.page_ids[g], a.n_pool) * (int64_t)a.page_bytes;
-  uint32_t* dst = reinterpret_cast<uint32_t*>(page + base);
-  for (int i = tid; i < n_words; i += 512) dst[i] = s_code[i];
-  if (active && wave == 0) reinterpret_cast<uint16_t*>(page)[j] = float_to_half_bits(scale);
-}
 
 struct SpVFullKArgs {
   int h_kv, n_pool, v_dtype;
@@ -250,8 +104,8 @@ struct SpVFullKArgs {
 
 constexpr int kSpMaxC = 1024;
 
-// The full-C value codec (codecs.py:616-636 at h = 1): grid (16-token pages x
-// 4), block 256, one quarter q of a page (tokens 4q .. 4q + 3: the tokens of
+// The full-C value codec (codecs.py:616-636 at h = 1): 256 threads, block
+// 4 page + q: one quarter q of a page (tokens 4q .. 4q + 3: the tokens of
 // one VCODE dword) per workgroup.  Per token the fp16 norm of all C channels
 // (squares in 8 strided fp32 FMA accumulators, then those left to right:
 // torch's CPU order), the unit row times the C signs, a C-point FWHT in LDS
@@ -259,13 +113,19 @@ constexpr int kSpMaxC = 1024;
 // 2-bit codes against the codebook's midpoints, packed per 128-channel slice
 // in the per-head VCODE layout.
 constexpr int kVfTok = 4;   // tokens per workgroup
-__global__ __launch_bounds__(256) void spectral_vfull_kernel(const SpVFullKArgs a) {
-  const int pg = blockIdx.x >> 2, qt = blockIdx.x & 3, tid = threadIdx.x;
+struct VFullLds {
+  float x[kVfTok][kSpMaxC];
+  float acc[kVfTok][8];
+  float norm[kVfTok];
+  uint8_t code[kVfTok][kSpMaxC];
+};
+__device__ __forceinline__ void encode_vfull(const SpVFullKArgs& a, VFullLds& s, int block) {
+  const int pg = block >> 2, qt = block & 3, tid = threadIdx.x;
   const int C = kD * a.h_kv, lc = 7 + __builtin_ctz((unsigned)a.h_kv);   // C = 2^lc (h_kv a power of two)
-  __shared__ float x[kVfTok][kSpMaxC];
-  __shared__ float s_acc[kVfTok][8];
-  __shared__ float s_norm[kVfTok];
-  __shared__ uint8_t code[kVfTok][kSpMaxC];
+  auto& x = s.x;
+  auto& s_acc = s.acc;
+  auto& s_norm = s.norm;
+  auto& code = s.code;
   uint8_t* page = a.pages + clamp_page(a.page_ids[pg], a.n_pool) * (int64_t)a.L.bytes;
   const int tok0 = pg * kPT + kVfTok * qt;
   for (int e = tid; e < kVfTok * C; e += 256) {
@@ -331,6 +191,297 @@ __global__ __launch_bounds__(256) void spectral_vfull_kernel(const SpVFullKArgs 
     }
     *reinterpret_cast<uint32_t*>(page + a.L.vcode + sl * 512 + lane * 8 + w * 4) = dword;
   }
+}
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// x / d correctly rounded from r = fl(1 / d) (k2b_append.hip: div_by).
+__device__ __forceinline__ float sp_div_by(float x, float d, float r) {
+  const float q0 = x * r;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, d, x), r, q0);
+  return __builtin_fmaf(__builtin_fmaf(-q1, d, x), r, q1);
+}
+
+// Block 256.  Workgroups [0, n_blocks): wave w of workgroup g nx + x (nx =
+// ceil(c_pad / 64)) accumulates Y[t][j] for tokens 16w .. 16w + 15 of group g and
+// page columns 64x .. 64x + 63 over the C channels in order, every product and
+// every sum rounded on its own; then the step of each column (max|Y| / qmax and
+// 10 rounds of <Y, Q> / <Q, Q>; for the Lloyd payload the sample deviation and 3
+// rounds of <Y, l> / <l, l>) and its codes, the workgroup's 8 slices assembled in
+// LDS and written with dword stores.  The workgroups after them encode full-C
+// values (encode_vfull), which depend on nothing here and fill the idle slots.
+//
+// Bound: VALU issue.  The format rounds product and sum apart, so no FMA (and
+// no accumulating MFMA) may be used: two VALU instructions a term.  The products
+// come from the fp32 MFMA instead, one outer product (K = 1) of 16 tokens and 64
+// columns at a time with a zero accumulator -- its result is the rounded
+// product, bit for bit, denormals included -- beside the VALU's sums: one VALU
+// instruction a term.  A lane's 16-byte piece of a key row (channels
+// 32c + 8k .. + 7 in the lanes of block k) serves 32 products, its block chosen
+// by the MFMA's A broadcast, so the operands cost a load per 32 channels and one
+// per enc row, with no LDS and no barrier.  The fit's integers and products are
+// made by every wave, its sums (left to right) by one.
+// Measured at C 1024, 968 columns: a call of 1,920 tokens 100.8 us, of 128 tokens
+// 72.8 us; with both operands from LDS (9 reads per 16 VALU), the fit in one wave
+// of 8 and the values in a launch of their own 195.4 and 136.2 us.  3 of 8
+// channels' products on the VALU beside the MFMA's: 127 -> 137 us at 1,920 tokens
+// (the VALU is the bound, not the MFMA).
+// kVec: key rows 16-byte aligned; else the 8 channels are read one by one.
+template <bool kLloyd>
+struct EncodeLds {
+  float y[kGroup][65];                       // Y: [token][column]
+  float l[kGroup][65];                       // <Y, Q> terms; Lloyd: the level of each (token, column)
+  uint32_t code[8 * kGroup * 8 / 4];         // 8 slices of at most 512 bytes
+  float lv[kLloyd ? kLqLevels : 1], mid[kLloyd ? kLqLevels : 1];   // levels, midpoints
+  uint8_t cd[kLloyd ? kGroup : 1][64];       // Lloyd: the final level indices
+  float sc[64], part[4][64];                 // each column's current step; per-wave maxima, <Q, Q>
+};
+
+template <bool kLloyd, bool kVec, int DT>
+__global__ __launch_bounds__(256, 2) void spectral_encode_kernel(const SpEncodeKArgs a, const SpVFullKArgs av) {
+  __shared__ union Lds {
+    EncodeLds<kLloyd> e;
+    VFullLds v;
+  } s_lds;
+  if ((int)blockIdx.x >= a.n_blocks) {
+    encode_vfull(av, s_lds.v, (int)blockIdx.x - a.n_blocks);
+    return;
+  }
+  auto& s_y = s_lds.e.y;
+  auto& s_l = s_lds.e.l;
+  auto& s_code = s_lds.e.code;
+  auto& s_lv = s_lds.e.lv;
+  auto& s_mid = s_lds.e.mid;
+  auto& s_cd = s_lds.e.cd;
+  auto& s_sc = s_lds.e.sc;
+  auto& s_part = s_lds.e.part;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nx = (a.c_pad + 63) >> 6, g = blockIdx.x / nx, bx = blockIdx.x - g * nx, j = bx * 64 + lane;
+  const bool active = j < a.c_pad;
+  constexpr bool lloyd = kLloyd;
+  if (lloyd)
+    for (int i = tid; i < kLqLevels; i += 256) s_lv[i] = a.lq[i];
+  {
+    // the lane's key row: token lane & 15 of the wave's 16, piece k = lane >> 4
+    const int64_t row = (int64_t)(g * kGroup + 16 * wave + (lane & 15)) * a.kst;
+    struct Piece {   // channels c32 + 8k .. + 7 as they lie in memory
+      uint32_t w[DT == BMX_K2B_F32 ? 8 : 4];
+      __device__ __forceinline__ float at(int v) const {
+        if constexpr (DT == BMX_K2B_F32) return __uint_as_float(w[v]);
+        const uint32_t u = (v & 1) ? w[v >> 1] >> 16 : w[v >> 1] & 0xffffu;
+        return DT == BMX_K2B_BF16 ? __uint_as_float(u << 16) : half_bits_to_float((uint16_t)u);
+      }
+    };
+    auto load_m = [&](int c32, Piece& m) {
+      const int c = c32 + 8 * (lane >> 4);
+      const int64_t at = (c >> 7) * a.ksh + row + (c & (kD - 1));
+      constexpr int NW = DT == BMX_K2B_F32 ? 8 : 4;
+      if constexpr (kVec) {
+        const uint4* p = reinterpret_cast<const uint4*>(static_cast<const char*>(a.k) + at * (NW / 2));
+#pragma unroll
+        for (int i = 0; i < NW / 4; ++i) {
+          const uint4 v = p[i];
+          m.w[4 * i] = v.x; m.w[4 * i + 1] = v.y; m.w[4 * i + 2] = v.z; m.w[4 * i + 3] = v.w;
+        }
+      } else if constexpr (DT == BMX_K2B_F32) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m.w[i] = static_cast<const uint32_t*>(a.k)[at + i];
+      } else {
+        const uint16_t* p = static_cast<const uint16_t*>(a.k) + at;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m.w[i] = p[2 * i] | (uint32_t)p[2 * i + 1] << 16;
+      }
+    };
+    // enc rows through a buffer descriptor: row offset scalar, column offset fixed
+    const auto enc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.encp), (short)0,
+                                                       (int)((int64_t)a.C * a.c_pad * 4), 0x00020000);
+    const int ecol = 4 * min(j, a.c_pad - 1);
+    auto load_e = [&](int c32, float (&e)[32]) {
+#pragma unroll
+      for (int c = 0; c < 32; ++c)
+        e[c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(enc, ecol, (c32 + c) * a.c_pad * 4, 0));
+    };
+    f32x16_t y;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) y[i] = 0.f;
+    const f32x16_t zero = y;
+    // 32 channels: products two channels ahead of the sums, so that the sums do not
+    // wait for the MFMA; meanwhile the next 32 channels' operands are in flight
+    f32x16_t p0, p1;
+    auto product = [&](auto kc, const float (&mv)[8], const float (&e)[32], int v) {   // channel 8k + v
+      constexpr int k = decltype(kc)::value;   // value v of block k of the A operand
+      return __builtin_amdgcn_mfma_f32_16x16x1f32(mv[v], e[8 * k + v], zero, 2, k, 0);
+    };
+    auto eight = [&](auto kc, const float (&mv)[8], const float (&e)[32], auto kn, const float (&mn)[8],
+                     const float (&en)[32]) {
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        const f32x16_t p2 = v < 6 ? product(kc, mv, e, v + 2) : product(kn, mn, en, v - 6);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) y[i] = __fadd_rn(y[i], p0[i]);
+        __builtin_amdgcn_sched_barrier(0);
+        p0 = p1;
+        p1 = p2;
+      }
+    };
+    using K0 = std::integral_constant<int, 0>;
+    using K1 = std::integral_constant<int, 1>;
+    using K2 = std::integral_constant<int, 2>;
+    using K3 = std::integral_constant<int, 3>;
+    auto values = [&](const Piece& m, float (&mv)[8]) {
+#pragma unroll
+      for (int v = 0; v < 8; ++v) mv[v] = m.at(v);
+    };
+    Piece m0, m1;
+    float e0[32], e1[32], mv0[8], mv1[8];
+    load_m(0, m0);
+    load_e(0, e0);
+    load_m(32, m1);
+    load_e(32, e1);
+    values(m0, mv0);
+    p0 = product(K0{}, mv0, e0, 0);
+    p1 = product(K0{}, mv0, e0, 1);
+    auto step = [&](const float (&mv)[8], float (&e)[32], Piece& m, const Piece& mnext, float (&mvn)[8],
+                    const float (&en)[32], int c_load) {
+      eight(K0{}, mv, e, K1{}, mv, e);
+      eight(K1{}, mv, e, K2{}, mv, e);
+      eight(K2{}, mv, e, K3{}, mv, e);
+      values(mnext, mvn);
+      eight(K3{}, mv, e, K0{}, mvn, en);
+      c_load = min(c_load, a.C - 32);
+      load_m(c_load, m);
+      load_e(c_load, e);
+    };
+    for (int c0 = 0; c0 < a.C; c0 += 64) {   // C is a multiple of 128
+      step(mv0, e0, m0, m1, mv1, e1, c0 + 64);
+      step(mv1, e1, m1, m0, mv0, e0, c0 + 96);
+    }
+    // lane 16 r + n holds, in 4b + i, row 4r + i and column 16b + n
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s_y[16 * wave + 4 * (lane >> 4) + (i & 3)][16 * (i >> 2) + (lane & 15)] = y[i];
+  }
+  __syncthreads();
+  // midpoints (l_i + l_{i+1}) / 2 within each tier (the slot after a tier's
+  // last level is never read)
+  if (lloyd)
+    for (int i = tid; i + 1 < kLqLevels; i += 256) s_mid[i] = (s_lv[i] + s_lv[i + 1]) * 0.5f;
+  const int s = j >> 3, k = j & 7;
+  const uint32_t tab = active ? (uint32_t)a.slice_tab[s] : 0u;
+  const int b = active ? (int)(tab >> 24) : 2, w = sp_width(b);
+  const float qmax = (float)((1 << (b - 1)) - 1);
+  const float* lv = s_lv + (kLloyd ? lq_off(b) : 0);
+  const float* mid = s_mid + (kLloyd ? lq_off(b) : 0);
+  float scale = 1e-12f;
+  float yv[16];   // column j's values of the wave's 16 tokens
+#pragma unroll
+  for (int i = 0; i < 16; ++i) yv[i] = active ? s_y[16 * wave + i][lane] : 0.f;
+  // the codes' integers of the wave's tokens at the current step: rint(y / scale)
+  // clamped; the short division where its operands are in range
+  float qv[16];
+  auto quantize = [&](float amax) {
+    const float rs = 1.0f / scale;
+    if (__all(amax * rs < 1e37f && scale < 3e38f)) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) qv[i] = fminf(fmaxf(rintf(sp_div_by(yv[i], scale, rs)), -qmax - 1.f), qmax);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) qv[i] = fminf(fmaxf(rintf(yv[i] / scale), -qmax - 1.f), qmax);
+    }
+  };
+  if constexpr (kLloyd) {
+    // the starting step in wave 0 (lane = column), then 4 rounds: every wave
+    // finds the level indices of its tokens (binary searches in parallel), and
+    // for the 3 refits wave 0 sums <Y, l> and <l, l> left to right
+    if (wave == 0) {
+      double sum = 0.0;
+      for (int t = 0; t < kGroup; ++t) sum += (double)s_y[t][lane];
+      const double mean = sum / 64.0;
+      double ss = 0.0;
+      for (int t = 0; t < kGroup; ++t) {
+        const double d = (double)s_y[t][lane] - mean;
+        ss += d * d;
+      }
+      s_sc[lane] = fmaxf((float)__dsqrt_rn(ss / 63.0), 1e-12f);
+    }
+    for (int r = 0; r <= 3; ++r) {
+      __syncthreads();   // the step written; the previous round's levels read
+      const float sc = s_sc[lane];
+      for (int t = wave; t < kGroup; t += 4) {
+        const int c = lq_index(mid, b, s_y[t][lane] / sc);
+        if (r < 3) s_l[t][lane] = lv[c];
+        else s_cd[t][lane] = (uint8_t)c;
+      }
+      if (r == 3) break;
+      __syncthreads();
+      if (wave == 0) {
+        float num = 0.f, den = 0.f;
+        for (int t = 0; t < kGroup; ++t) {
+          const float yy = s_y[t][lane], l = s_l[t][lane];
+          num = __fadd_rn(num, __fmul_rn(yy, l));
+          den = __fadd_rn(den, __fmul_rn(l, l));
+        }
+        s_sc[lane] = fmaxf(num / fmaxf(den, 1e-12f), 1e-12f);
+      }
+    }
+    scale = s_sc[lane];
+  } else {
+    // every wave its 16 tokens' integers and products; the products' sum left to
+    // right in wave 0, the integers' squares (exact in any order: at most 2^20)
+    // by wave
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(yv[i]));
+    s_part[wave][lane] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(s_part[0][lane], s_part[1][lane]), fmaxf(s_part[2][lane], s_part[3][lane]));
+    scale = fmaxf(amax, 1e-12f) / qmax;
+    __syncthreads();   // the maxima read
+    for (int it = 0; it < 10; ++it) {
+      quantize(amax);
+      float den = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s_l[16 * wave + i][lane] = __fmul_rn(yv[i], qv[i]);
+        den = __builtin_fmaf(qv[i], qv[i], den);
+      }
+      s_part[wave][lane] = den;
+      __syncthreads();
+      if (wave == 0) {
+        float num = 0.f;
+#pragma unroll 16
+        for (int t = 0; t < kGroup; ++t) num = __fadd_rn(num, s_l[t][lane]);
+        den = (s_part[0][lane] + s_part[1][lane]) + (s_part[2][lane] + s_part[3][lane]);
+        s_sc[lane] = fmaxf(num / fmaxf(den, 1e-12f), 1e-12f);
+      }
+      __syncthreads();
+      scale = s_sc[lane];
+    }
+    quantize(amax);
+  }
+  // the block's slices are contiguous in the page: [base, end)
+  const int n_sl = a.c_pad >> 3, s_first = bx * 8, s_last = min(s_first + 8, n_sl) - 1;
+  const uint32_t tab0 = (uint32_t)a.slice_tab[s_first], tabl = (uint32_t)a.slice_tab[s_last];
+  const int base = (int)(tab0 & 0xFFFFFFu);
+  const int n_words = ((int)(tabl & 0xFFFFFFu) + kGroup * sp_width((int)(tabl >> 24)) - base) >> 2;
+  for (int i = tid; i < n_words; i += 256) s_code[i] = 0u;
+  __syncthreads();
+  if (active) {
+    const int bit0 = ((int)(tab & 0xFFFFFFu) - base) * 8 + k * w;
+    const uint32_t bias = 1u << (b - 1);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int t = 16 * wave + i;
+      const uint32_t stored = lloyd ? (uint32_t)s_cd[kLloyd ? t : 0][lane] : (uint32_t)((int)qv[i] + (int)bias);
+      const int bit = bit0 + t * w * 8;
+      atomicOr(&s_code[bit >> 5], stored << (bit & 31));
+    }
+  }
+  __syncthreads();
+  uint8_t* page = a.pages + clamp_page(a.page_ids[g], a.n_pool) * (int64_t)a.page_bytes;
+  uint32_t* dst = reinterpret_cast<uint32_t*>(page + base);
+  for (int i = tid; i < n_words; i += 256) dst[i] = s_code[i];
+  if (active && wave == 0) reinterpret_cast<uint16_t*>(page)[j] = float_to_half_bits(scale);
 }
 
 struct SpDequantKArgs {
@@ -1896,21 +2047,35 @@ extern "C" int32_t bmx_spectral_append(const bmx_spectral_append_args* a, void* 
   k.k = a->k_pre; k.ksh = a->k_sh; k.kst = a->k_st;
   k.encp = a->enc_perm; k.slice_tab = a->L.slice_tab; k.pages = a->k_pages; k.page_ids = a->k_page_ids;
   k.lq = a->L.lloyd_levels;
-  if (k.lq)
-    hipLaunchKernelGGL(spectral_encode_kernel<true>, dim3((a->L.c_pad + 63) / 64, a->n_groups), dim3(512), 0, st, k);
-  else
-    hipLaunchKernelGGL(spectral_encode_kernel<false>, dim3((a->L.c_pad + 63) / 64, a->n_groups), dim3(512), 0, st, k);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess && a->v_codec == BMX_SPECTRAL_V_FULL) {
-    SpVFullKArgs v{};
+  const int elem = a->k_dtype == BMX_K2B_F32 ? 4 : 2;
+  const bool vec = (reinterpret_cast<uintptr_t>(a->k_pre) & 15) == 0 && a->k_sh * elem % 16 == 0 && a->k_st * elem % 16 == 0;
+  // full-C values ride in the same launch (4 workgroups a page, independent of the keys')
+  SpVFullKArgs v{};
+  int v_blocks = 0;
+  if (a->v_codec == BMX_SPECTRAL_V_FULL) {
     v.h_kv = a->L.h_kv; v.n_pool = a->n_v_pool; v.v_dtype = a->v_dtype;
     v.v = a->v; v.vsh = a->v_sh; v.vst = a->v_st;
     v.pages = a->v_pages; v.page_ids = a->v_page_ids; v.L = value_layout(a->L.h_kv, true);
     for (int i = 0; i < 4; ++i) v.codebook[i] = a->v_codebook[i];
     for (int i = 0; i < 32; ++i) v.sign_c[i] = a->v_sign_bits_c[i];
-    hipLaunchKernelGGL(spectral_vfull_kernel, dim3(4 * 4 * a->n_groups), dim3(256), 0, st, v);
-    e = hipGetLastError();
-  } else if (e == hipSuccess) {
+    v_blocks = 4 * 4 * a->n_groups;
+  }
+  k.n_blocks = (a->L.c_pad + 63) / 64 * a->n_groups;
+  auto encode = [&](auto dt) {
+    auto launch = [&](auto lq, auto vc) {
+      hipLaunchKernelGGL((spectral_encode_kernel<decltype(lq)::value, decltype(vc)::value, decltype(dt)::value>),
+                         dim3(k.n_blocks + v_blocks), dim3(256), 0, st, k, v);
+    };
+    if (k.lq && vec) launch(std::true_type{}, std::true_type{});
+    else if (k.lq) launch(std::true_type{}, std::false_type{});
+    else if (vec) launch(std::false_type{}, std::true_type{});
+    else launch(std::false_type{}, std::false_type{});
+  };
+  if (a->k_dtype == BMX_K2B_F32) encode(std::integral_constant<int, BMX_K2B_F32>{});
+  else if (a->k_dtype == BMX_K2B_BF16) encode(std::integral_constant<int, BMX_K2B_BF16>{});
+  else encode(std::integral_constant<int, BMX_K2B_F16>{});
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess && a->v_codec != BMX_SPECTRAL_V_FULL) {
     AppendKArgs v{};
     v.h_kv = a->L.h_kv; v.n_pool = a->n_v_pool;
     v.v = a->v; v.vsh = a->v_sh; v.vst = a->v_st; v.v_dtype = a->v_dtype;
