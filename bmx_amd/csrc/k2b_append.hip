@@ -39,26 +39,48 @@ __device__ __forceinline__ float div_by(float x, float d, float r) {
   return __builtin_fmaf(__builtin_fmaf(-q1, d, x), r, q1);
 }
 
+// 4x4 transpose between four registers and the four 16-lane rows of a wave:
+// register e of row q in, register q of row e out.
+__device__ __forceinline__ void transpose_rows(float (&x)[8], int at) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  uint32_t w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = __float_as_uint(x[at + e]);
+  const u32x2 a = __builtin_amdgcn_permlane16_swap(w[0], w[1], false, false);   // odd rows of the first, even of the second
+  const u32x2 b = __builtin_amdgcn_permlane16_swap(w[2], w[3], false, false);
+  const u32x2 c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);   // upper half of the first, lower of the second
+  const u32x2 d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  x[at] = __uint_as_float(c[0]);
+  x[at + 1] = __uint_as_float(d[0]);
+  x[at + 2] = __uint_as_float(c[1]);
+  x[at + 3] = __uint_as_float(d[1]);
+}
+
 // grid (16-token pages of the call, R / 16), block 256 = 4 waves.
 // Us[t][r] = sum_c M[t][c] basis32[c][r] in fp32 (the reference's M @ V): wave w
-// sums channels [w C/4, (w+1) C/4) in order, lane (t = lane & 15, rq = lane >> 4)
-// owns ranks 16 blockIdx.y + 4 rq .. + 3, and the four partial sums are added in
-// wave order.  The first codec page of a sequence takes its SVD factor instead.
-// Bound: one wave's chain of C / 4 dependent steps (a commit of one codec page
-// has only 8 R / 16 workgroups), so a step must cost its 4 FMAs and no memory
-// round trip: the workgroup's 16 basis columns are staged in LDS up front, the
-// lane's key row is read 8 channels per 16-byte load with 16 loads in flight,
-// and a chunk's basis values leave LDS a chunk ahead of their FMAs.
-// Measured at h_kv 8: 10.8 us for one codec page at R 32, 16.3 us for 63 at
-// R 16; with the basis read from global memory inside the chain and the keys
-// staged in LDS 26.0 and 35.4 us.
+// sums channels [w C/4, (w+1) C/4) in order, and the four partial sums are added
+// in wave order.  The first codec page of a sequence takes its SVD factor instead.
+// The wave's 16 tokens x 16 ranks go on v_mfma_f32_16x16x4_f32, which adds its 4
+// products one after another, each as an fma: 64 instructions make the chain of
+// 256 steps that a lane's own FMAs made (C 1024), with the same bits.  Its A
+// operand is token lane & 15, channel 4 m + (lane >> 4) of step m: a lane loads 8
+// channels of its token (16 bytes) at 8 (lane >> 4) of a 32-channel chunk, and two
+// 4x4 transposes across the wave's rows put them in order.  Its B operand is one
+// dword a lane, whole lines of basis32, straight from memory.
+// Bound: the chain (a commit of one codec page has only 8 R / 16 workgroups) and
+// the round trip before it: the loads of 8 chunks, a quarter of C 1024, are in
+// flight at once, and there is no barrier before the sum over the waves.
+// Measured at h_kv 8: 5.7 us for one codec page at R 32, 8.4 us for 63 at
+// R 16; with FMAs on the VALU and the basis columns staged in LDS 10.8 and 16.3 us.
 // kVec: rows 16-byte aligned; else the 8 channels are read one by one.
+constexpr int kUsSets = 8;   // chunks of 32 channels in flight
+
 template <bool kVec>
-__global__ __launch_bounds__(256) void append_us_kernel(const AppendKArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float s_b[];   // [C][16] fp32 basis columns
+__global__ __launch_bounds__(256, 2) void append_us_kernel(const AppendKArgs a) {
   __shared__ float s_part[4][kPT][17];
   const int pg = blockIdx.x, rg = blockIdx.y;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int C = a.C, R = a.R, ld = a.log2d, d = 1 << ld;
   uint8_t* page = append_page(a, pg);
   uint16_t* us = reinterpret_cast<uint16_t*>(page + a.L.us);
@@ -68,75 +90,54 @@ __global__ __launch_bounds__(256) void append_us_kernel(const AppendKArgs a) {
     us[oi] = float_to_half_bits(a.us_first[(pg * kPT + ot) * R + orank]);
     return;
   }
-  const int t = lane & 15, rq = lane >> 4;
-  const uint16_t* row = a.k_pre + (int64_t)(pg * kPT + t) * a.kst;
-  const int c0 = wave * (C / 4), n8 = C / 32;     // the wave's channels, in chunks of 8
-  auto load8 = [&](int k) -> uint4 {
-    const int c = c0 + 8 * min(k, n8 - 1);
+  const int n = lane & 15, q = lane >> 4;
+  const int Q = C / 4, c0 = wave * Q;             // the wave's channels: a multiple of 8
+  const int n32 = (Q + 31) / 32;                  // chunks, the last of 8, 16, 24 or 32 channels
+  const uint16_t* row = a.k_pre + (int64_t)(pg * kPT + n) * a.kst;
+  const float* bp = a.basis32 + (int64_t)(c0 + q) * R + 16 * rg + n;
+  uint4 kx[kUsSets];
+  float bx[kUsSets][8];
+  auto load = [&](int s, int k) {   // chunk k; past the wave's channels: its last ones again, not used
+    const int c = c0 + min(32 * k + 8 * q, Q - 8);
     const uint16_t* p = row + (int64_t)(c >> ld) * a.ksh + (c & (d - 1));
-    if constexpr (kVec) return *reinterpret_cast<const uint4*>(p);
-    uint32_t w[4];
+    if constexpr (kVec) {
+      kx[s] = *reinterpret_cast<const uint4*>(p);
+    } else {
+      uint32_t w[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = p[2 * i] | (uint32_t)p[2 * i + 1] << 16;
-    return make_uint4(w[0], w[1], w[2], w[3]);
-  };
-  // the row in batches of 4 chunks, 4 batches in flight (a ring of registers)
-  constexpr int kB = 4, kSets = 4;
-  const int nb = n8 / kB;
-  uint4 ring[kSets][kB];
-#pragma unroll
-  for (int s = 0; s < kSets; ++s)
-#pragma unroll
-    for (int i = 0; i < kB; ++i) ring[s][i] = load8(kB * s + i);
-  for (int e0 = tid; e0 < C * 4; e0 += 8 * 256) {   // 8 loads in flight per thread
-    float4_t v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = min(e0 + 256 * i, C * 4 - 1);
-      v[i] = *reinterpret_cast<const float4_t*>(a.basis32 + (int64_t)(e >> 2) * R + 16 * rg + 4 * (e & 3));
+      for (int i = 0; i < 4; ++i) w[i] = p[2 * i] | (uint32_t)p[2 * i + 1] << 16;
+      kx[s] = make_uint4(w[0], w[1], w[2], w[3]);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (e0 + 256 * i < C * 4) reinterpret_cast<float4_t*>(s_b)[e0 + 256 * i] = v[i];
-  }
-  __syncthreads();
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  float4_t b[2][8];   // the basis values of a chunk, read one chunk ahead of their FMAs
-  auto read_b = [&](float4_t (&dst)[8], int k) {
-    const float4_t* p = reinterpret_cast<const float4_t*>(s_b + (c0 + 8 * min(k, n8 - 1)) * 16 + 4 * rq);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) dst[j] = p[4 * j];
+    for (int m = 0; m < 8; ++m) bx[s][m] = bp[(int64_t)min(32 * k + 4 * m, Q - 4) * R];
   };
-  auto chunk = [&](const uint4& x, const float4_t (&bv)[8]) {
-    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float m = (float)as_h2(w[j >> 1])[j & 1];
+  for (int s = 0; s < kUsSets; ++s)
+    if (s < n32) load(s, s);
+  float4_t acc = {0.f, 0.f, 0.f, 0.f};   // tokens 4 q + i, rank 16 rg + n
+  for (int k0 = 0; k0 < n32; k0 += kUsSets) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] = __builtin_fmaf(m, bv[j][r], acc[r]);
-    }
-  };
-  read_b(b[0], 0);
-  for (int k0 = 0; k0 < nb; k0 += kSets) {
+    for (int s = 0; s < kUsSets; ++s) {
+      const int k = k0 + s;
+      if (k >= n32) break;
+      const uint32_t w[4] = {kx[s].x, kx[s].y, kx[s].z, kx[s].w};
+      float m[8];
 #pragma unroll
-    for (int s = 0; s < kSets; ++s) {
-      if (k0 + s >= nb) break;
+      for (int e = 0; e < 8; ++e) m[e] = (float)as_h2(w[e >> 1])[e & 1];
+      transpose_rows(m, 0);   // channels 8 i + q
+      transpose_rows(m, 4);   // channels 8 i + 4 + q
+      const int steps = (Q - 32 * k) / 4;
 #pragma unroll
-      for (int i = 0; i < kB; ++i) {
-        read_b(b[(i + 1) & 1], kB * (k0 + s) + i + 1);
-        __builtin_amdgcn_sched_barrier(0);   // the reads stay a chunk ahead
-        chunk(ring[s][i], b[i & 1]);
+      for (int i = 0; i < 4; ++i) {
+        if (2 * i >= steps) break;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(m[i], bx[s][2 * i], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(m[4 + i], bx[s][2 * i + 1], acc, 0, 0, 0);
       }
-#pragma unroll
-      for (int i = 0; i < kB; ++i) ring[s][i] = load8(kB * (k0 + s + kSets) + i);
+      if (k + kUsSets < n32) load(s, k + kUsSets);
     }
   }
-  for (int k = kB * nb; k < n8; ++k) {   // C / 32 not a multiple of 4
-    read_b(b[0], k);
-    chunk(load8(k), b[0]);
-  }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) s_part[wave][t][4 * rq + r] = acc[r];
+  for (int i = 0; i < 4; ++i) s_part[wave][4 * q + i][n] = acc[i];
   __syncthreads();
   const int o = tid & 15;
   us[oi] = float_to_half_bits(((s_part[0][ot][o] + s_part[1][ot][o]) + s_part[2][ot][o]) + s_part[3][ot][o]);
@@ -426,18 +427,11 @@ hipError_t launch_k2b_values(const AppendKArgs& a, int n_pages16, int h_kv, hipS
   return hipGetLastError();
 }
 
-// Us of every page slot: the basis columns take C 64 bytes of LDS, above 64 KB
-// with the partial sums from C 1024 on (the limit is raised once).
-static hipError_t launch_us(const AppendKArgs& k, int n_slots, hipStream_t st) {
-  const size_t lds = (size_t)k.C * 16 * sizeof(float);
+static void launch_us(const AppendKArgs& k, int n_slots, hipStream_t st) {
   const bool vec = (reinterpret_cast<uintptr_t>(k.k_pre) & 15) == 0 && k.ksh % 8 == 0 && k.kst % 8 == 0;
-  const void* fn = vec ? (const void*)append_us_kernel<true> : (const void*)append_us_kernel<false>;
-  const hipError_t e = bmx_ensure_dynamic_lds(fn, lds);
-  if (e != hipSuccess) return e;
   const dim3 grid(n_slots, k.R / 16);
-  if (vec) hipLaunchKernelGGL(append_us_kernel<true>, grid, dim3(256), lds, st, k);
-  else hipLaunchKernelGGL(append_us_kernel<false>, grid, dim3(256), lds, st, k);
-  return hipGetLastError();
+  if (vec) hipLaunchKernelGGL(append_us_kernel<true>, grid, dim3(256), 0, st, k);
+  else hipLaunchKernelGGL(append_us_kernel<false>, grid, dim3(256), 0, st, k);
 }
 
 template <int R>
@@ -496,8 +490,7 @@ extern "C" int bmx_k2b_append(const bmx_k2b_append_args* a, void* stream) {
   set_code_cuts(k, a->codebook, geo.d);
   hipStream_t st = (hipStream_t)stream;
   const int slots = a->n_codec_pages * 8;
-  hipError_t e = launch_us(k, slots, st);
-  if (e != hipSuccess) return afail(BMX_E_HIP, std::string("bmx_k2b_append: launch: ") + hipGetErrorString(e));
+  launch_us(k, slots, st);
   if (!geo.general) {
     const int n_res = a->n_codec_pages * 2 * g.h_kv;   // workgroups of the residual, and as many of the values
     if (geo.R == 32) hipLaunchKernelGGL(append_codes_kernel<32>, dim3(2 * n_res), dim3(512), 0, st, k, n_res);
@@ -513,7 +506,7 @@ extern "C" int bmx_k2b_append(const bmx_k2b_append_args* a, void* stream) {
     else if (geo.d == 64) hipLaunchKernelGGL(value_codes_kernel<64>, vgrid, dim3(128), 0, st, k);
     else hipLaunchKernelGGL(value_codes_kernel<128>, vgrid, dim3(128), 0, st, k);
   }
-  e = hipGetLastError();
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return afail(BMX_E_HIP, std::string("bmx_k2b_append: launch: ") + hipGetErrorString(e));
   return BMX_OK;
 }

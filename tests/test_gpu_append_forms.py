@@ -37,7 +37,9 @@ def _odd_rows(t):
 # (h, d, rank, group, bits): tokens per thread group * d / 512 = 1, 2, 4, 8, 16, 32 with each rank
 @pytest.mark.parametrize("h,d,rank,group,bits", [
     (1, 32, 16, 16, 2), (3, 32, 32, 32, 4), (4, 64, 64, 32, 3), (2, 64, 128, 64, 3), (5, 128, 16, 64, 4),
-    (1, 128, 128, 128, 3), (2, 128, 64, 16, 2), (1, 128, 32, 64, 3), (7, 128, 16, 64, 3)])
+    (1, 128, 128, 128, 3), (2, 128, 64, 16, 2), (1, 128, 32, 64, 3), (7, 128, 16, 64, 3),
+    # a wave's share of the channels ends in a chunk of 8, and takes two rounds of chunks
+    (5, 32, 16, 16, 2), (16, 128, 32, 64, 3)])
 def test_append_forms_bit_exact(h, d, rank, group, bits):
     gen = torch.Generator().manual_seed(h * 1000 + d + rank)
     S, C = 256, h * d
