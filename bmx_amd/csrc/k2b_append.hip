@@ -143,14 +143,16 @@ __global__ __launch_bounds__(256, 2) void append_us_kernel(const AppendKArgs a) 
   us[oi] = float_to_half_bits(((s_part[0][ot][o] + s_part[1][ot][o]) + s_part[2][ot][o]) + s_part[3][ot][o]);
 }
 
-// One residual group's tokens x one head's channels, 512 threads: thread
-// (channel j = tid % d, part tid / d) takes tokens part, part + 512/d, ...
-// (PER of them): L = sum_r Us16[t][r] basis16[c][r] (fp32, ranks in order),
-// R = M - L; the channel's scale is max |R| over the group / qmax and its codes
-// clamp(rint(R / scale), -qmax - 1, qmax).  VALU-bound: R FMAs per element.
-// The thread's basis row stays in registers (fp16 pairs, exact) and a token's
-// Us row is one LDS broadcast per 8 ranks: 32 FMAs to 4 LDS reads at R 32,
-// where both operands from LDS made 2 reads per FMA.
+// One residual group's tokens x one head's channels, 512 threads: a thread has
+// one channel and PER tokens: L = sum_r Us16[t][r] basis16[c][r] (fp32, ranks in
+// order), R = M - L; the channel's scale is max |R| over the group / qmax and its
+// codes clamp(rint(R / scale), -qmax - 1, qmax).  VALU-bound.
+// Recipe's page (64 tokens, 128 channels): L on v_mfma_f32_16x16x4_f32 as Us is
+// (the same bits as the chain of FMAs), a wave for 16 channels; the page's Us and
+// the basis rows are read as the decode kernels read them, 4 or 8 ranks a lane.
+// General page: thread (channel j = tid % d, part tid / d) takes tokens part,
+// part + 512/d, ...; its basis row stays in registers (fp16 pairs, exact) and a
+// token's Us row is one LDS broadcast per 8 ranks.
 template <int R, int PER>
 struct ResidualLds {
   static constexpr int kNG = 16 * PER < 128 ? 16 * PER : 128;   // tokens of a group, at most
@@ -164,42 +166,84 @@ __device__ __forceinline__ void encode_residual(const AppendKArgs& a, ResidualLd
   const int tid = threadIdx.x, ld = kGeneral ? a.log2d : 7, D = 1 << ld;
   const int NG = (512 * PER) >> ld, C = a.C;
   const int slot0 = gi * (NG / kPT);                 // first 16-token page slot of the group
-  const int j = tid & (D - 1), part = tid >> ld, parts = 512 >> ld;
-  half8_t b[R / 8];                                  // the channel's basis row
-  const uint16_t* bp = a.basis16 + (int64_t)(h * D + j) * R;
-  if ((reinterpret_cast<uintptr_t>(a.basis16) & 15) == 0) {
-#pragma unroll
-    for (int i = 0; i < R / 8; ++i) b[i] = *reinterpret_cast<const half8_t*>(bp + 8 * i);
-  } else {
-#pragma unroll
-    for (int i = 0; i < R; ++i) b[i / 8][i % 8] = __builtin_bit_cast(_Float16, bp[i]);
-  }
+  const int n = tid & 15, q = (tid >> 4) & 3;
+  const int j = kGeneral ? tid & (D - 1) : 16 * (tid >> 6) + n, part = kGeneral ? tid >> ld : q;
+  const int parts = kGeneral ? 512 >> ld : 4;
+  auto tok = [&](int k) { return kGeneral ? part + parts * k : 16 * (k >> 2) + 4 * q + (k & 3); };
+  const bool aligned = (reinterpret_cast<uintptr_t>(a.basis16) & 15) == 0;
   float res[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k)
-    res[k] = half_bits_to_float(a.k_pre[h * a.ksh + (int64_t)(slot0 * kPT + part + parts * k) * a.kst + j]);
-  for (int e = tid; e < NG * R / 2; e += 512) {      // rank pairs (2 e' even: within one row of either page)
-    const int t = 2 * e / R, r = 2 * e % R;
-    const uint8_t* page = append_page(a, slot0 + t / kPT);
-    const int i = kGeneral ? (t % kPT) * R + r : us_half(R, t % kPT, r);
-    reinterpret_cast<uint32_t*>(s.us)[e] = *reinterpret_cast<const uint32_t*>(page + a.L.us + 2 * i);
-  }
-  __syncthreads();
+    res[k] = half_bits_to_float(a.k_pre[h * a.ksh + (int64_t)(slot0 * kPT + tok(k)) * a.kst + j]);
   float amax = 0.f;
+  if constexpr (kGeneral) {
+    half8_t b[R / 8];                                  // the channel's basis row
+    const uint16_t* bp = a.basis16 + (int64_t)(h * D + j) * R;
+    if (aligned) {
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const half8_t* u = reinterpret_cast<const half8_t*>(s.us + (part + parts * k) * R);
-    float L = 0.f;
+      for (int i = 0; i < R / 8; ++i) b[i] = *reinterpret_cast<const half8_t*>(bp + 8 * i);
+    } else {
 #pragma unroll
-    for (int i = 0; i < R / 8; ++i) {
-      const half8_t uv = u[i];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) L = __builtin_fmaf((float)uv[e], (float)b[i][e], L);
+      for (int i = 0; i < R; ++i) b[i / 8][i % 8] = __builtin_bit_cast(_Float16, bp[i]);
     }
-    res[k] = res[k] - L;
-    amax = fmaxf(amax, fabsf(res[k]));
+    for (int e = tid; e < NG * R / 2; e += 512) {      // rank pairs (2 e' even: within one row)
+      const int t = 2 * e / R, r = 2 * e % R;
+      reinterpret_cast<uint32_t*>(s.us)[e] =
+          *reinterpret_cast<const uint32_t*>(append_page(a, slot0 + t / kPT) + a.L.us + 2 * ((t % kPT) * R + r));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const half8_t* u = reinterpret_cast<const half8_t*>(s.us + tok(k) * R);
+      float L = 0.f;
+#pragma unroll
+      for (int i = 0; i < R / 8; ++i) {
+        const half8_t uv = u[i];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) L = __builtin_fmaf((float)uv[e], (float)b[i][e], L);
+      }
+      res[k] = res[k] - L;
+      amax = fmaxf(amax, fabsf(res[k]));
+    }
+  } else {
+    // lane (n, q): ranks KQ q .. + KQ - 1 of token (A) or channel (B) n; after the
+    // transposes register i holds rank 4 i + q of the step that takes it
+    constexpr int KQ = R / 4;
+    typedef _Float16 hvec_t __attribute__((ext_vector_type(KQ)));
+    auto in_order = [&](const hvec_t& x, float (&f)[8]) {
+#pragma unroll
+      for (int e = 0; e < KQ; ++e) f[e] = (float)x[e];
+      transpose_rows(f, 0);
+      if constexpr (KQ == 8) transpose_rows(f, 4);
+    };
+    auto step = [](const float (&f)[8], int m) { return KQ == 8 ? f[4 * (m & 1) + (m >> 1)] : f[m]; };
+    hvec_t uh[PER / 4], bh;
+#pragma unroll
+    for (int k = 0; k < PER / 4; ++k)
+      uh[k] = *reinterpret_cast<const hvec_t*>(append_page(a, slot0 + k) + a.L.us + (tid & 63) * (2 * KQ));
+    const uint16_t* bp = a.basis16 + (int64_t)(h * D + j) * R + KQ * q;
+    if (aligned) {
+      bh = *reinterpret_cast<const hvec_t*>(bp);
+    } else {
+#pragma unroll
+      for (int i = 0; i < KQ; ++i) bh[i] = __builtin_bit_cast(_Float16, bp[i]);
+    }
+    float bf[8], uf[8];
+    in_order(bh, bf);
+#pragma unroll
+    for (int k = 0; k < PER / 4; ++k) {
+      in_order(uh[k], uf);
+      float4_t L = {0.f, 0.f, 0.f, 0.f};   // tokens 16 k + 4 q + i, the lane's channel
+#pragma unroll
+      for (int m = 0; m < R / 4; ++m) L = __builtin_amdgcn_mfma_f32_16x16x4f32(step(uf, m), step(bf, m), L, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        res[4 * k + i] = res[4 * k + i] - L[i];
+        amax = fmaxf(amax, fabsf(res[4 * k + i]));
+      }
+    }
   }
-  s.amax[tid] = amax;
+  s.amax[(part << ld) + j] = amax;
   __syncthreads();
   float mx = s.amax[j];
   for (int p = 1; p < parts; ++p) mx = fmaxf(mx, s.amax[(p << ld) + j]);
@@ -212,11 +256,11 @@ __device__ __forceinline__ void encode_residual(const AppendKArgs& a, ResidualLd
     const float rs = 1.0f / scale;
 #pragma unroll
     for (int k = 0; k < PER; ++k)
-      s.code[(part + parts * k) * (D + 4) + j] = (int8_t)fminf(fmaxf(rintf(div_by(res[k], scale, rs)), lo), hi);
+      s.code[tok(k) * (D + 4) + j] = (int8_t)fminf(fmaxf(rintf(div_by(res[k], scale, rs)), lo), hi);
   } else {
 #pragma unroll
     for (int k = 0; k < PER; ++k)
-      s.code[(part + parts * k) * (D + 4) + j] = (int8_t)fminf(fmaxf(rintf(res[k] / scale), lo), hi);
+      s.code[tok(k) * (D + 4) + j] = (int8_t)fminf(fmaxf(rintf(res[k] / scale), lo), hi);
   }
   if (part == 0) {
     const int f = kGeneral ? h * D + j : kscale_flat(h * D + j), per_slot = C / (NG / kPT);
@@ -369,8 +413,9 @@ __device__ __forceinline__ void encode_values(const AppendKArgs& a, int pg, int 
 // The recipe's page: workgroups [0, 2 h n) encode the residual of one 64-token
 // group of one head, the rest the values of 64 tokens of one head (8 waves x 8
 // tokens).  One launch for both: a commit of one codec page has 16 workgroups
-// of each, and they run side by side.  Measured at h_kv 8: 6.8 us for one codec
-// page at R 32 and 19.7 us for 63 at R 16; the two as kernels of their own, with
+// of each, and they run side by side.  Measured at h_kv 8: 5.8 us for one codec
+// page at R 32 and 18.9 us for 63 at R 16 (6.6 and 19.8 with the residual's
+// product as FMAs); the two as kernels of their own, with
 // both residual operands from LDS and the FWHT's stages through LDS with a
 // barrier each, 21.7 + 7.5 and 27.1 + 27.1 us.
 template <int R>
