@@ -561,13 +561,16 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
         // a row given apart goes into the window buffer (once: by query 0's merge)
         if (r % a.G == 0 && elem(t0, u) < T && fresh_row(a.nw, elem(t0, u)) >= 0)
           *reinterpret_cast<uint2*>(a.nw.v_dst + (vb - a.v_tail) + (int64_t)elem(t0, u) * a.ts_t) = wv[u];
-        const float w = elem(t0, u) < T ? __builtin_amdgcn_exp2f(ws[u] - mnew) : 0.f;
+        // rows at or past T are not the caller's values (they may be NaN or infinite):
+        // select, not weight by 0
+        const bool ok = elem(t0, u) < T;
+        const float w = ok ? __builtin_amdgcn_exp2f(ws[u] - mnew) : 0.f;
         const float4_t vf = a.tail_bf16
             ? float4_t{__uint_as_float(wv[u].x << 16), __uint_as_float(wv[u].x & 0xffff0000u),
                        __uint_as_float(wv[u].y << 16), __uint_as_float(wv[u].y & 0xffff0000u)}
             : float4_t{half_bits_to_float(wv[u].x & 0xffff), half_bits_to_float(wv[u].x >> 16),
                        half_bits_to_float(wv[u].y & 0xffff), half_bits_to_float(wv[u].y >> 16)};
-        xt += w * vf;
+        xt += ok ? w * vf : float4_t{0.f, 0.f, 0.f, 0.f};
         lt += w;
       }
       mt = mnew;
