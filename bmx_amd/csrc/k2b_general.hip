@@ -192,18 +192,19 @@ struct GenBytes {
   }
 };
 
-__device__ __forceinline__ half2_t gen_rtz(float x, float y) {
-  return __builtin_bit_cast(half2_t, __builtin_amdgcn_cvt_pkrtz(x, y));
+__device__ __forceinline__ half2_t gen_half2(float x, float y) {   // one v_cvt_pk_f16_f32: to nearest
+  typedef float f2_t __attribute__((ext_vector_type(2)));
+  return __builtin_convertvector((f2_t{x, y}), half2_t);
 }
 
-// x and y as fp16 high parts (towards zero) and the fp16 low parts that remain
-// (x = h + l to 2^-21).  m1: -1 in a register the compiler cannot see through,
-// so that x - h reads the fp16 h in place (v_fma_mix_f32; exact), with no
-// conversion instruction.
+// x and y as fp16 high parts and the fp16 low parts that remain, both to nearest
+// (x = h + l to 2^-23 where l is normal).  m1: -1 in a register the compiler
+// cannot see through, so that x - h reads the fp16 h in place (v_fma_mix_f32;
+// exact), with no conversion instruction.
 __device__ __forceinline__ void gen_split2(float x, float y, float m1, uint32_t& hi, uint32_t& lo) {
-  const half2_t h = gen_rtz(x, y);
+  const half2_t h = gen_half2(x, y);
   hi = as_u32(h);
-  lo = as_u32(gen_rtz(__builtin_fmaf((float)h[0], m1, x), __builtin_fmaf((float)h[1], m1, y)));
+  lo = as_u32(gen_half2(__builtin_fmaf((float)h[0], m1, x), __builtin_fmaf((float)h[1], m1, y)));
 }
 
 // One 16-token tile of one head's recent window against its G queries, in

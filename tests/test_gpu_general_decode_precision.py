@@ -1,0 +1,57 @@
+"""GPU tests of the general page's decode precision, against float64 attention
+over the pages' dequantized rows.  The RoPE frequencies are 0 (every rotation is
+exactly the identity), so that nothing but the arithmetic of scores, weights and
+sums is between the two."""
+
+import pytest
+import torch
+
+from bmx_amd import k2b, synth
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _pages(k, v, rank, group, bits):
+    """The committed tokens' decode arguments, and their dense keys and values in float64."""
+    h, S, d = k.shape
+    c = k2b.CodecConsts.make(head_dim=d)
+    consts = k2b.CodecConsts(c.codebook, c.sign_bits, (0.0,) * (d // 2), 1.0)
+    pool = synth.PagePool(S // 16, h, rank, DEV, head_dim=d, group=group, k_bits=bits)
+    seq = synth.encode_sequence(pool, k.to(DEV), v.float().to(DEV), rank, consts, svd=synth.first_page_svd(k, rank))
+    K, V = k2b.dequant(pool.pages, torch.tensor(seq.page_ids, dtype=torch.int32, device=DEV), S, seq.basis16, consts,
+                       h_kv=h, rank=rank, group=group, k_bits=bits)
+
+    def decode(q, **kw):
+        return k2b.decode(q[None], pool.pages, synth.page_table([seq], device=DEV),
+                          torch.tensor([S], dtype=torch.int32, device=DEV), S, seq.basis16, consts, d ** -0.5,
+                          rank=rank, group=group, k_bits=bits, **kw)[0].double()
+    return decode, K.double(), V.double()
+
+
+def test_key_parts_are_not_biased():
+    """Packed scores of 500 to 1,000 (base 2) keep their place against window scores of the same size: the share of
+    the packed tokens, read back from the output, gives the packed scores' relative error, here of 2,048 rows.
+    Key parts rounded to nearest err to either side, as the fp32 sums do (deviation of a row 3e-7, of the mean 7e-9;
+    the bound 2^-25 is four of them); parts cut towards zero take up to 2^-21 off every key."""
+    h, G, d, n = 16, 16, 64, 128
+    errs = []
+    for seed in range(8):
+        gen = torch.Generator().manual_seed(seed)
+        k = torch.randn(h, 1, d, generator=gen).half().expand(h, n, d).contiguous()
+        decode, K, V = _pages(k, torch.randn(h, n, d, generator=gen), 16, 32, 3)
+        kt, vt = k.to(DEV)[None], torch.randn(1, h, n, d, generator=gen).half().to(DEV)
+        size = torch.linspace(500, 1000, G, dtype=torch.float64, device=DEV)[None, :, None]
+        q = (K[:, :1] / K[:, :1].square().sum(-1, keepdim=True) * d ** 0.5 / 1.4426950408889634 * size).float()
+        out = decode(q, k_tail=kt, v_tail=vt, tail_len=n, tail_cap=n)
+        s = torch.matmul(q.double(), torch.cat([K, kt[0].double()], 1).transpose(1, 2).contiguous()) * d ** -0.5
+
+        def part(x, val):   # log of the part's weight, its mean value
+            return torch.logsumexp(x, -1), torch.matmul(torch.softmax(x, -1), val)
+        (lp, P), (lw, W) = part(s[..., :n], V), part(s[..., n:], vt[0].double())
+        share = ((out - W) * (P - W)).sum(-1) / (P - W).square().sum(-1)
+        assert share.min() > 0.02 and share.max() < 0.98
+        errs.append((torch.logit(share) - (lp - lw)) / s[..., :n].mean(-1))
+    err = torch.stack(errs)
+    print(f"mean {err.mean().item():.2e}, deviation {err.std().item():.2e}", flush=True)
+    assert abs(err.mean().item()) <= 2 ** -25
