@@ -125,9 +125,18 @@ __device__ __forceinline__ void gen_rope(const GenReadArgs& a, float4_t kt[D / 1
 //     -> lane: score of token 4qd + e for query n
 //   V^T P^T: A = the levels (fp16 high and low parts) of channel n d/16 + ct,
 //     tokens 4qd .. 4qd+3 (one code byte through an LDS table), B = the lane's own
-//     P norm as high and low parts: (lh, lh) against (ph, pl) per page and
-//     (ll, ll') against (ph, ph') per page pair
+//     weight times norm as high and low parts: (lh, lh) against (ph, pl) per page
+//     and (ll, ll') against (ph, ph') per page pair
 //     -> lane: channel (4qd + e) d/16 + ct for query n
+// A low part holds nothing below 2^-25, so weight times norm is not taken
+// relative to the largest weight (as the weights' sum is): with small norms, or
+// with all tokens under a sink, it would lose its bits.  The accumulator has a
+// maximum of its own, a bound of score + log2(norm) -- a lane's largest score plus
+// its largest norm --, and its operand fills fp16's range up to 2^14 of it: what
+// lies up to 2^-24 below the bound keeps 2^-22 of itself.  Both maxima are whole
+// numbers of base-2 scores, so rescaling by them is exact.  Error against float64
+// at norms of 1e-4: 7e-4 with weight times norm relative to the largest weight,
+// 2e-4 with the weight and level times norm as a pair each, 1e-6 now.
 // G queries fill G of the 16 columns; pages are compacted SW columns apart (as
 // k2b_decode_split_kernel does), so the softmax runs once per 16/SW pages.
 //
@@ -139,7 +148,6 @@ __device__ __forceinline__ void gen_rope(const GenReadArgs& a, float4_t kt[D / 1
 // per (split, head) with a page at a time per wave, the rotation remade per head
 // and page (22 of them, f64 included, per RoPE pair) and a merge workgroup per
 // query took 31.6 + 8.5 us, 37.9 us a call.  d 128, rank 64: 92 -> 39 us a call.
-// Kept in 32 bits as before: keys, weights and partial sums (fp16 pairs on MFMA).
 // ---------------------------------------------------------------------------
 struct GenDecodeArgs {
   GenReadArgs r;
@@ -163,6 +171,7 @@ struct GenDecodeArgs {
 };
 
 constexpr int kGenQuad = 4;        // pages a wave takes at a time
+constexpr float kGenUp = 14.f;     // log2 of the largest weight times norm as an operand (fp16's largest is 2^16)
 constexpr int kGenTables = 4;      // RoPE tables (64 positions each) in LDS
 constexpr int kGenIds = 64;        // page ids held per lane vector
 template <int D>
@@ -444,7 +453,8 @@ __global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const G
   float4_t acc[NT];
 #pragma unroll
   for (int ct = 0; ct < NT; ++ct) acc[ct] = float4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;          // l_run: the weights' sum, relative to 2^m_run
+  float z_run = -INFINITY, up = 0.f;             // acc: relative to 2^(z_run - kGenUp); up = 2^(m_run - z_run + kGenUp)
   const int len = __builtin_amdgcn_readfirstlane(min(max(len_raw, 0), a.max_packed_len));
   if (len != a.max_packed_len) {                 // a shorter sequence: its own quads
     set_range(len);
@@ -567,22 +577,33 @@ __global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const G
           for (int i = 0; i < 4; ++i) cr[r][i] = dpp<kRowShr + 8, 0xC>(cr[r][i], st[r * NSLOT + 1][i]);
         }
       }
-      // ---- online softmax (one running max per query, the accumulator rescaled
-      // only when some max grows)
+      // ---- online softmax (two running maxima per query, sums rescaled only when
+      // one of them grows); z_run stays within 64 of m_run where every norm is 0
       float mx = -INFINITY;
+      half4_t vm = vn[0];
 #pragma unroll
-      for (int r = 0; r < NCR; ++r) mx = fmaxf(mx, fmaxf(fmaxf(cr[r][0], cr[r][1]), fmaxf(cr[r][2], cr[r][3])));
-      if (__any(mx > m_run)) {
-        if constexpr (NSLOT == 4) mx = fmaxf(mx, dpp_row<kRowRor + 4>(mx));
-        if constexpr (NSLOT >= 2) mx = fmaxf(mx, dpp_row<kRowRor + 8>(mx));
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m_run, mx);
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        l_run *= alpha;
+      for (int r = 0; r < NCR; ++r) {
+        mx = fmaxf(mx, fmaxf(fmaxf(cr[r][0], cr[r][1]), fmaxf(cr[r][2], cr[r][3])));
+        vm = __builtin_elementwise_max(vm, vn[r]);
+      }
+      const half2_t vm2 = __builtin_elementwise_max(half2_t{vm[0], vm[1]}, half2_t{vm[2], vm[3]});
+      const float mz = mx + __builtin_amdgcn_logf(fmaxf((float)vm2[0], (float)vm2[1]));
+      if (__any(mx > m_run || mz > z_run)) {
+        auto of_query = [](float x) {
+          if constexpr (NSLOT == 4) x = fmaxf(x, dpp_row<kRowRor + 4>(x));
+          if constexpr (NSLOT >= 2) x = fmaxf(x, dpp_row<kRowRor + 8>(x));
+          x = fmaxf(x, __shfl_xor(x, 16));
+          return ceilf(fmaxf(x, __shfl_xor(x, 32)));
+        };
+        const float m_new = fmaxf(m_run, of_query(mx));
+        const float z_new = fmaxf(fmaxf(z_run, of_query(mz)), m_new - 64.f);
+        const float beta = __builtin_amdgcn_exp2f(z_run - z_new);
+        l_run *= __builtin_amdgcn_exp2f(m_run - m_new);
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) acc[ct] *= alpha;
+        for (int ct = 0; ct < NT; ++ct) acc[ct] *= beta;
         m_run = m_new;
+        z_run = z_new;
+        up = __builtin_amdgcn_exp2f(m_run - z_run + kGenUp);
       }
       uint2 ph[NCR], pl[NCR];
 #pragma unroll
@@ -592,7 +613,7 @@ __global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const G
         for (int i = 0; i < 4; ++i) {
           const float p = __builtin_amdgcn_exp2f(cr[r][i] - m_run);
           l_run += p;
-          x[i] = p * (float)vn[r][i];
+          x[i] = p * ((float)vn[r][i] * up);
         }
         gen_split2(x[0], x[1], m1, ph[r].x, pl[r].x);
         gen_split2(x[2], x[3], m1, ph[r].y, pl[r].y);
@@ -677,7 +698,7 @@ __global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const G
       }
   }
   if (n >= G) return;
-  const float inv = l_run > 0.f ? 1.0f / ((float)D * l_run) : 0.f;
+  const float inv = l_run > 0.f ? __builtin_amdgcn_exp2f(z_run - m_run - kGenUp) / ((float)D * l_run) : 0.f;
   const int S = a.n_split * a.wph, slot = split * a.wph + sub;
   const int64_t row = ((int64_t)b * L.h + h) * G + n;
   float* rec = a.ws_acc + row * D * S + slot * 16;   // chunk k at + 16 k S

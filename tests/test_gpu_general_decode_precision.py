@@ -55,3 +55,30 @@ def test_key_parts_are_not_biased():
     err = torch.stack(errs)
     print(f"mean {err.mean().item():.2e}, deviation {err.std().item():.2e}", flush=True)
     assert abs(err.mean().item()) <= 2 ** -25
+
+
+@pytest.mark.parametrize("S,split", [(2048, 0), (4096, 4096)])     # few pages a wave; all of them on one workgroup
+@pytest.mark.parametrize("d,rank,G", [(64, 16, 4), (128, 64, 1), (32, 32, 16)])
+@pytest.mark.parametrize("norm,sink_norm,gap", [
+    (8.0, 8.0, 0), (0.1, 0.1, 0), (1e-2, 1e-2, 0), (1e-4, 1e-4, 0),      # norms of all tokens, no sink
+    (0.16, 0.16, 11), (1e-2, 1e-2, 13), (1e-4, 1e-4, 11),                # all tokens gap nats below the first
+    (8.0, 1e-2, 11), (8.0, 0.0, 13), (1e-2, 100.0, 11), (1e-2, 100.0, -11),
+])
+def test_value_product(norm, sink_norm, gap, d, rank, G, S, split):
+    """The output against float64 where values are small, or where the first token's score stands gap nats above (or
+    below) the others, with a norm of its own.  An operand keeps 2^-22 of itself, a score of up to 30 (base 2) the
+    roundings of its fp32 sum, 4 of 2^-20, and with it the weight (times ln 2): 2.7e-6; the fp32 sums of 4,096 terms,
+    largest first or last, 2^-24 times 64 at most in the mean: 3.8e-6.  Together below 8e-6."""
+    h = 3
+    gen = torch.Generator().manual_seed(S + d)
+    v = torch.randn(h, S, d, generator=gen) * norm / d ** 0.5
+    v[:, 0] *= sink_norm / norm
+    decode, K, V = _pages(synth.k2b_keys(h, S, rank, gen, head_dim=d), v, rank, 32, 3)
+    q = torch.randn(h, G, d, generator=gen).to(DEV)
+    q = (q + K[:, :1] / K[:, :1].square().sum(-1, keepdim=True) * gap * d ** 0.5).float().contiguous()
+    out = decode(q, split_tokens=split)
+    s = torch.matmul(q.double(), K.transpose(1, 2).contiguous()) * d ** -0.5
+    ref = torch.matmul(torch.softmax(s, -1), V)
+    err = ((out - ref).norm() / ref.norm()).item()
+    print(f"error {err:.2e}", flush=True)
+    assert err <= 8e-6
