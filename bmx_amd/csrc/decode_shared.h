@@ -547,6 +547,11 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
   float4_t xt = {0.f, 0.f, 0.f, 0.f};
   for (int t0 = 0; t0 < T; t0 += kTokenPass) {
     if (t0 != 0) load_tokens(t0, T);
+    // a row given apart goes into the window buffer (once: by query 0's merge), whatever its score
+#pragma unroll
+    for (int u = 0; u < kTok; ++u)
+      if (r % a.G == 0 && elem(t0, u) < T && fresh_row(a.nw, elem(t0, u)) >= 0)
+        *reinterpret_cast<uint2*>(a.nw.v_dst + (vb - a.v_tail) + (int64_t)elem(t0, u) * a.ts_t) = wv[u];
     float mloc = -INFINITY;
 #pragma unroll
     for (int u = 0; u < kTok; ++u)
@@ -558,9 +563,6 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
       lt *= sc;
 #pragma unroll
       for (int u = 0; u < kTok; ++u) {
-        // a row given apart goes into the window buffer (once: by query 0's merge)
-        if (r % a.G == 0 && elem(t0, u) < T && fresh_row(a.nw, elem(t0, u)) >= 0)
-          *reinterpret_cast<uint2*>(a.nw.v_dst + (vb - a.v_tail) + (int64_t)elem(t0, u) * a.ts_t) = wv[u];
         // rows at or past T are not the caller's values (they may be NaN or infinite):
         // select, not weight by 0
         const bool ok = elem(t0, u) < T;

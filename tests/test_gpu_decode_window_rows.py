@@ -1,5 +1,6 @@
 """GPU tests of the decode calls' recent window on all three pages (k2b, RTN,
-general): what lies past the window's length in its buffers reaches no output."""
+general): what lies past the window's length in its buffers reaches no output,
+and rows given apart are stored whatever the query holds."""
 
 import pytest
 import torch
@@ -52,3 +53,19 @@ def test_rows_past_the_window_are_not_attended(kind, T, cap, on_device):
     for bad in (float("nan"), float("inf"), float("-inf")):
         kt[:, :, T:], vt[:, :, T:] = bad, bad
         assert torch.equal(decode(q, kt, vt, tail_len=n, tail_cap=cap), want)
+
+
+@pytest.mark.parametrize("T,cap", [(1, 16), (17, 128), (150, 160)])
+@pytest.mark.parametrize("kind", ["k2b", "rtn", "general"])
+def test_rows_given_apart_are_stored_whatever_their_scores(kind, T, cap):
+    """A query row that is not a number has no score above minus infinity; the later rows and calls need the window."""
+    gen = torch.Generator().manual_seed(T)
+    decode, d = _page(kind, gen)
+    kt, vt = (torch.randn(1, H, cap, d, generator=gen).half().to(DEV) for _ in range(2))
+    q = torch.randn(1, H, G, d, generator=gen).to(DEV)
+    q[:, 0, 0] = float("nan")
+    new = tuple(torch.randn(1, H, 1, d, generator=gen).half().to(DEV) for _ in range(2))
+    out = decode(q, kt, vt, tail_len=T, tail_cap=cap, new_kv=new)
+    assert torch.equal(kt[:, :, T - 1:T], new[0]) and torch.equal(vt[:, :, T - 1:T], new[1])
+    want = decode(q, kt, vt, tail_len=T, tail_cap=cap)      # the same rows from the buffers
+    assert torch.equal(out[0, 0, 1:], want[0, 0, 1:]) and torch.equal(out[0, 1], want[0, 1])
