@@ -3,9 +3,8 @@
 // merge kernel that combines the split partials with the window.
 #pragma once
 
-#include <algorithm>
-
 #include "k2b_common.h"
+#include "split_plan.h"
 
 namespace bmx {
 
@@ -298,47 +297,6 @@ __device__ __forceinline__ void score_window(const A& a, float qscale, int b, in
   if (apart ? split < S : wave >= 4) return;
   score_win_pairs(a, qscale, b, apart ? split - S + a.win_wgs * (int)blockIdx.z : split,
                   apart ? a.win_wgs * (int)gridDim.z : S, wave, apart ? waves : 4, n, q);
-}
-
-// The split grid of a call (k2b and RTN): S splits of a sequence, its heads in
-// `blocks` blocks of hpb (grid z), and win_wgs workgroups (grid x, after the
-// splits) that score the window and do nothing else.
-//   S: one workgroup per CU over the batch, or what split_tokens asks for; at
-//     most one per 64-token group.
-//   blocks: a range with few groups leaves CUs idle while the 8 waves of a
-//     workgroup, two per SIMD, share its issue slots; its heads are spread over
-//     2, 4 or 8 workgroups as long as all of them, and the window's, have a CU.
-//   win_wgs: as many as give every (tile, head) pair a wave, 4 pairs a workgroup
-//     where there is room; none where there is not enough: the splits then score
-//     the window after their groups, and, where they are fewer than its tiles,
-//     are as many as those (one per CU at most).
-// Measured, us a call at h_kv 8, G 4 (with neither, and with both): k2b rank 16,
-// 256 tokens and a 60-row window 17.4 -> 12.1 (the query loads together in both:
-// see load_q4); 8,576 tokens, bf16, a 161-row window (no room to spread) 17.7 ->
-// 15.5; RTN 128 tokens 16.9 -> 12.4.
-// Everything follows from the bounds (max_len, tail_cap), not from a call's own
-// window length, so a bound call's workspace fits it at any length.
-struct SplitPlan {
-  int S, blocks, hpb, win_wgs;
-};
-inline SplitPlan plan_splits(int batch, int h_kv, int groups, int max_len, int split_tokens, int tail_cap, int cus) {
-  SplitPlan p;
-  const int per_seq = std::max(1, cus / batch);
-  const int tiles = (tail_cap + 15) / 16, pairs = tiles * h_kv;
-  p.S = split_tokens > 0 ? (max_len + split_tokens - 1) / split_tokens : per_seq;
-  p.S = std::max(1, std::min(p.S, groups));
-  p.blocks = 1;
-  p.win_wgs = 0;
-  if (split_tokens == 0) {
-    while (2 * p.blocks <= h_kv && (int64_t)batch * (2 * p.blocks * (int64_t)p.S + (pairs + 3) / 4) <= cus)
-      p.blocks *= 2;
-    const int spare = per_seq / p.blocks - p.S;
-    p.win_wgs = std::max(0, std::min(spare, (pairs + 4 * p.blocks - 1) / (4 * p.blocks)));
-    if (p.win_wgs * p.blocks * 8 < pairs) p.win_wgs = 0;
-  }
-  if (p.win_wgs == 0 && p.S < tiles) p.S = std::min(tiles, std::max(p.S, per_seq));
-  p.hpb = (h_kv + p.blocks - 1) / p.blocks;
-  return p;
 }
 
 // ---------------------------------------------------------------------------

@@ -81,3 +81,23 @@ def test_bound_call_at_any_window_length(S):
         got = plan.run(tail_len=T, new_kv=new).clone()
         want = k2b.decode(q, pool.pages, None, ln, S, seq.basis16, consts, 128 ** -0.5, tail_len=T, **kw)
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,h,S,T,on_device", [(3, 8, 640, 16, False), (3, 2, 2688, 16, True), (5, 8, 384, 5, True),
+                                               (7, 4, 512, 17, True)])
+def test_rtn_batch_of_spread_heads(B, h, S, T, on_device):
+    """Batches that do not divide the CUs, whose heads the plan may spread: the plain grid's outputs, bit for bit, with
+    lengths and windows shorter than their bounds."""
+    gen = torch.Generator().manual_seed(B)
+    codec = dict(k_bits=4, v_bits=4, k_group=32, v_group=64)
+    k, v = (torch.randn(h, S, 128, generator=gen).half().to(DEV) for _ in range(2))
+    pages = torch.zeros(S // 16, rtn.page_bytes(h, **codec), dtype=torch.uint8, device=DEV)
+    ids = torch.arange(S // 16, dtype=torch.int32, device=DEV)
+    rtn.append(k, v, pages, ids, **codec)
+    kt, vt = (torch.randn(B, h, T, 128, generator=gen).half().to(DEV) for _ in range(2))
+    q = torch.randn(B, h, 4, 128, generator=gen).to(DEV)
+    ln = torch.tensor([S - 128 * (b % 3) for b in range(B)], dtype=torch.int32, device=DEV)
+    n = torch.tensor([T - b % 3 for b in range(B)], dtype=torch.int32, device=DEV) if on_device else T - 1
+    outs = [rtn.decode(q, pages, ids.repeat(B, 1), ln, S, 128 ** -0.5, k_tail=kt, v_tail=vt, tail_len=n, tail_cap=T,
+                       split_tokens=st, **codec) for st in (0, 64)]
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
