@@ -288,15 +288,20 @@ __device__ __forceinline__ void score_win_pairs(const A& a, float qscale, int b,
 
 // The window's pairs of a split kernel's workgroup, at its end: those of the
 // window's own workgroups (split >= S), or, where it has none, dealt over the
-// splits on waves 0-3 (of the two waves of a SIMD, w and w + 4, these end their
-// groups first).  One call for both, so that the kernel holds its code once.
+// splits: on waves 0-3 (of the two waves of a SIMD, w and w + 4, these end their
+// groups first) up to two pairs each, on all waves beyond that.  Four waves for
+// any number: 193 us for an RTN call of 72 sequences with 2,048 tokens and a
+// 1,000-row window (h_kv 8, G 1); eight: 178, and k2b 236 -> 205.  Keeping a head's
+// query between a wave's pairs gave k2b 183 but RTN 183.
+// One call for all, so that the kernel holds its code once.
 template <class A>
 __device__ __forceinline__ void score_window(const A& a, float qscale, int b, int split, int S, int wave, int waves,
                                              int n, int q) {
   const bool apart = a.win_wgs != 0;
-  if (apart ? split < S : wave >= 4) return;
+  const int nw = apart || a.win_tiles * a.h_kv > 8 * S ? waves : 4;
+  if (apart ? split < S : wave >= nw) return;
   score_win_pairs(a, qscale, b, apart ? split - S + a.win_wgs * (int)blockIdx.z : split,
-                  apart ? a.win_wgs * (int)gridDim.z : S, wave, apart ? waves : 4, n, q);
+                  apart ? a.win_wgs * (int)gridDim.z : S, wave, nw, n, q);
 }
 
 // ---------------------------------------------------------------------------

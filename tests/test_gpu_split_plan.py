@@ -101,3 +101,38 @@ def test_rtn_batch_of_spread_heads(B, h, S, T, on_device):
     outs = [rtn.decode(q, pages, ids.repeat(B, 1), ln, S, 128 ** -0.5, k_tail=kt, v_tail=vt, tail_len=n, tail_cap=T,
                        split_tokens=st, **codec) for st in (0, 64)]
     assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+
+
+@pytest.mark.parametrize("T", [48, 49, 300])    # 8 heads x 3, 4 or 19 tiles over 3 splits: 24 pairs is the line
+@pytest.mark.parametrize("page", ["k2b", "rtn"])
+def test_windows_of_more_pairs_than_the_first_waves_take(page, T):
+    """72 sequences (3 splits each) score their windows behind the groups, on 4 waves or on all 8: each sequence's
+    output is that of the sequence alone (other splits; fp16 partial records)."""
+    B, h, G, S = 72, 8, 2, 256
+    gen = torch.Generator().manual_seed(T)
+    kt, vt = (torch.randn(B, h, T, 128, generator=gen).half().to(DEV) for _ in range(2))
+    q = torch.randn(B, h, G, 128, generator=gen).to(DEV)
+    ln = torch.full((B,), S, dtype=torch.int32, device=DEV)
+    if page == "k2b":
+        consts = k2b.CodecConsts.make()
+        pool = synth.PagePool(S // 16, h, 16, DEV)
+        seq = synth.encode_sequence(pool, synth.k2b_keys(h, S, 16, gen).to(DEV), synth.values(h, S, gen).to(DEV), 16,
+                                    consts)
+
+        def decode(s):
+            return k2b.decode(q[s], pool.pages, synth.page_table([seq] * len(q[s]), device=DEV), ln[s], S, seq.basis16,
+                              consts, 128 ** -0.5, rank=16, k_tail=kt[s], v_tail=vt[s], tail_len=T, tail_cap=T)
+    else:
+        codec = dict(k_bits=4, v_bits=4, k_group=32, v_group=64)
+        k, v = (torch.randn(h, S, 128, generator=gen).half().to(DEV) for _ in range(2))
+        pages = torch.zeros(S // 16, rtn.page_bytes(h, **codec), dtype=torch.uint8, device=DEV)
+        ids = torch.arange(S // 16, dtype=torch.int32, device=DEV)
+        rtn.append(k, v, pages, ids, **codec)
+
+        def decode(s):
+            return rtn.decode(q[s], pages, ids.repeat(len(q[s]), 1), ln[s], S, 128 ** -0.5, k_tail=kt[s], v_tail=vt[s],
+                              tail_len=T, tail_cap=T, **codec)
+    out = decode(slice(0, B))
+    for b in (0, 35, 71):
+        alone = decode(slice(b, b + 1))[0]
+        assert (out[b] - alone).abs().max().item() <= 2 ** -10 * alone.abs().max().item()
