@@ -802,13 +802,15 @@ void fill_read(GenReadArgs& r, const Geo& g) {
 
 // The decode grid of a sequence: n_split workgroups (its 4-page quads dealt
 // evenly) x head blocks of hpb heads, wph waves per head.  One workgroup per CU
-// over the batch; a wave per head, or several where there are fewer heads than
-// waves, each with its own partial slot.  A range with fewer quads than CUs
-// spreads its heads over more blocks (a wave alone on its SIMD takes a quad in
-// about half the time), and where CUs are still idle the window's tiles get
-// workgroups of their own (d 64, 2,048 tokens and a 128-row window: 17.1 us a call
-// with neither, 15.8 with the window apart, 12.6 with both).  The sequences are launched `chunk` at
-// a time, so that the workspace stays within kGenWorkspace whatever the batch.
+// over the batch, or as many as split_tokens asks for; a wave per head, or several
+// where there are fewer heads than waves, each with its own partial slot.  A range
+// of fewer splits than CUs spreads its heads over more blocks (a wave alone on its
+// SIMD takes a quad in about half the time), and where CUs are still idle the
+// window's tiles get workgroups of their own (d 64, 2,048 tokens and a 128-row
+// window: 17.1 us a call with neither, 15.8 with the window apart, 12.6 with both).
+// With split_tokens 512 and the heads of 2,048 tokens (d 64, rank 32, h_kv 8, G 4) on
+// one workgroup a split 48.9 us, spread 19.5.  The sequences are launched `chunk`
+// at a time, so that the workspace stays within kGenWorkspace whatever the batch.
 constexpr size_t kGenWorkspace = 24u << 20;   // one sequence takes at most 21.5 MB (16 heads x 16 queries, d 128)
 
 struct GenPlan {
@@ -821,22 +823,25 @@ GenPlan gen_plan(const bmx_k2b_decode_args* a, const Geo& g) {
   GenPlan p;
   const int nw = gen_waves(g.d, g.R), cus = bmx_device_cu_count();
   const int quads = std::max(1, (a->max_packed_len / kPT + kGenQuad - 1) / kGenQuad);
-  const int win_pairs = (a->tail_cap + 15) / 16 * g.h;   // the bound: a bound call's plan holds at any length
+  // at most so many splits (with split_tokens: exactly)
+  const int most = a->split_tokens > 0
+                       ? std::max(1, std::min(quads, (a->max_packed_len + a->split_tokens - 1) / a->split_tokens))
+                       : quads;
+  // the window's bound: a bound call's plan holds at any length
+  const int pairs = (a->tail_cap + 15) / 16 * g.h;
   p.chunk = a->batch;
   for (;; p.chunk = (p.chunk + 1) / 2) {
     p.blocks = (g.h + nw - 1) / nw;
-    while (a->split_tokens == 0 && 2 * p.blocks <= g.h &&
-           (int64_t)p.chunk * (2 * p.blocks * (int64_t)quads + (win_pairs + 3) / 4) <= cus)
+    const int win_most = a->split_tokens > 0 ? 0 : (pairs + 3) / 4;   // room kept for the window
+    while (2 * p.blocks <= g.h && (int64_t)p.chunk * (2 * p.blocks * (int64_t)most + win_most) <= cus)
       p.blocks *= 2;
     p.hpb = (g.h + p.blocks - 1) / p.blocks;
     const int per_seq = cus / (p.chunk * p.blocks);
-    p.n_split = a->split_tokens > 0 ? (a->max_packed_len + a->split_tokens - 1) / a->split_tokens : per_seq;
-    p.n_split = std::max(1, std::min(p.n_split, quads));
+    p.n_split = a->split_tokens > 0 ? most : std::max(1, std::min(per_seq, most));
     p.wph = std::max(1, std::min(nw / p.hpb, (quads + p.n_split - 1) / p.n_split));
     // as many as give every (tile, head) pair a wave, 4 pairs a workgroup if there is room, else none
-    const int spare = a->split_tokens > 0 ? 0 : per_seq - p.n_split;
-    p.win_wgs = std::min(spare, (win_pairs + 4 * p.blocks - 1) / (4 * p.blocks));
-    if (p.win_wgs * p.blocks * nw < win_pairs) p.win_wgs = 0;
+    p.win_wgs = std::max(0, std::min(per_seq - p.n_split, (pairs + 4 * p.blocks - 1) / (4 * p.blocks)));
+    if (p.win_wgs * p.blocks * nw < pairs) p.win_wgs = 0;
     p.bytes = (size_t)p.chunk * g.h * g.G * ((size_t)p.slots() * (g.d + 2) + a->tail_cap) * sizeof(float);
     if (p.chunk == 1 || p.bytes <= kGenWorkspace) return p;
   }
