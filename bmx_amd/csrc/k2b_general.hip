@@ -810,8 +810,10 @@ void fill_read(GenReadArgs& r, const Geo& g) {
 // window: 17.1 us a call with neither, 15.8 with the window apart, 12.6 with both).
 // With split_tokens 512 and the heads of 2,048 tokens (d 64, rank 32, h_kv 8, G 4) on
 // one workgroup a split 48.9 us, spread 19.5.  The sequences are launched `chunk`
-// at a time, so that the workspace stays within kGenWorkspace whatever the batch.
-constexpr size_t kGenWorkspace = 24u << 20;   // one sequence takes at most 21.5 MB (16 heads x 16 queries, d 128)
+// at a time, so that the workspace stays within kGenWorkspace whatever the batch;
+// one sequence needs 12.8 MB at most (16 heads x 16 queries, d 128, a 4,096-row
+// window), unless split_tokens asks for more splits than fit: it gets those that do.
+constexpr size_t kGenWorkspace = 24u << 20;
 
 struct GenPlan {
   int chunk, n_split, hpb, blocks, wph, win_wgs;
@@ -839,6 +841,13 @@ GenPlan gen_plan(const bmx_k2b_decode_args* a, const Geo& g) {
     const int per_seq = cus / (p.chunk * p.blocks);
     p.n_split = a->split_tokens > 0 ? most : std::max(1, std::min(per_seq, most));
     p.wph = std::max(1, std::min(nw / p.hpb, (quads + p.n_split - 1) / p.n_split));
+    if (p.chunk == 1) {
+      const int fit = ((int)(kGenWorkspace / (sizeof(float) * g.h * g.G)) - a->tail_cap) / (g.d + 2);   // >= 157
+      if (p.slots() > fit) {
+        p.wph = 1;
+        p.n_split = std::min(p.n_split, fit);
+      }
+    }
     // as many as give every (tile, head) pair a wave, 4 pairs a workgroup if there is room, else none
     p.win_wgs = std::max(0, std::min(per_seq - p.n_split, (pairs + 4 * p.blocks - 1) / (4 * p.blocks)));
     if (p.win_wgs * p.blocks * nw < pairs) p.win_wgs = 0;

@@ -168,7 +168,8 @@ typedef struct {
                                  to the sequences' device lengths (the workspace then
                                  holds CU count - batch + 1 partial slots per row);
                                  > 0 (multiple of 64) = about max_packed_len / split_tokens
-                                 workgroups per sequence.  Packed tokens are dealt in
+                                 workgroups per sequence (general page: and head block,
+                                 no more than 24 MiB of partials hold).  Packed tokens are dealt in
                                  64-token groups, balanced over the workgroups; the
                                  recent window is scored by the split kernel in
                                  16-token tiles (at least one workgroup per tile, up

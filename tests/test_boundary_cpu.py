@@ -183,3 +183,23 @@ def test_product_inv_freq_matches_hf_config():
     inv, scale = K.rope_inv_freq(cfg)
     inv0, scale0 = K.rope_inv_freq(head_dim=128, theta=500000.0)
     assert torch.equal(inv, inv0) and scale == scale0 == 1.0
+
+
+def test_general_page_workspace_is_bounded():
+    """Every decode call on the general page, whatever its splits, window and batch, stays within 24 MiB, below the
+    allocation-free call's scratch, and keeps a partial record for every (row, split) it is granted."""
+    L = _lib.lib()
+    a = _lib.DecodeArgs()
+    most = 0
+    for h, d, rank in ((1, 32, 16), (2, 64, 16), (3, 128, 64), (8, 32, 32), (16, 64, 128), (16, 128, 16)):
+        for G in (1, 4, 16):
+            a.geom = _lib.Geom(h, rank, G, d, 32, 3)
+            for length in (128, 2048, 1 << 17, 900 * 1024, 1 << 20):
+                for split in (0, 64, 256, 512, 4096, 65536):
+                    for tail in (0, 255, 4096):
+                        for batch in (1, 2, 7, 64):
+                            a.batch, a.max_packed_len, a.split_tokens, a.tail_cap = batch, length, split, tail
+                            n = L.bmx_k2b_decode_workspace_bytes(ct.byref(a))
+                            assert h * G * (d + 2 + tail) * 4 <= n <= 24 << 20, (h, d, G, length, split, tail, batch)
+                            most = max(most, n)
+    assert most > 20 << 20

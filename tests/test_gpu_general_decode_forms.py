@@ -119,3 +119,24 @@ def test_decode_batch_served_in_parts():
         alone = k2b.decode(q[s], pool.pages, table[s], lens[s], S, seq.basis16, consts, d ** -0.5, k_tail=one_k[s],
                            v_tail=one_v[s], tail_len=T, new_kv=(new[0][s], new[1][s]), **kw)
         assert (out[s] - alone).abs().max().item() <= 2e-6
+
+
+def test_decode_with_more_splits_than_the_workspace_holds():
+    """256 splits of 16 heads x 16 queries with room for 157: the call without split_tokens, to fp32 summation."""
+    h, d, rank, group, bits, G, S, cap = 16, 128, 16, 16, 2, 16, 16384, 4096
+    gen = torch.Generator().manual_seed(9)
+    consts = k2b.CodecConsts.make(head_dim=d)
+    pages = torch.randint(0, 256, (S // 16, k2b.page_bytes(h, rank, head_dim=d, group=group, k_bits=bits)),
+                          generator=gen, dtype=torch.uint8).to(DEV)
+    k = torch.randn(h, S, d, generator=gen).half().to(DEV)
+    basis = torch.linalg.qr(torch.randn(h * d, rank, generator=gen))[0].contiguous().to(DEV)
+    ids = torch.arange(S // 16, dtype=torch.int32, device=DEV)
+    k2b.append(k, k.flip(1), basis, basis.half(), pages, ids, consts, rank=rank, group=group, k_bits=bits)
+    kt, vt = (torch.randn(1, h, cap, d, generator=gen).half().to(DEV) for _ in range(2))
+    q = torch.randn(1, h, G, d, generator=gen).to(DEV)
+    ws = k2b.DecodeWorkspace()
+    outs = [k2b.decode(q, pages, ids[None], torch.tensor([S], dtype=torch.int32, device=DEV), S, basis.half(), consts,
+                       d ** -0.5, rank=rank, k_tail=kt, v_tail=vt, tail_len=77, tail_cap=cap, group=group, k_bits=bits,
+                       split_tokens=st, workspace=ws) for st in (0, 64)]
+    assert ws.buf.numel() <= 24 << 20
+    assert (outs[0] - outs[1]).abs().max().item() <= 2e-6
