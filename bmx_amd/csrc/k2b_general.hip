@@ -216,54 +216,92 @@ __device__ __forceinline__ void gen_split2(float x, float y, float m1, uint32_t&
   lo = as_u32(gen_half2(__builtin_fmaf((float)h[0], m1, x), __builtin_fmaf((float)h[1], m1, y)));
 }
 
-// One 16-token tile of one head's recent window against its G queries, in
-// fp32: lane (token n, channel quarter qd).  Rows given apart are also stored
-// into the window buffer.
+// One 16-token tile of one head's recent window against its G queries: S^T = K Q^T
+// on MFMA (A: token n, channels 32c + 8qd ..; B: query n, the same channels; the
+// lane gets tokens 4qd + e of query n).  The query row is scaled by a power of two
+// so that its largest element is 2^13 .. 2^14, and split into rounded parts that
+// carry it to fp32: two of fp16, or three of bf16 for a bf16 window; the sums are
+// fp32, the later parts' apart, and scaled back: an output's error against float64
+// 3e-7, 6e-7 with fp32 products.  Rows given apart are also stored into the window buffer.
+// Bound: one load round trip, whatever G is.  Products on the VALU took the queries
+// 2 or 4 at a time, a round trip each, at one or two waves a SIMD: 40 sequences of
+// 128 tokens and 128 window rows, G 16: 16 heads, d 64, rank 128 150.4 -> 124.2 us a
+// call, 8 heads, d 32, rank 16 51.5 -> 33.5.  Loading a wave's next tile ahead: the
+// same to 2 %.
 template <int D>
 __device__ __forceinline__ void gen_window_tile(const GenDecodeArgs& a, int b, int h, int j, int n, int qd) {
-  constexpr int NQ = D / 16;   // 4-channel pieces of the lane's quarter
-  const int H = a.r.L.h, t = 16 * j + n, i_new = fresh_row(a.nw, t);
+  constexpr int NP = D / 16;   // 4-channel pieces of a lane: two of each 32 channels
+  auto at = [](int k) { return 32 * (k >> 1) + 4 * (k & 1); };
+  const int t = 16 * j + n, i_new = fresh_row(a.nw, t);
   const int64_t tb = (int64_t)b * a.ts_b + (int64_t)h * a.ts_h;
   const uint16_t* row = (i_new >= 0 ? a.nw.k + (int64_t)b * a.nw.sb + (int64_t)h * a.nw.sh + (int64_t)i_new * a.nw.st
-                                    : a.k_tail + tb + (int64_t)(t < a.tail_cap ? t : 0) * a.ts_t) + qd * (D / 4);
-  uint2 kv[NQ];
+                                    : a.k_tail + tb + (int64_t)(t < a.tail_cap ? t : 0) * a.ts_t) + 8 * qd;
+  uint2 kw[NP];
 #pragma unroll
-  for (int c = 0; c < NQ; ++c) kv[c] = *reinterpret_cast<const uint2*>(row + 4 * c);
-  const bool bf = __builtin_amdgcn_readfirstlane(a.tail_bf16) != 0;
-  const int64_t r0 = ((int64_t)b * H + h) * a.G;
-  constexpr int GB = D == 128 ? 2 : 4;   // queries whose loads are in flight with the tile's
-  RawQ4 qr[GB * NQ];
-  auto load_q = [&](int g0) {
-    load_q4(a.q, a.io_dtype,
-            [&](int k) { return (r0 + min(g0 + k / NQ, a.G - 1)) * D + qd * (D / 4) + 4 * (k % NQ); }, qr);
-  };
-  load_q(0);
+  for (int k = 0; k < NP; ++k) kw[k] = *reinterpret_cast<const uint2*>(row + at(k));
+  const int64_t r0 = ((int64_t)b * a.r.L.h + h) * a.G, q0 = (r0 + (n < a.G ? n : 0)) * D + 8 * qd;
+  RawQ4 qr[NP];
+  load_q4(a.q, a.io_dtype, [&](int k) { return q0 + at(k); }, qr);
   if (i_new >= 0) {
-    uint16_t* dst = a.nw.k_dst + tb + (int64_t)t * a.ts_t + qd * (D / 4);
+    uint16_t* dst = a.nw.k_dst + tb + (int64_t)t * a.ts_t + 8 * qd;
 #pragma unroll
-    for (int c = 0; c < NQ; ++c) *reinterpret_cast<uint2*>(dst + 4 * c) = kv[c];
+    for (int k = 0; k < NP; ++k) *reinterpret_cast<uint2*>(dst + at(k)) = kw[k];
   }
-  for (int g0 = 0; g0 < a.G; g0 += GB) {
-    if (g0 > 0) load_q(g0);
-    float4_t qv[GB * NQ];
-    cvt_q4(qr, a.io_dtype, qv);
+  float4_t x[NP];
+  cvt_q4(qr, a.io_dtype, x);
+  const float sc = n < a.G ? a.qscale : 0.f;
+  float mx = 0.f;
 #pragma unroll
-    for (int i = 0; i < GB; ++i) {
-      float s = 0.f;
+  for (int k = 0; k < NP; ++k)
 #pragma unroll
-      for (int c = 0; c < NQ; ++c) {
-        const uint2 r = kv[c];
-        const float4_t x = bf ? float4_t{__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u),
-                                         __uint_as_float(r.y << 16), __uint_as_float(r.y & 0xffff0000u)}
-                              : float4_t{half_bits_to_float(r.x & 0xffff), half_bits_to_float(r.x >> 16),
-                                         half_bits_to_float(r.y & 0xffff), half_bits_to_float(r.y >> 16)};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s = __builtin_fmaf(qv[i * NQ + c][e] * a.qscale, x[e], s);
-      }
-      s += __shfl_xor(s, 16);
-      s += __shfl_xor(s, 32);
-      if (qd == 0 && t < a.tail_cap && g0 + i < a.G) a.ws_win[(r0 + g0 + i) * a.tail_cap + t] = s;
+    for (int e = 0; e < 4; ++e) {
+      x[k][e] *= sc;
+      mx = fmaxf(mx, fabsf(x[k][e]));
     }
+  mx = fmaxf(mx, __shfl_xor(mx, 16));
+  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  const int up = 14 - __builtin_amdgcn_frexp_expf(mx);
+  const bool bf = __builtin_amdgcn_readfirstlane(a.tail_bf16) != 0;
+  float4_t s = {0.f, 0.f, 0.f, 0.f}, low = s;   // sums of the first parts, of the later ones
+#pragma unroll
+  for (int c = 0; c < NP / 2; ++c) {
+    union { uint2 u[2]; half8_t h; bf16x8_t v; } kk = {{kw[2 * c], kw[2 * c + 1]}};
+    float r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = __builtin_amdgcn_ldexpf(x[2 * c + (i >> 2)][i & 3], up);
+    if (bf) {
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+        union { uint16_t w[8]; bf16x8_t v; } q;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t w = bf16_bits(r[i]);
+          q.w[i] = (uint16_t)w;
+          r[i] -= __uint_as_float(w << 16);
+        }
+        float4_t& sum = part ? low : s;
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kk.v, q.v, sum, 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int part = 0; part < 2; ++part) {
+        half8_t q;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          q[i] = (_Float16)r[i];
+          r[i] -= (float)q[i];
+        }
+        float4_t& sum = part ? low : s;
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk.h, q, sum, 0, 0, 0);
+      }
+    }
+  }
+  s += low;
+  if (n < a.G) {
+    float* dst = a.ws_win + (r0 + n) * a.tail_cap;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (16 * j + 4 * qd + e < a.tail_cap) dst[16 * j + 4 * qd + e] = __builtin_amdgcn_ldexpf(s[e], -up);
   }
 }
 
@@ -296,15 +334,15 @@ __global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const G
   // the window's (16-token tile, head) pairs, dealt over workgroups and waves:
   // over the sequence's own workgroups at their end, or over win_wgs more that do
   // nothing else
-  auto window_pairs = [&](int wg, int n) {
-    const int n_wg = n * gridDim.y, n_pairs = a.win_tiles * L.h;
-    for (int p = wg + n * blockIdx.y + wave * n_wg; p < n_pairs; p += NWV * n_wg) {
+  auto window = [&](int wg, int n_x) {
+    const int n_wg = n_x * gridDim.y, n_pairs = a.win_tiles * L.h;
+    for (int p = wg + n_x * blockIdx.y + wave * n_wg; p < n_pairs; p += NWV * n_wg) {
       const int j = p / L.h;
-      gen_window_tile<D>(a, b, p - j * L.h, j, lane & 15, qd);
+      gen_window_tile<D>(a, b, p - j * L.h, j, n, qd);
     }
   };
   if (split >= a.n_split) {
-    window_pairs(split - a.n_split, a.win_wgs);
+    window(split - a.n_split, a.win_wgs);
     return;
   }
   const float freq = a.r.inv_freq[tid & (D / 2 - 1)];   // the RoPE frequency this thread makes table entries of
@@ -649,7 +687,7 @@ __global__ __launch_bounds__(64 * gen_waves(D, R)) void gen_split_kernel(const G
     }
   }
 
-  if (a.win_wgs == 0) window_pairs(split, a.n_split);
+  if (a.win_wgs == 0) window(split, a.n_split);
   if (!active) return;
   // ---- fold the page slots, then the inverse Hadamard of channel
   // (4qd + e) NT + ct: ct and e in registers, qd across the rows; signs, 1/d
@@ -806,8 +844,10 @@ void fill_read(GenReadArgs& r, const Geo& g) {
 // where there are fewer heads than waves, each with its own partial slot.  A range
 // of fewer splits than CUs spreads its heads over more blocks (a wave alone on its
 // SIMD takes a quad in about half the time), and where CUs are still idle the
-// window's tiles get workgroups of their own (d 64, 2,048 tokens and a 128-row
-// window: 17.1 us a call with neither, 15.8 with the window apart, 12.6 with both).
+// window's pairs get workgroups of their own (d 64, 2,048 tokens and a 128-row
+// window: 17.1 us a call with neither, 15.8 with the window apart, 12.6 with both),
+// 4 pairs each if there is room, unless a wave would have more of them there than
+// behind the quads.
 // With split_tokens 512 and the heads of 2,048 tokens (d 64, rank 32, h_kv 8, G 4) on
 // one workgroup a split 48.9 us, spread 19.5.  The sequences are launched `chunk`
 // at a time, so that the workspace stays within kGenWorkspace whatever the batch;
@@ -834,7 +874,7 @@ GenPlan gen_plan(const bmx_k2b_decode_args* a, const Geo& g) {
   p.chunk = a->batch;
   for (;; p.chunk = (p.chunk + 1) / 2) {
     p.blocks = (g.h + nw - 1) / nw;
-    const int win_most = a->split_tokens > 0 ? 0 : (pairs + 3) / 4;   // room kept for the window
+    const int win_most = a->split_tokens > 0 ? 0 : (pairs + nw - 1) / nw;   // room kept for the window
     while (2 * p.blocks <= g.h && (int64_t)p.chunk * (2 * p.blocks * (int64_t)most + win_most) <= cus)
       p.blocks *= 2;
     p.hpb = (g.h + p.blocks - 1) / p.blocks;
@@ -848,9 +888,9 @@ GenPlan gen_plan(const bmx_k2b_decode_args* a, const Geo& g) {
         p.n_split = std::min(p.n_split, fit);
       }
     }
-    // as many as give every (tile, head) pair a wave, 4 pairs a workgroup if there is room, else none
     p.win_wgs = std::max(0, std::min(per_seq - p.n_split, (pairs + 4 * p.blocks - 1) / (4 * p.blocks)));
-    if (p.win_wgs * p.blocks * nw < pairs) p.win_wgs = 0;
+    auto rounds = [&](int wgs) { return (pairs + wgs * p.blocks * nw - 1) / (wgs * p.blocks * nw); };
+    if (p.win_wgs > 0 && rounds(p.win_wgs) > rounds(p.n_split)) p.win_wgs = 0;
     p.bytes = (size_t)p.chunk * g.h * g.G * ((size_t)p.slots() * (g.d + 2) + a->tail_cap) * sizeof(float);
     if (p.chunk == 1 || p.bytes <= kGenWorkspace) return p;
   }

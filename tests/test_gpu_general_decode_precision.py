@@ -22,9 +22,9 @@ def _pages(k, v, rank, group, bits):
     K, V = k2b.dequant(pool.pages, torch.tensor(seq.page_ids, dtype=torch.int32, device=DEV), S, seq.basis16, consts,
                        h_kv=h, rank=rank, group=group, k_bits=bits)
 
-    def decode(q, **kw):
+    def decode(q, n=S, **kw):
         return k2b.decode(q[None], pool.pages, synth.page_table([seq], device=DEV),
-                          torch.tensor([S], dtype=torch.int32, device=DEV), S, seq.basis16, consts, d ** -0.5,
+                          torch.tensor([n], dtype=torch.int32, device=DEV), S, seq.basis16, consts, d ** -0.5,
                           rank=rank, group=group, k_bits=bits, **kw)[0].double()
     return decode, K.double(), V.double()
 
@@ -81,4 +81,26 @@ def test_value_product(norm, sink_norm, gap, d, rank, G, S, split):
     ref = torch.matmul(torch.softmax(s, -1), V)
     err = ((out - ref).norm() / ref.norm()).item()
     print(f"error {err:.2e}", flush=True)
+    assert err <= 8e-6
+
+
+@pytest.mark.parametrize("size", [1.0, 2.0 ** -12, 2.0 ** 9])     # of the window's keys; the query is 1 / size
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,rank,G", [(64, 16, 4), (128, 64, 1), (32, 32, 16)])
+def test_window_scores(d, rank, G, dtype, size):
+    """Window scores carry the fp32 query: a window alone against float64, scores of up to 30 (base 2), the query far
+    below and above 1 and its elements over 2^10 (the bound is test_value_product's, for the same kind of sums)."""
+    h, T = 3, 100
+    gen = torch.Generator().manual_seed(d)
+    decode, _, _ = _pages(synth.k2b_keys(h, 128, rank, gen, head_dim=d), torch.randn(h, 128, d, generator=gen), rank,
+                          32, 3)
+    ramp = torch.logspace(-5, 5, d, base=2.0)
+    kt = (torch.randn(1, h, T, d, generator=gen) / ramp * size).to(dtype).to(DEV)
+    vt = torch.randn(1, h, T, d, generator=gen).to(dtype).to(DEV)
+    q = (torch.randn(h, G, d, generator=gen) * ramp / size * 5).to(DEV)
+    out = decode(q, n=0, k_tail=kt, v_tail=vt, tail_len=T, tail_cap=T)
+    s = torch.matmul(q.double(), kt[0].double().transpose(1, 2).contiguous()) * d ** -0.5
+    ref = torch.matmul(torch.softmax(s, -1), vt[0].double())
+    err = ((out - ref).norm() / ref.norm()).item()
+    print(f"error {err:.2e}, scores to {s.abs().max().item() * 1.4427:.0f}", flush=True)
     assert err <= 8e-6
