@@ -510,11 +510,6 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
   float4_t xt = {0.f, 0.f, 0.f, 0.f};
   for (int t0 = 0; t0 < T; t0 += kTokenPass) {
     if (t0 != 0) load_tokens(t0, T);
-    // a row given apart goes into the window buffer (once: by query 0's merge), whatever its score
-#pragma unroll
-    for (int u = 0; u < kTok; ++u)
-      if (r % a.G == 0 && elem(t0, u) < T && fresh_row(a.nw, elem(t0, u)) >= 0)
-        *reinterpret_cast<uint2*>(a.nw.v_dst + (vb - a.v_tail) + (int64_t)elem(t0, u) * a.ts_t) = wv[u];
     float mloc = -INFINITY;
 #pragma unroll
     for (int u = 0; u < kTok; ++u)
@@ -527,18 +522,26 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
 #pragma unroll
       for (int u = 0; u < kTok; ++u) {
         // rows at or past T are not the caller's values (they may be NaN or infinite):
-        // select, not weight by 0
+        // zeros in their place, not only the weight 0
         const bool ok = elem(t0, u) < T;
         const float w = ok ? __builtin_amdgcn_exp2f(ws[u] - mnew) : 0.f;
+        const uint2 v = ok ? wv[u] : make_uint2(0u, 0u);
         const float4_t vf = a.tail_bf16
-            ? float4_t{__uint_as_float(wv[u].x << 16), __uint_as_float(wv[u].x & 0xffff0000u),
-                       __uint_as_float(wv[u].y << 16), __uint_as_float(wv[u].y & 0xffff0000u)}
-            : float4_t{half_bits_to_float(wv[u].x & 0xffff), half_bits_to_float(wv[u].x >> 16),
-                       half_bits_to_float(wv[u].y & 0xffff), half_bits_to_float(wv[u].y >> 16)};
-        xt += ok ? w * vf : float4_t{0.f, 0.f, 0.f, 0.f};
+            ? float4_t{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u),
+                       __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)}
+            : float4_t{half_bits_to_float(v.x & 0xffff), half_bits_to_float(v.x >> 16),
+                       half_bits_to_float(v.y & 0xffff), half_bits_to_float(v.y >> 16)};
+        xt += w * vf;
         lt += w;
       }
       mt = mnew;
+    }
+    // a row given apart goes into the window buffer (once: by query 0's merge), whatever its score
+    if (a.nw.n > 0 && r == h * a.G) {
+#pragma unroll
+      for (int u = 0; u < kTok; ++u)
+        if (elem(t0, u) < T && fresh_row(a.nw, elem(t0, u)) >= 0)
+          *reinterpret_cast<uint2*>(a.nw.v_dst + (vb - a.v_tail) + (int64_t)elem(t0, u) * a.ts_t) = wv[u];
     }
   }
   // ---- row sums (every row holds all of the wave's splits and tokens, for
