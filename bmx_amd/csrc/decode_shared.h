@@ -420,8 +420,9 @@ __device__ __forceinline__ float part_weight(float mi, float M) {
 // so that the window is one pass, one memory round trip.
 // kDim: head_dim; Rec: the records' element (uint16_t: fp16 bits; float: the
 // general page's fp32 records, whose empty attention -- no token at all -- is 0).
-template <bool kRotated, int kTok, int kDim = kD, class Rec = uint16_t>
-__global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs a) {
+// kWaves: waves of a workgroup.
+template <bool kRotated, int kTok, int kDim = kD, class Rec = uint16_t, int kWaves = kCmbWaves>
+__global__ __launch_bounds__(64 * kWaves) void combine_kernel(const CombineKArgs a) {
   const int ch = blockIdx.x, r = blockIdx.y, b = blockIdx.z;
   const int h = r / a.G;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, p = lane & 15, c4 = lane >> 4;
@@ -433,10 +434,10 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
   const uint16_t* vb = a.v_tail + b * a.ts_b + h * a.ts_h + kChunk * ch + 4 * c4;
   const int64_t new_base = b * a.nw.sb + h * a.nw.sh + kChunk * ch + 4 * c4;
   typedef float f2_t __attribute__((ext_vector_type(2)));
-  // element e of this lane in pass j0: p + 16 (wave + kCmbWaves u) + j0
-  auto elem = [&](int j0, int u) { return j0 + p + 16 * (wave + kCmbWaves * u); };
-  constexpr int kSplitPass = 16 * kCmbWaves * kCmbSplits;   // splits per pass of the workgroup
-  constexpr int kTokenPass = 16 * kCmbWaves * kTok;   // window tokens per pass
+  // element e of this lane in pass j0: p + 16 (wave + kWaves u) + j0
+  auto elem = [&](int j0, int u) { return j0 + p + 16 * (wave + kWaves * u); };
+  constexpr int kSplitPass = 16 * kWaves * kCmbSplits;   // splits per pass of the workgroup
+  constexpr int kTokenPass = 16 * kWaves * kTok;   // window tokens per pass
 
   f2_t ml[kCmbSplits];
   float4_t pv[kCmbSplits];
@@ -547,8 +548,8 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
   // ---- row sums (every row holds all of the wave's splits and tokens, for
   // its 4 channels), then the waves meet in LDS: per wave (mp, lp, mt, lt)
   // and the 16 channels' packed and window sums ----
-  __shared__ float s_m[kCmbWaves][4];
-  __shared__ float4_t s_y[kCmbWaves][4], s_z[kCmbWaves][4];
+  __shared__ float s_m[kWaves][4];
+  __shared__ float4_t s_y[kWaves][4], s_z[kWaves][4];
   float4_t y, z;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -571,14 +572,14 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
   if (wave != 0) return;
   float Mp = -INFINITY, Mt = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < kCmbWaves; ++w) {
+  for (int w = 0; w < kWaves; ++w) {
     Mp = fmaxf(Mp, s_m[w][0]);
     Mt = fmaxf(Mt, s_m[w][2]);
   }
   lp = lt = 0.f;
   y = z = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int w = 0; w < kCmbWaves; ++w) {
+  for (int w = 0; w < kWaves; ++w) {
     const float wp = part_weight(s_m[w][0], Mp), wt = part_weight(s_m[w][2], Mt);
     lp = __builtin_fmaf(wp, s_m[w][1], lp);
     lt = __builtin_fmaf(wt, s_m[w][3], lt);
@@ -622,11 +623,21 @@ __global__ __launch_bounds__(kCmbThreads) void combine_kernel(const CombineKArgs
   }
 }
 
-// The merge launch: the window in one pass when it holds more than 128 rows.
+// The merge launch: the window in one pass when it holds more than 128 rows.  On
+// the general page with one wave a workgroup where there are more than 4 workgroups
+// a CU and at most 64 splits (one pass of one wave): the chip is full without the
+// other waves, which would have a share of the window at most.  40 sequences of 128
+// tokens, G 16, h_kv 16, d 32, rank 32: 51.0 us a call with 4 waves, 28.8 with one (a
+// window of 20 rows); 58.2 and 42.5 (128 rows).
 template <bool kRotated, int kDim = kD, class Rec = uint16_t>
 inline void launch_combine(const CombineKArgs& c, int rows, int batch, hipStream_t st) {
+  constexpr bool general = sizeof(Rec) == 4;
   const dim3 grid(kDim / kChunk, rows, batch);
-  if (c.tail_cap > 16 * kCmbWaves * kCmbTokens)
+  if (general && c.max_splits <= 16 * kCmbSplits &&
+      (int64_t)grid.x * rows * batch > 4 * (int64_t)bmx_device_cu_count())
+    hipLaunchKernelGGL((combine_kernel<kRotated, 4, kDim, Rec, general ? 1 : kCmbWaves>), grid,
+                       dim3(general ? 64 : kCmbThreads), 0, st, c);
+  else if (c.tail_cap > 16 * kCmbWaves * kCmbTokens)
     hipLaunchKernelGGL((combine_kernel<kRotated, 4, kDim, Rec>), grid, dim3(kCmbThreads), 0, st, c);
   else
     hipLaunchKernelGGL((combine_kernel<kRotated, kCmbTokens, kDim, Rec>), grid, dim3(kCmbThreads), 0, st, c);

@@ -140,3 +140,25 @@ def test_decode_with_more_splits_than_the_workspace_holds():
                        split_tokens=st, workspace=ws) for st in (0, 64)]
     assert ws.buf.numel() <= 24 << 20
     assert (outs[0] - outs[1]).abs().max().item() <= 2e-6
+
+
+@pytest.mark.parametrize("T", [0, 64, 65, 200])      # a window wave's pass is 64 rows
+@pytest.mark.parametrize("S,cap", [(256, 200), (4096, 255)])
+def test_decode_batch_of_many_rows(S, T, cap):
+    """40 sequences of 8 heads and 4 queries (more merge workgroups than the chip holds at a time): every sequence
+    equals the same sequence alone, to fp32 summation."""
+    h, d, rank, group, bits, G, B = 8, 32, 16, 32, 3, 4, 40
+    gen = torch.Generator().manual_seed(8)
+    _, _, _, consts, pool, seq = _case_pages(gen, h, d, rank, group, bits, S)
+    table = synth.page_table([seq] * B, device=DEV)
+    kt, vt = (torch.randn(B, h, cap, d, generator=gen).half().to(DEV) for _ in range(2))
+    q = torch.randn(B, h, G, d, generator=gen).to(DEV)
+    lens = torch.full((B,), S, dtype=torch.int32, device=DEV)
+    lens[1::3] -= 128
+    kw = dict(rank=rank, tail_cap=cap, group=group, k_bits=bits, tail_len=T)
+    out = k2b.decode(q, pool.pages, table, lens, S, seq.basis16, consts, d ** -0.5, k_tail=kt, v_tail=vt, **kw)
+    for b in (0, 1, 20, 39):
+        s = slice(b, b + 1)
+        alone = k2b.decode(q[s], pool.pages, table[s], lens[s], S, seq.basis16, consts, d ** -0.5, k_tail=kt[s],
+                           v_tail=vt[s], **kw)
+        assert (out[s] - alone).abs().max().item() <= 2e-6
