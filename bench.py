@@ -905,7 +905,7 @@ def run_general(args, torch, dev) -> dict:
     head_dim 32/64, rank 64/128, residual groups 16/32/128, 2- or 4-bit keys),
     batch 1, --ctx tokens = packed + --window fp16 window rows, --layers
     distinct layer caches in one pool, contiguous pages.  A call is
-    gen_split_kernel + gen_merge_kernel; the roofline counts the pages, the
+    gen_split_kernel + combine_kernel; the roofline counts the pages, the
     basis, the window and q/out."""
     from bmx_amd import k2b, synth
 
@@ -955,7 +955,7 @@ def run_general(args, torch, dev) -> dict:
                                f"{bits}-bit keys, batch 1, ctx {args.ctx} = {packed} packed + {tail} window, "
                                f"{L} layers, contiguous pages",
                    "page_bytes": pool.page_bytes},
-        "roofline": {"bound": "hbm", "kernel": "gen_split_kernel + gen_merge_kernel", "achieved":
+        "roofline": {"bound": "hbm", "kernel": "gen_split_kernel + combine_kernel", "achieved":
                      round(bytes_call / (call_us * 1e-6) / 1e9, 1), "peak": 8000.0, "unit": "GB/s",
                      "frac": round(bytes_call / (call_us * 1e-6) / 8e12, 4), "traffic": None,
                      "bytes_per_launch": bytes_call},

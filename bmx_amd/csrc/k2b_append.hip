@@ -29,16 +29,6 @@ __device__ __forceinline__ uint8_t* append_page(const AppendKArgs& a, int slot) 
   return a.pages + clamp_page(a.page_ids[slot], a.n_pool) * (int64_t)a.L.bytes;
 }
 
-// x / d correctly rounded from r = fl(1 / d): two residual corrections of x r.
-// The first leaves a quotient within an ulp, the second then rounds correctly
-// (Markstein 1990; d, r and the quotient normal, |x| >= 2^-100 or x = 0).
-// 5 instructions against ~11 of the general division.
-__device__ __forceinline__ float div_by(float x, float d, float r) {
-  const float q0 = x * r;
-  const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, d, x), r, q0);
-  return __builtin_fmaf(__builtin_fmaf(-q1, d, x), r, q1);
-}
-
 // 4x4 transpose between four registers and the four 16-lane rows of a wave:
 // register e of row q in, register q of row e out.
 __device__ __forceinline__ void transpose_rows(float (&x)[8], int at) {

@@ -262,6 +262,17 @@ __device__ __forceinline__ void dq_store_tile(const DqTile16<DT>& tl, void* out,
   for (int u = 0; u < 4; ++u) dst[u] = src[u];
 }
 
+// x / d correctly rounded from r = fl(1 / d): two residual corrections of x r.
+// The first leaves a quotient within an ulp, the second then rounds correctly
+// (Markstein 1990; d, the quotient and its residuals normal: |x| >= 2^-100 or x = 0;
+// d up to 3e38, where r is subnormal, gave no other quotient in 4 million).
+// 5 instructions against ~11 of the general division.
+__device__ __forceinline__ float div_by(float x, float d, float r) {
+  const float q0 = x * r;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, d, x), r, q0);
+  return __builtin_fmaf(__builtin_fmaf(-q1, d, x), r, q1);
+}
+
 // Arguments of the k2b write kernels (k2b_append.hip), either page format.
 struct AppendKArgs {
   int h_kv, R, n_codec_pages, n_pool;

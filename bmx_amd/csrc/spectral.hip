@@ -195,13 +195,6 @@ __device__ __forceinline__ void encode_vfull(const SpVFullKArgs& a, VFullLds& s,
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-// x / d correctly rounded from r = fl(1 / d) (k2b_append.hip: div_by).
-__device__ __forceinline__ float sp_div_by(float x, float d, float r) {
-  const float q0 = x * r;
-  const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, d, x), r, q0);
-  return __builtin_fmaf(__builtin_fmaf(-q1, d, x), r, q1);
-}
-
 // Block 256.  Workgroups [0, n_blocks): wave w of workgroup g nx + x (nx =
 // ceil(c_pad / 64)) accumulates Y[t][j] for tokens 16w .. 16w + 15 of group g and
 // page columns 64x .. 64x + 63 over the C channels in order, every product and
@@ -225,7 +218,9 @@ __device__ __forceinline__ float sp_div_by(float x, float d, float r) {
 // 72.8 us; with both operands from LDS (9 reads per 16 VALU), the fit in one wave
 // of 8 and the values in a launch of their own 195.4 and 136.2 us.  3 of 8
 // channels' products on the VALU beside the MFMA's: 127 -> 137 us at 1,920 tokens
-// (the VALU is the bound, not the MFMA).
+// (the VALU is the bound, not the MFMA).  The Lloyd payload (level searches with
+// general divisions): 128 tokens 101.9 us, 1,920 124.6, 8,192 412.5 with full-C
+// values, 115.2, 253.2 and 975.2 before; 128 with per-head values the same, 106.
 // kVec: key rows 16-byte aligned; else the 8 channels are read one by one.
 template <bool kLloyd>
 struct EncodeLds {
@@ -383,7 +378,7 @@ __global__ __launch_bounds__(256, 2) void spectral_encode_kernel(const SpEncodeK
     const float rs = 1.0f / scale;
     if (__all(amax * rs < 1e37f && scale < 3e38f)) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) qv[i] = fminf(fmaxf(rintf(sp_div_by(yv[i], scale, rs)), -qmax - 1.f), qmax);
+      for (int i = 0; i < 16; ++i) qv[i] = fminf(fmaxf(rintf(div_by(yv[i], scale, rs)), -qmax - 1.f), qmax);
     } else {
 #pragma unroll
       for (int i = 0; i < 16; ++i) qv[i] = fminf(fmaxf(rintf(yv[i] / scale), -qmax - 1.f), qmax);
