@@ -295,13 +295,19 @@ __device__ __forceinline__ void score_win_pairs(const A& a, float qscale, int b,
 // query between a wave's pairs gave k2b 183 but RTN 183.
 // One call for all, so that the kernel holds its code once.
 template <class A>
-__device__ __forceinline__ void score_window(const A& a, float qscale, int b, int split, int S, int wave, int waves,
-                                             int n, int q) {
+__device__ __forceinline__ void score_window(const A& a, float qscale, int b, int split, int S, int wave, int n,
+                                             int q) {
   const bool apart = a.win_wgs != 0;
-  const int nw = apart || a.win_tiles * a.h_kv > 8 * S ? waves : 4;
-  if (apart ? split < S : wave >= nw) return;
+  if (apart ? split < S : wave >= a.win_waves) return;
   score_win_pairs(a, qscale, b, apart ? split - S + a.win_wgs * (int)blockIdx.z : split,
-                  apart ? a.win_wgs * (int)gridDim.z : S, wave, nw, n, q);
+                  apart ? a.win_wgs * (int)gridDim.z : S, wave, a.win_waves, n, q);
+}
+
+// Waves of a workgroup of 8 that score the window (win_waves), S splits a sequence:
+// reckoned by the host, so that the kernel has no further arguments to wait for (an
+// RTN call of 512 tokens: split kernel 8.5 us, 9.0 with the comparison in it).
+inline int window_waves(int win_wgs, int win_tiles, int h_kv, int S) {
+  return win_wgs || win_tiles * h_kv > 8 * S ? 8 : 4;
 }
 
 // ---------------------------------------------------------------------------

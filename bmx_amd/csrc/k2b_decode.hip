@@ -97,6 +97,7 @@ struct DecodeKArgs {
   int hpb;             // heads per workgroup (blockIdx.z: the head block)
   int win_tiles;       // 16-token tiles of the window that are scored
   int win_wgs;         // workgroups of a sequence for the window alone, after its max_splits (0: none)
+  int win_waves;       // waves of a workgroup that score it
   float qscale_rope;   // sm_scale * log2(e) * rope_scaling (the cos/sin table is unscaled)
   uint32_t level_hi[4];   // fp16 bits of the value levels as used by the MFMA:
                           // hi_c = kappa * codebook_c + mu (+ < 1e-6 relative)
@@ -672,7 +673,7 @@ __global__ __launch_bounds__(kThreads) void k2b_decode_split_kernel(const Decode
     store_partial(a, b, split, h, n, q, acc, m_run, l_run, w_run);
   }
   } while (false);
-  score_window(a, a.qscale_rope, b, split, S, wave, kWaves, n, q);
+  score_window(a, a.qscale_rope, b, split, S, wave, n, q);
 }
 
 }  // namespace bmx
@@ -1031,6 +1032,7 @@ static int decode_launch(const bmx_k2b_decode_args* a, void* stream, void* ws, s
   const bool balanced = balanced_batch(a);
   const int n_wg = balanced ? device_cu_count() : max_splits * a->batch;
   const int least_share = balanced ? 1 + (n_wg - a->batch) / a->batch : max_splits;
+  k.win_waves = window_waves(k.win_wgs, k.win_tiles, g.h_kv, balanced ? n_wg / a->batch : max_splits);
   const int max_groups = ((a->max_packed_len / kGroup) + least_share - 1) / least_share;
   k.cs_bufs = std::max(1, std::min(max_groups, kCsMaxBufs));
   k.balanced = balanced ? 1 : 0;

@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256) void rtn_dequant_kernel(const RtnDequantKArgs 
 struct RtnDecodeKArgs {
   int h_kv, G, max_splits, max_pages, max_packed_len, n_pool;
   int gk, gv;
-  int hpb, win_tiles, win_wgs;   // plan_splits (decode_shared.h)
+  int hpb, win_tiles, win_wgs, win_waves;   // plan_splits, window_waves (decode_shared.h)
   int prefix_bytes;    // scale bytes of one page (KSCALE + VSCALE), multiple of 16
   const void* q;       // [B][h_kv][G][128] in io_dtype
   int io_dtype;
@@ -706,7 +706,7 @@ __global__ __launch_bounds__(kRThreads) void rtn_decode_split_kernel(const RtnDe
     rtn_store_partial(a, b, split, h, n, q, acc, m_run, l_run);
   }
   } while (false);
-  score_window(a, a.qscale, b, split, S, wave, kRWaves, n, q);
+  score_window(a, a.qscale, b, split, S, wave, n, q);
 }
 
 }  // namespace bmx
@@ -888,6 +888,7 @@ extern "C" int bmx_rtn_decode(const bmx_rtn_decode_args* a, void* stream) {
   RtnDecodeKArgs k{};
   k.hpb = plan.hpb; k.win_wgs = plan.win_wgs;
   k.win_tiles = ((a->tail_len ? a->tail_cap : a->tail_len_value) + 15) / 16;
+  k.win_waves = window_waves(k.win_wgs, k.win_tiles, g.h_kv, S);
   k.h_kv = g.h_kv; k.G = g.n_q_groups; k.max_splits = S; k.max_pages = a->max_pages;
   k.max_packed_len = a->max_packed_len; k.n_pool = a->n_pool_pages > 0 ? a->n_pool_pages : 1;
   k.gk = g.k_group; k.gv = g.v_group;
