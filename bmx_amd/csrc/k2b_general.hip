@@ -144,10 +144,10 @@ __device__ __forceinline__ void gen_rope(const GenReadArgs& a, float4_t kt[D / 1
 // one head takes ~135 VALU (residual 48, rotation 32, high and low parts 32)
 // and, a quarter of its quad's softmax and products, ~45 more at d 64; the
 // HBM floor of 32,640 tokens at d 64, rank 16, h_kv 8 is 2.6 us.  Measured there
-// (G 4, 128-row window): split 17.6 + merge 4.5 us, 20.6 us a call; a workgroup
+// (G 4, 128-row window): split 17.5 + merge 4.3 us, 19.7 us a call; a workgroup
 // per (split, head) with a page at a time per wave, the rotation remade per head
 // and page (22 of them, f64 included, per RoPE pair) and a merge workgroup per
-// query took 31.6 + 8.5 us, 37.9 us a call.  d 128, rank 64: 92 -> 39 us a call.
+// query took 31.6 + 8.5 us, 37.4 us a call.  d 128, rank 64: 92 -> 37 us a call.
 // ---------------------------------------------------------------------------
 struct GenDecodeArgs {
   GenReadArgs r;
