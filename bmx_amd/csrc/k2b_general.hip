@@ -296,7 +296,10 @@ __device__ __forceinline__ void gen_window_tile(const GenDecodeArgs& a, int b, i
       }
     }
   }
-  s += low;
+  // an infinite key makes its later parts' products infinite of either sign, or not
+  // a number: the score is the first parts' infinity
+#pragma unroll
+  for (int e = 0; e < 4; ++e) s[e] = fabsf(s[e]) == INFINITY ? s[e] : s[e] + low[e];
   if (n < a.G) {
     float* dst = a.ws_win + (r0 + n) * a.tail_cap;
 #pragma unroll

@@ -104,3 +104,21 @@ def test_window_scores(d, rank, G, dtype, size):
     err = ((out - ref).norm() / ref.norm()).item()
     print(f"error {err:.2e}, scores to {s.abs().max().item() * 1.4427:.0f}", flush=True)
     assert err <= 8e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_window_key_of_minus_infinite_score(dtype):
+    """A window row whose key is infinite, at a score of minus infinity for every query, has no weight."""
+    h, d, rank, G, T = 2, 64, 16, 4, 20
+    gen = torch.Generator().manual_seed(2)
+    decode, _, _ = _pages(synth.k2b_keys(h, 128, rank, gen, head_dim=d), torch.randn(h, 128, d, generator=gen), rank,
+                          32, 3)
+    kt, vt = (torch.randn(1, h, T, d, generator=gen).to(dtype).to(DEV) for _ in range(2))
+    q = torch.randn(h, G, d, generator=gen).to(DEV)
+    q[..., 5] = -1 - q[..., 5].abs()
+    kt[:, :, 7, 5] = float("inf")
+    out = decode(q, k_tail=kt, v_tail=vt, tail_len=T, tail_cap=T)
+    keep = [t for t in range(T) if t != 7]
+    want = decode(q, k_tail=kt[:, :, keep].contiguous(), v_tail=vt[:, :, keep].contiguous(), tail_len=T - 1,
+                  tail_cap=T - 1)
+    assert torch.isfinite(want).all() and (out - want).abs().max().item() <= 2e-6
